@@ -242,7 +242,7 @@ int  ucns_residual_device(ucns_ctx *ctx, double *rhs_dev, int32_t layout);
 /* ucns_residual_device that allocates nothing.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under
  * HIP graph capture, serving loops, harnesses that forbid hipMalloc).  Its
- * scratch (the face fluxes and troubled-cell counters) is a static device
+ * scratch (the face fluxes) is a static device
  * array of 256 MiB per GPU, held from the library's first use on that GPU
  * until the process ends; meshes with more than about 6.7 million faces are
  * rejected with UCNS_EUNSUPPORTED.  Every call on one GPU shares that array:

@@ -41,6 +41,7 @@ namespace {
 constexpr int NV = 5;
 constexpr int WAVE = 64;
 constexpr int NXCD = 8;
+constexpr int NPART = 64;  // blocks (and results) of k_marks_sum
 // distinct stencil members of a tile held in LDS by the residual product's scatter
 #define UCNS_TILE_UQ 512
 #define UCNS_NOSLOT 0xFFFFu
@@ -88,7 +89,7 @@ struct ReconParams {
     const int32_t *cinfo;  // [ncell]
     const int32_t *cnb;    // [ncell][nf] face neighbours
     R *uleft;              // [ncell][nf][nqm][5]
-    int *counters;         // [0] MUSCL cells, [1] first-order cells
+    int *marks;            // [ncell] per block: MUSCL cells + 65536 * first-order cells (k_marks_sum)
     // CWENO (ees 5) in the per-cell kernel: P holds the central stencil only
     // ([ncell][imax][ideg]); the sectors' low-order pseudo-inverses, their
     // indicators (packed) and mbar - mbar_c over their coefficients
@@ -765,10 +766,10 @@ __global__ __launch_bounds__(WAVE, CW ? 2 : 1) void k_recon(ReconParams<R> p) {
                 sh.u.late.ul[e * NV + v] = (R)((double)res * slope[v]);
             }
         }
-        if (lane == 0) atomicAdd(&p.counters[0], 1);
         __syncthreads();
     }
 
+    bool first = false;
     // ---- phase 7: CHECKSOLX (0.95) -> first order (src/reconstruct_p.f90:3245-3406) ----
     {
         double wi[NV];
@@ -787,15 +788,19 @@ __global__ __launch_bounds__(WAVE, CW ? 2 : 1) void k_recon(ReconParams<R> p) {
             for (int v = 0; v < NV; ++v) uq[v] = ui[v] + (double)sh.u.late.ul[e * NV + v];
             if (jump_test(p.gamma, wi, uq, 0.95)) trouble = 1;
         }
-        const bool first = __syncthreads_or(trouble) != 0;
+        first = __syncthreads_or(trouble) != 0;
         if (first) {
             for (int e = lane; e < nslot; e += WAVE)
 #pragma unroll
                 for (int v = 0; v < NV; ++v) sh.u.late.ul[e * NV + v] = R(0);
-            if (lane == 0) atomicAdd(&p.counters[1], 1);
             __syncthreads();
         }
     }
+
+    // a plain store per cell: the counts' atomicAdd on one address took 12 ns
+    // each, all of a small MUSCL mesh's time (24^3 cells, 10 RK3 steps: 5.60
+    // ms with it, 1.40 ms without)
+    if (lane == 0) p.marks[cell] = (reduce ? 1 : 0) + (first ? 65536 : 0);
 
     // ---- phase 8: ULEFT out, one contiguous block per cell ----
     R *out = p.uleft + (size_t)cell * p.nf * p.nqm * NV;
@@ -824,7 +829,7 @@ struct ReconWParams {
     const int32_t *cinfo;
     const int32_t *cnb;    // [ncell][nf]
     R *uleft;              // [ncell][nf][nqm][5] deviations from the cell average
-    int *counters;
+    int *marks;            // [ntile] per tile: MUSCL cells + 65536 * first-order cells (k_marks_sum)
     const unsigned char *stream;  // per-tile row stream of the DMA kernels (StreamShape)
     long long tile_bytes;
     R *gstore;             // optional [ntile][ideg*5 + 10][8*ts]: every stencil's coefficients, then
@@ -1201,10 +1206,12 @@ __device__ __forceinline__ void recon_late(const ReconWParams<R> &p, R (&g)[IDEG
                 for (int v = 0; v < NV; ++v) out[q * NV + v] = first ? R(0) : res0[r][v];
             }
         }
-        if (s == 0) {
-            atomicAdd(&p.counters[0], 1);
-            if (first) atomicAdd(&p.counters[1], 1);
-        }
+    }
+    {
+        // the tile's counts, summed by k_marks_sum when a caller asks for
+        // them (same-address atomics retire one per 12 ns on this chip)
+        const int nred = __popcll(__ballot(s == 0 && reduce)), nfst = __popcll(__ballot(s == 0 && first));
+        if (lc == 0 && s == 0) p.marks[cell >> 3] = nred + 65536 * nfst;
     }
     if (STORE && s == 0 && cvalid) p.fstore[cell] = (reduce ? 1 : 0) | (first ? 2 : 0);
 }
@@ -3689,9 +3696,29 @@ __global__ void k_rk3_adj_stage(int ncell, int stage, const double *y, const dou
 }
 
 __global__ void k_fill_u64(unsigned long long *p, unsigned long long v) { *p = v; }
-__global__ void k_zero_i32(int *p, int n) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < n) p[e] = 0;
+// sums of the blocks' troubled-cell marks into part[gridDim.x][2]
+__global__ __launch_bounds__(256) void k_marks_sum(const int *marks, int n, int *part) {
+    __shared__ int sh[2][256 / WAVE];
+    int a = 0, b = 0;
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) {
+        a += marks[e] & 65535;
+        b += marks[e] >> 16;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        a += __shfl_xor(a, o, WAVE);
+        b += __shfl_xor(b, o, WAVE);
+    }
+    if ((threadIdx.x & (WAVE - 1)) == 0) {
+        sh[0][threadIdx.x / WAVE] = a;
+        sh[1][threadIdx.x / WAVE] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        int t = 0;
+        for (int w = 0; w < 256 / WAVE; ++w) t += sh[threadIdx.x][w];
+        part[blockIdx.x * 2 + threadIdx.x] = t;
+    }
 }
 
 // Per-cell 5-vectors across the ABI: the caller's cell o = perm[c] (o = c
@@ -3743,14 +3770,14 @@ __global__ void k_relayout_p(const double *src, R *dst, int ncells, int ts_in, i
 template <typename T>
 int dalloc(ucns_ctx *ctx, T **p, size_t n);
 
-// Scratch of ucns_residual_noalloc: its troubled-cell counters (the first
-// 256 bytes) and face fluxes, in a file-scope device array that every GPU the
+// Scratch of ucns_residual_noalloc: its face fluxes (behind a reserved head
+// of 256 bytes), in a file-scope device array that every GPU the
 // library runs on holds from the library's first use on it until the process
 // ends, so that the call allocates nothing.  In host code the array's name is
 // a stand-in, not a device address: scratch_on() takes each device's own
 // address once, with hipGetSymbolAddress, and only that address is used.
 constexpr size_t UCNS_SCRATCH_BYTES = (size_t)256 << 20;  // 256 MiB: 6.7 M faces
-constexpr size_t UCNS_SCRATCH_HEAD = 256;                  // counters
+constexpr size_t UCNS_SCRATCH_HEAD = 256;                  // reserved
 
 }  // namespace
 
@@ -3838,7 +3865,9 @@ struct ucns_ctx {
     // state (device)
     double *U = nullptr, *U2 = nullptr, *fflux = nullptr, *rhs = nullptr, *t = nullptr, *dtfix = nullptr;
     unsigned long long *dtv = nullptr;  // [2] ping-pong dt slots
-    int *counters = nullptr, *flag = nullptr;
+    int *marks = nullptr, *marks_part = nullptr;  // troubled cells per reconstruction block; their sums [NPART][2]
+    int nmark = 0;
+    int *flag = nullptr;
     // adjoint (allocated on first use): face-point cotangents, state-sized
     // work arrays, the free-stream cotangent, stage checkpoints and step dts
     double *adj_ubf = nullptr, *adj_lam = nullptr, *adj_ubar = nullptr, *adj_x = nullptr, *adj_a = nullptr;
@@ -3926,7 +3955,7 @@ int launch_recon_t(ucns_ctx *ctx) {
     p.cinfo = ctx->cinfo;
     p.cnb = ctx->cnb;
     p.uleft = (R *)ctx->uleft;
-    p.counters = ctx->counters;
+    p.marks = ctx->marks;
     p.Pc = (const R *)ctx->Pc;
     p.Bc = (const R *)ctx->Bc;
     p.dmb = (const R *)ctx->dmb;
@@ -3958,7 +3987,7 @@ int launch_recon_t(ucns_ctx *ctx) {
         w.cinfo = ctx->cinfo;
         w.cnb = ctx->cnb;
         w.uleft = (R *)ctx->uleft;
-        w.counters = ctx->counters;
+        w.marks = ctx->marks;
         const dim3 grid(w.tiles_per_xcd * NXCD), block(WAVE);
         w.stream = ctx->rows;
         w.tile_bytes = ctx->tile_bytes;
@@ -4139,7 +4168,6 @@ void tcollect(ucns_ctx *ctx, int k, double *acc, int64_t *n) {
 
 // reconstruction + face fluxes of the current state (ULEFT and face fluxes on device)
 int residual_kernels(ucns_ctx *ctx) {
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, ctx->stream, ctx->counters, 2);
     tstart(ctx, 0);
     int rc = ctx->precision == UCNS_MIXED ? launch_recon_t<float>(ctx) : launch_recon_t<double>(ctx);
     if (rc) return rc;
@@ -4177,6 +4205,24 @@ int update_kernel(ucns_ctx *ctx, int stage, const double *dt, unsigned long long
     hipLaunchKernelGGL(k_update, dim3((ctx->ncell + 255) / 256), dim3(256), 0, ctx->stream, p);
     tstop(ctx, 2);
     tcollect(ctx, 2, &ctx->st.ms_update, &ctx->st.n_update);
+    return UCNS_OK;
+}
+
+// the troubled-cell counts of the last reconstruction into the statistics;
+// waits for the stream
+int collect_counts(ucns_ctx *ctx) {
+    int part[2 * NPART];
+    hipLaunchKernelGGL(k_marks_sum, dim3(NPART), dim3(256), 0, ctx->stream, ctx->marks, ctx->nmark, ctx->marks_part);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(part, ctx->marks_part, sizeof(part), hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    int64_t red = 0, fst = 0;
+    for (int b = 0; b < NPART; ++b) {
+        red += part[2 * b];
+        fst += part[2 * b + 1];
+    }
+    ctx->st.n_reduced_last = red;
+    ctx->st.n_firstorder_last = fst;
     return UCNS_OK;
 }
 
@@ -4440,7 +4486,6 @@ void launch_scatter_t(ucns_ctx *ctx, double *ubar) {
 // weights and the cell flags
 template <typename R>
 int vjp_recon_t(ucns_ctx *ctx) {
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, ctx->stream, ctx->counters, 2);
     ctx->adj_g_on = ctx->smode && ctx->adj_g;
     tstart(ctx, 3);
     const int rc = launch_recon_t<R>(ctx);
@@ -4778,6 +4823,7 @@ void release_prestore(ucns_ctx *ctx) {
     dfree(ctx->P);
     dfree(ctx->rows);
     dfree(ctx->u64);
+    dfree(ctx->marks);
     dfree(ctx->B);
     dfree(ctx->mbar);
     if (ctx->Bc) (void)hipFree(ctx->Bc);
@@ -5242,7 +5288,7 @@ int ucns_create(const ucns_mesh_v2 *m, const ucns_scheme_v2 *s, ucns_ctx **out) 
         (rc = dalloc(ctx, &ctx->U2, (size_t)nc * NV)) || (rc = dalloc(ctx, &ctx->rhs, (size_t)nc * NV)) ||
         (rc = dalloc(ctx, &ctx->fflux, (size_t)ctx->nface * NV)) || (rc = dalloc(ctx, &ctx->t, 1)) ||
         (rc = dalloc(ctx, &ctx->dtfix, 1)) || (rc = dalloc(ctx, &ctx->dtv, 2)) ||
-        (rc = dalloc(ctx, &ctx->counters, 2)) || (rc = dalloc(ctx, &ctx->flag, 1)) ||
+        (rc = dalloc(ctx, &ctx->marks_part, 2 * NPART)) || (rc = dalloc(ctx, &ctx->flag, 1)) ||
         (rc = dalloc(ctx, &ctx->stage, (size_t)nc * NV)))
         return rc;
     if (!ctx->h_perm.empty()) {
@@ -5336,6 +5382,10 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
         ctx->smode = stream_ok ? ts : 0;
     }
     ctx->ntile = (nc + 7) / 8;
+    ctx->nmark = ctx->tiled ? ctx->ntile : nc;
+    int rc = dalloc(ctx, &ctx->marks, (size_t)ctx->nmark);
+    if (rc) return rc;
+    HIP_TRY(hipMemset(ctx->marks, 0, (size_t)ctx->nmark * sizeof(int)));
     // stencil members without the cell itself
     //   tiled: [tile][imax][8*ts], lane position 8-cell-tile local
     //   plain: [cell][ts][imax]
@@ -5366,8 +5416,7 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
             }
         }
     }
-    int rc = dalloc(ctx, &ctx->nbr, std::max<size_t>(nbr.size(), 1));
-    if (rc) return rc;
+    if ((rc = dalloc(ctx, &ctx->nbr, std::max<size_t>(nbr.size(), 1)))) return rc;
     if (!nbr.empty())
         HIP_TRY(hipMemcpy(ctx->nbr, nbr.data(), nbr.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(ctx->cinfo, cinfo.data(), nc * sizeof(int32_t), hipMemcpyHostToDevice));
@@ -5731,7 +5780,6 @@ int ucns_reconstruct(ucns_ctx *ctx, double *uleft_out) {
     int rc = ready(ctx);
     if (rc) return rc;
     HIP_TRY(hipSetDevice(ctx->device));
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, ctx->stream, ctx->counters, 2);
     rc = ctx->precision == UCNS_MIXED ? launch_recon_t<float>(ctx) : launch_recon_t<double>(ctx);
     if (rc) return rc;
     HIP_TRY(hipGetLastError());
@@ -5759,11 +5807,7 @@ int ucns_reconstruct(ucns_ctx *ctx, double *uleft_out) {
                     uleft_out[((o * nfa + f) * nqa + q) * NV + v] =
                         u[(size_t)i * NV + v] + d[(((size_t)i * ctx->nf + f) * ctx->nqm + q) * NV + v];
     }
-    int cnt[2];
-    HIP_TRY(hipMemcpy(cnt, ctx->counters, sizeof(cnt), hipMemcpyDeviceToHost));
-    ctx->st.n_reduced_last = cnt[0];
-    ctx->st.n_firstorder_last = cnt[1];
-    return UCNS_OK;
+    return collect_counts(ctx);
 }
 
 static int residual_to(ucns_ctx *ctx, double *rhs_out, int32_t layout, bool host) {
@@ -5775,11 +5819,7 @@ static int residual_to(ucns_ctx *ctx, double *rhs_out, int32_t layout, bool host
     if ((rc = residual_kernels(ctx))) return rc;
     update_kernel(ctx, 0, nullptr, nullptr, 0.0, ctx->rhs);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
-    int cnt[2];
-    HIP_TRY(hipMemcpy(cnt, ctx->counters, sizeof(cnt), hipMemcpyDeviceToHost));
-    ctx->st.n_reduced_last = cnt[0];
-    ctx->st.n_firstorder_last = cnt[1];
+    if ((rc = collect_counts(ctx))) return rc;
     if (rhs_out) return cells_out(ctx, ctx->rhs, layout, rhs_out, host);
     return UCNS_OK;
 }
@@ -5803,29 +5843,15 @@ int ucns_residual_noalloc(ucns_ctx *ctx, double *rhs_dev, int32_t layout) {
         return UCNS_ESTATE;
     }
     HIP_TRY(hipSetDevice(ctx->device));
-    // the same kernels as ucns_residual_device, with their counters and face
-    // fluxes in the static scratch (the counters are cleared by a kernel at
-    // the start of every reconstruction; every face flux is written before
-    // it is read)
-    int *const own_counters = ctx->counters;
+    // the same kernels as ucns_residual_device, with their face fluxes in the
+    // static scratch (every face flux is written before it is read)
     double *const own_fflux = ctx->fflux;
-    ctx->counters = (int *)ctx->scratch;
     ctx->fflux = (double *)((unsigned char *)ctx->scratch + UCNS_SCRATCH_HEAD);
     rc = residual_kernels(ctx);
     if (rc == UCNS_OK) update_kernel(ctx, 0, nullptr, nullptr, 0.0, ctx->rhs);
-    int cnt[2] = {0, 0};
-    if (rc == UCNS_OK && hipMemcpyAsync(cnt, ctx->counters, sizeof(cnt), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess)
-        rc = UCNS_EHIP;
-    if (rc == UCNS_OK && hipStreamSynchronize(ctx->stream) != hipSuccess) rc = UCNS_EHIP;
-    ctx->counters = own_counters;
+    if (rc == UCNS_OK) rc = collect_counts(ctx);
     ctx->fflux = own_fflux;
-    if (rc == UCNS_EHIP) {
-        ctx->err = std::string("ucns_residual_noalloc: ") + hipGetErrorString(hipGetLastError());
-        return rc;
-    }
     if (rc) return rc;
-    ctx->st.n_reduced_last = cnt[0];
-    ctx->st.n_firstorder_last = cnt[1];
     return cells_out(ctx, ctx->rhs, layout, rhs_dev, false);
 }
 
@@ -5869,12 +5895,8 @@ int ucns_rk3_steps(ucns_ctx *ctx, int32_t nsteps, double cfl, double dt_fixed, d
     double t1 = t0;
     HIP_TRY(hipMemcpyAsync(&flag, ctx->flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipMemcpyAsync(&t1, ctx->t, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if ((rc = collect_counts(ctx))) return rc;  // waits for the copies above
     if (t_io) *t_io = t1;
-    int cnt[2];
-    HIP_TRY(hipMemcpy(cnt, ctx->counters, sizeof(cnt), hipMemcpyDeviceToHost));
-    ctx->st.n_reduced_last = cnt[0];
-    ctx->st.n_firstorder_last = cnt[1];
     if (flag) {
         ctx->err = "non-finite state after the RK3 steps";
         return UCNS_ENONFINITE;
@@ -6178,7 +6200,7 @@ void ucns_destroy(ucns_ctx *ctx) {
     dfree(ctx->t);
     dfree(ctx->dtfix);
     dfree(ctx->dtv);
-    dfree(ctx->counters);
+    dfree(ctx->marks_part);
     dfree(ctx->flag);
     dfree(ctx->uleft);
     for (auto &e : ctx->ev)
