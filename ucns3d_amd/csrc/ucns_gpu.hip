@@ -2301,8 +2301,9 @@ struct UpdateParams {
     const double *minedge;
     double *U, *U2;
     double *rhs_out;         // optional [ncell][5]
-    const double *dt;        // this step's dt
-    unsigned long long *dt_next;  // atomic-min target (bits of a positive double), stage 3 only
+    const double *dt;        // this step's dt: one value, or (dt_slots) the slots it is the least of
+    int dt_slots;
+    unsigned long long *dt_next;  // the next step's slots: cleared to +inf in stage 2, atomic-min targets in stage 3
     double *t;               // advanced by dt in stage 3
 };
 
@@ -2310,10 +2311,41 @@ __device__ inline void atomic_min_pos(unsigned long long *addr, double v) {
     atomicMin(addr, (unsigned long long)__double_as_longlong(v));
 }
 
+// A CFL step is the least of DT_SLOTS values on cache lines of their own:
+// every block of 256 cells reduces its cells first and then lowers slot
+// (block mod DT_SLOTS).  Atomics on one address retire one per 12 ns, so one
+// per wave on a single value took 37 us of 196,608 cells' 38 us update (and
+// of their k_dt); 16 slots keep a chain of at most 48 atomics there, and a
+// reader still loads only 16 lines.
+constexpr int DT_SLOTS = 16, DT_STRIDE = 16;  // 128-byte lines
+
+__device__ inline double dt_of(const double *dt, bool slots) {
+    if (!slots) return *dt;
+    double v = dt[(threadIdx.x & (DT_SLOTS - 1)) * DT_STRIDE];
+#pragma unroll
+    for (int o = DT_SLOTS / 2; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, WAVE));
+    return v;
+}
+
+// the block's (256 threads) least d into its slot; every thread takes part
+__device__ inline void dt_lower(unsigned long long *slots, double d) {
+    __shared__ double sh[256 / WAVE];
+    d = wave_min(d);
+    if ((threadIdx.x & (WAVE - 1)) == 0) sh[threadIdx.x / WAVE] = d;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 256 / WAVE; ++w) d = fmin(d, sh[w]);
+        if (d < 1.0e300) atomic_min_pos(slots + (blockIdx.x & (DT_SLOTS - 1)) * DT_STRIDE, d);
+    }
+}
+
 // stage 0: gather only (rhs_out); stage 1..3: Shu-Osher update
 __global__ __launch_bounds__(256) void k_update(UpdateParams p) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     double dtl = 1.0e300;
+    const double dt = p.stage > 0 ? dt_of(p.dt, p.dt_slots) : 0.0;
+    if (p.stage == 2 && p.dt_next && blockIdx.x == 0) p.dt_next[threadIdx.x] = 0x7FF0000000000000ULL;
+    static_assert(DT_SLOTS * DT_STRIDE == 256, "one block of k_update clears the slots");
     if (i < p.ncell) {
         // every face's flux is loaded before the first is summed (face
         // slots past nf, and slots with no face, read face 0 and add nothing)
@@ -2344,7 +2376,7 @@ __global__ __launch_bounds__(256) void k_update(UpdateParams p) {
             for (int v = 0; v < NV; ++v) p.rhs_out[(size_t)i * NV + v] = r[v];
         }
         if (p.stage > 0) {
-            const double dt = *p.dt, oov = p.ovol[i];
+            const double oov = p.ovol[i];
             double *u = p.U + (size_t)i * NV, *u2 = p.U2 + (size_t)i * NV;
             const double to4 = 3.0 / 4.0, oo4 = 1.0 / 4.0, to3 = 2.0 / 3.0, oo3 = 1.0 / 3.0;
             double un[NV];
@@ -2373,11 +2405,8 @@ __global__ __launch_bounds__(256) void k_update(UpdateParams p) {
         }
     }
     if (p.stage == 3) {
-        if (p.dt_next) {
-            dtl = wave_min(dtl);
-            if ((threadIdx.x & (WAVE - 1)) == 0 && dtl < 1.0e300) atomic_min_pos(p.dt_next, dtl);
-        }
-        if (i == 0 && p.t) *p.t += *p.dt;
+        if (p.dt_next) dt_lower(p.dt_next, dtl);
+        if (i == 0 && p.t) *p.t += dt;
     }
 }
 
@@ -2398,8 +2427,13 @@ __global__ __launch_bounds__(256) void k_dt(DtParams p) {
         const double veln = fmax(fmax(fabs(w[1]), fabs(w[2])), fabs(w[3])) + c;
         d = (p.cfl / 3.0) * (p.minedge[i] / fabs(veln));
     }
-    d = wave_min(d);
-    if ((threadIdx.x & (WAVE - 1)) == 0 && d < 1.0e300) atomic_min_pos(p.dt_out, d);
+    dt_lower(p.dt_out, d);
+}
+
+// the step size of a set of slots
+__global__ void k_dt_value(const double *slots, double *out) {
+    const double v = dt_of(slots, true);
+    if (threadIdx.x == 0) *out = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -3695,7 +3729,7 @@ __global__ void k_rk3_adj_stage(int ncell, int stage, const double *y, const dou
     }
 }
 
-__global__ void k_fill_u64(unsigned long long *p, unsigned long long v) { *p = v; }
+__global__ void k_fill_u64(unsigned long long *p, unsigned long long v) { p[threadIdx.x] = v; }
 // sums of the blocks' troubled-cell marks into part[gridDim.x][2]
 __global__ __launch_bounds__(256) void k_marks_sum(const int *marks, int n, int *part) {
     __shared__ int sh[2][256 / WAVE];
@@ -3864,7 +3898,7 @@ struct ucns_ctx {
     long long tile_bytes = 0;
     // state (device)
     double *U = nullptr, *U2 = nullptr, *fflux = nullptr, *rhs = nullptr, *t = nullptr, *dtfix = nullptr;
-    unsigned long long *dtv = nullptr;  // [2] ping-pong dt slots
+    unsigned long long *dtv = nullptr;  // [2][DT_SLOTS * DT_STRIDE] ping-pong dt slots
     int *marks = nullptr, *marks_part = nullptr;  // troubled cells per reconstruction block; their sums [NPART][2]
     int nmark = 0;
     int *flag = nullptr;
@@ -4183,7 +4217,7 @@ int residual_kernels(ucns_ctx *ctx) {
     return UCNS_OK;
 }
 
-int update_kernel(ucns_ctx *ctx, int stage, const double *dt, unsigned long long *dt_next, double cfl,
+int update_kernel(ucns_ctx *ctx, int stage, const double *dt, bool dt_slots, unsigned long long *dt_next, double cfl,
                   double *rhs_out) {
     UpdateParams p{};
     p.ncell = ctx->ncell;
@@ -4199,6 +4233,7 @@ int update_kernel(ucns_ctx *ctx, int stage, const double *dt, unsigned long long
     p.U2 = ctx->U2;
     p.rhs_out = rhs_out;
     p.dt = dt;
+    p.dt_slots = dt_slots;
     p.dt_next = dt_next;
     p.t = ctx->t;
     tstart(ctx, 2);
@@ -4227,7 +4262,7 @@ int collect_counts(ucns_ctx *ctx) {
 }
 
 int dt_kernel(ucns_ctx *ctx, double cfl, unsigned long long *out) {
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(1), 0, ctx->stream, out,
+    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(DT_SLOTS * DT_STRIDE), 0, ctx->stream, out,
                        (unsigned long long)0x7FF0000000000000ULL);
     DtParams p{};
     p.ncell = ctx->ncell;
@@ -4739,10 +4774,7 @@ int rk3_step_ckpt(ucns_ctx *ctx, int it, const double *dt, unsigned long long *n
             rc = residual_kernels(ctx);
         }
         if (rc) return rc;
-        if (stage == 3 && next)
-            hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(1), 0, ctx->stream, next,
-                               (unsigned long long)0x7FF0000000000000ULL);
-        update_kernel(ctx, stage, dt, stage == 3 ? next : nullptr, cfl, nullptr);
+        update_kernel(ctx, stage, dt, next != nullptr, next, cfl, nullptr);
     }
     return UCNS_OK;
 }
@@ -5287,7 +5319,7 @@ int ucns_create(const ucns_mesh_v2 *m, const ucns_scheme_v2 *s, ucns_ctx **out) 
         (rc = dalloc(ctx, &ctx->minedge, nc)) || (rc = dalloc(ctx, &ctx->U, (size_t)nc * NV)) ||
         (rc = dalloc(ctx, &ctx->U2, (size_t)nc * NV)) || (rc = dalloc(ctx, &ctx->rhs, (size_t)nc * NV)) ||
         (rc = dalloc(ctx, &ctx->fflux, (size_t)ctx->nface * NV)) || (rc = dalloc(ctx, &ctx->t, 1)) ||
-        (rc = dalloc(ctx, &ctx->dtfix, 1)) || (rc = dalloc(ctx, &ctx->dtv, 2)) ||
+        (rc = dalloc(ctx, &ctx->dtfix, 1)) || (rc = dalloc(ctx, &ctx->dtv, 2 * DT_SLOTS * DT_STRIDE)) ||
         (rc = dalloc(ctx, &ctx->marks_part, 2 * NPART)) || (rc = dalloc(ctx, &ctx->flag, 1)) ||
         (rc = dalloc(ctx, &ctx->stage, (size_t)nc * NV)))
         return rc;
@@ -5769,9 +5801,11 @@ int ucns_compute_dt(ucns_ctx *ctx, double cfl, double *dt_out) {
         return UCNS_ESTATE;
     }
     HIP_TRY(hipSetDevice(ctx->device));
-    dt_kernel(ctx, cfl, &ctx->dtv[0]);
-    HIP_TRY(hipMemcpyAsync(dt_out, &ctx->dtv[0], sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    dt_kernel(ctx, cfl, ctx->dtv);
+    double slots[DT_SLOTS * DT_STRIDE];
+    HIP_TRY(hipMemcpyAsync(slots, ctx->dtv, sizeof(slots), hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
+    *dt_out = *std::min_element(slots, slots + DT_SLOTS * DT_STRIDE);
     return UCNS_OK;
 }
 
@@ -5817,7 +5851,7 @@ static int residual_to(ucns_ctx *ctx, double *rhs_out, int32_t layout, bool host
     if (rc) return rc;
     HIP_TRY(hipSetDevice(ctx->device));
     if ((rc = residual_kernels(ctx))) return rc;
-    update_kernel(ctx, 0, nullptr, nullptr, 0.0, ctx->rhs);
+    update_kernel(ctx, 0, nullptr, false, nullptr, 0.0, ctx->rhs);
     HIP_TRY(hipGetLastError());
     if ((rc = collect_counts(ctx))) return rc;
     if (rhs_out) return cells_out(ctx, ctx->rhs, layout, rhs_out, host);
@@ -5848,7 +5882,7 @@ int ucns_residual_noalloc(ucns_ctx *ctx, double *rhs_dev, int32_t layout) {
     double *const own_fflux = ctx->fflux;
     ctx->fflux = (double *)((unsigned char *)ctx->scratch + UCNS_SCRATCH_HEAD);
     rc = residual_kernels(ctx);
-    if (rc == UCNS_OK) update_kernel(ctx, 0, nullptr, nullptr, 0.0, ctx->rhs);
+    if (rc == UCNS_OK) update_kernel(ctx, 0, nullptr, false, nullptr, 0.0, ctx->rhs);
     if (rc == UCNS_OK) rc = collect_counts(ctx);
     ctx->fflux = own_fflux;
     if (rc) return rc;
@@ -5874,16 +5908,13 @@ int ucns_rk3_steps(ucns_ctx *ctx, int32_t nsteps, double cfl, double dt_fixed, d
     const bool fixed = dt_fixed > 0;
     if (fixed) HIP_TRY(hipMemcpyAsync(ctx->dtfix, &dt_fixed, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
     int cur = 0;
-    if (!fixed && nsteps > 0) dt_kernel(ctx, cfl, &ctx->dtv[cur]);
+    if (!fixed && nsteps > 0) dt_kernel(ctx, cfl, ctx->dtv);
     for (int it = 0; it < nsteps; ++it) {
-        const double *dt = fixed ? ctx->dtfix : (const double *)&ctx->dtv[cur];
-        unsigned long long *next = fixed ? nullptr : &ctx->dtv[1 - cur];
+        const double *dt = fixed ? ctx->dtfix : (const double *)(ctx->dtv + cur * DT_SLOTS * DT_STRIDE);
+        unsigned long long *next = fixed ? nullptr : ctx->dtv + (1 - cur) * DT_SLOTS * DT_STRIDE;
         for (int stage = 1; stage <= 3; ++stage) {
             if ((rc = residual_kernels(ctx))) return rc;
-            if (stage == 3 && next)
-                hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(1), 0, ctx->stream, next,
-                                   (unsigned long long)0x7FF0000000000000ULL);
-            update_kernel(ctx, stage, dt, stage == 3 ? next : nullptr, cfl, nullptr);
+            update_kernel(ctx, stage, dt, !fixed, next, cfl, nullptr);
         }
         HIP_TRY(hipGetLastError());
         if (!fixed) cur = 1 - cur;
@@ -5966,11 +5997,14 @@ static int rk3_adjoint_impl(ucns_ctx *ctx, int32_t nsteps, double cfl, double dt
     const bool fixed = dt_fixed > 0;
     if (fixed) HIP_TRY(hipMemcpyAsync(ctx->dtfix, &dt_fixed, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
     int cur = 0;
-    if (!fixed) dt_kernel(ctx, cfl, &ctx->dtv[cur]);
+    if (!fixed) dt_kernel(ctx, cfl, ctx->dtv);
     for (int it = 0; it < nsteps; ++it) {
-        const double *dt = fixed ? ctx->dtfix : (const double *)&ctx->dtv[cur];
-        unsigned long long *next = fixed ? nullptr : &ctx->dtv[1 - cur];
-        HIP_TRY(hipMemcpyAsync(ctx->dts + it, dt, sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
+        const double *dt = fixed ? ctx->dtfix : (const double *)(ctx->dtv + cur * DT_SLOTS * DT_STRIDE);
+        unsigned long long *next = fixed ? nullptr : ctx->dtv + (1 - cur) * DT_SLOTS * DT_STRIDE;
+        if (fixed)
+            HIP_TRY(hipMemcpyAsync(ctx->dts + it, dt, sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
+        else
+            hipLaunchKernelGGL(k_dt_value, dim3(1), dim3(WAVE), 0, ctx->stream, dt, ctx->dts + it);
         if ((rc = rk3_step_ckpt(ctx, it, dt, next, cfl, keep0))) return rc;
         HIP_TRY(hipGetLastError());
         if (!fixed) cur = 1 - cur;
