@@ -3416,35 +3416,44 @@ __global__ __launch_bounds__(WAVE) void k_recon_vjp_s(VjpParams<R> p) {
 }
 
 // ubar[n] += the rows of every tile's member table that belong to cell n
-// (CSR: rows ent[off[n]] .. ent[off[n+1]-1]); each cell is one thread's, so
-// no atomics
+// (CSR: rows ent[off[n]] .. ent[off[n+1]-1]); no atomics.  Bound by the
+// latency of the dependent loads entry -> row: 8 lanes share a cell, each
+// taking every 8th row, so that a cell of WENO-4 tetrahedra (43 rows) is 6
+// trips and the launch has 8 times the waves of one thread per cell.
+// 24,576 tetrahedra: 54.7 -> 26.0 us (one thread per cell before); a
+// 14,000-cell channel: 27.6 -> 9.5 us.
 __global__ __launch_bounds__(256) void k_adj_gather(int ncell, const int64_t *off, const int32_t *ent,
                                                     const double *tab, double *ubar) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= ncell) return;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, n = t >> 3, s = t & 7;
     double a[NV] = {0, 0, 0, 0, 0};
-    // GU rows in flight: their indices, then the rows, are loaded before any
-    // is added (the sum keeps the entries' order)
-    constexpr int GU = 4;
-    const int64_t e0 = off[n], e1 = off[n + 1];
-    for (int64_t e = e0; e < e1; e += GU) {
-        int32_t rr[GU];
+    if (n < ncell) {
+        constexpr int GU = 2;  // rows in flight per lane
+        const int64_t e0 = off[n], e1 = off[n + 1];
+        for (int64_t e = e0 + s; e < e1; e += 8 * GU) {
+            int32_t rr[GU];
 #pragma unroll
-        for (int u = 0; u < GU; ++u) rr[u] = ent[min(e + u, e1 - 1)];
-        double x[GU][NV];
+            for (int u = 0; u < GU; ++u) rr[u] = ent[min(e + 8 * u, e1 - 1)];
+            double x[GU][NV];
 #pragma unroll
-        for (int u = 0; u < GU; ++u)
+            for (int u = 0; u < GU; ++u)
 #pragma unroll
-            for (int v = 0; v < NV; ++v) x[u][v] = tab[(size_t)rr[u] * NV + v];
+                for (int v = 0; v < NV; ++v) x[u][v] = tab[(size_t)rr[u] * NV + v];
 #pragma unroll
-        for (int u = 0; u < GU; ++u)
-            if (e + u < e1) {
+            for (int u = 0; u < GU; ++u)
+                if (e + 8 * u < e1) {
 #pragma unroll
-                for (int v = 0; v < NV; ++v) a[v] += x[u][v];
-            }
+                    for (int v = 0; v < NV; ++v) a[v] += x[u][v];
+                }
+        }
     }
 #pragma unroll
-    for (int v = 0; v < NV; ++v) ubar[(size_t)n * NV + v] += a[v];
+    for (int v = 0; v < NV; ++v) a[v] = grp_sum8(a[v]);
+    if (n < ncell && s < NV) {
+        double m = a[0];
+#pragma unroll
+        for (int v = 1; v < NV; ++v) m = s == v ? a[v] : m;
+        ubar[(size_t)n * NV + s] += m;
+    }
 }
 
 // CSR of the member tables by cell: counts, then positions
@@ -3468,63 +3477,44 @@ __global__ void k_adj_csr(int ntile, int cap, const int32_t *uq, const int32_t *
 // BND: the launch over boundary faces (ghost-state Jacobians by forward
 // mode); the other launch takes the interior and periodic faces, whose
 // kernel then carries none of the boundary code's registers
+//
+// One thread per (face, quadrature point): the points are independent, their
+// writes are contiguous across lanes, and a small mesh still fills the chip
+// (one thread per face left 121 blocks for a 14,000-cell channel).  The
+// boundary launch runs over the list of boundary faces, so its waves are
+// full, and reduces the ten free-stream cotangents in the block before its
+// atomics (same-address atomics retire one per 12 ns).
+// 14,000-cell channel: interior 19.4 -> 10.6 us, boundary 113.7 -> 20.6 us;
+// 24,576 tetrahedra: 34.9 -> 22.4 us.
 template <typename R, bool BND>
-__global__ __launch_bounds__(256) void k_flux_vjp(FluxParams<R> p, const double *lam, double *ubf, double *bcbar) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= p.nface) return;
-    const int cL = p.fcell[2 * f], cR = p.fcell[2 * f + 1];
-    if ((cR < 0) != BND) return;
-    const int s0 = p.fslot[2 * f], sR = p.fslot[2 * f + 1];
-    const int sL = s0 & 255;
-    const bool tri = (s0 >> 8) & 1;
-    const int nq = tri ? p.qpt : p.qpq;
-    const double *w = tri ? p.wt : p.wq;
-    const double c1 = p.frot[4 * f], s1 = p.frot[4 * f + 1], c2 = p.frot[4 * f + 2], s2 = p.frot[4 * f + 3];
-    const double area = p.farea[f];
+__global__ __launch_bounds__(256) void k_flux_vjp(FluxParams<R> p, const int32_t *bfaces, int nbface,
+                                                  const double *lam, double *ubf, double *bcbar) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int fi = t / p.nqm, q = t - fi * p.nqm;
+    const int f = BND ? (fi < nbface ? bfaces[fi] : p.nface) : fi;
     constexpr bool bnd = BND;
-    double uL[NV], uR[NV], Fb[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        uL[v] = p.U[(size_t)cL * NV + v];
-        uR[v] = bnd ? 0.0 : p.U[(size_t)cR * NV + v];
-        Fb[v] = lam[(size_t)cL * NV + v] - (bnd ? 0.0 : lam[(size_t)cR * NV + v]);
-    }
-    double hb0[NV];
-    rotf(Fb, c1, s1, c2, s2, hb0);
-    const R *ulL = p.uleft + ((size_t)cL * p.nf + sL) * p.nqm * NV;
-    const R *ulR = p.uleft + ((size_t)(bnd ? cL : cR) * p.nf + (bnd ? sL : sR)) * p.nqm * NV;
-    double *obL = ubf + ((size_t)cL * p.nf + sL) * p.nqm * NV;
-    double *obR = ubf + ((size_t)(bnd ? cL : cR) * p.nf + (bnd ? sL : sR)) * p.nqm * NV;
     double bcacc[2 * NV] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    // QB points' deviations are loaded before any is used, as in k_flux
-    constexpr int QB = 3;
-    R dl[QB][NV], dr[QB][NV];
-    for (int q = 0; q < nq; ++q) {
-        const int qb = q % QB;
-        if (qb == 0) {
-#pragma unroll
-            for (int u = 0; u < QB; ++u) {
-                const int qq = min(q + u, nq - 1);
-#pragma unroll
-                for (int v = 0; v < NV; ++v) {
-                    dl[u][v] = ulL[qq * NV + v];
-                    dr[u][v] = ulR[qq * NV + v];
-                }
-            }
-        }
-        double a[NV], bq[NV];
+    auto point = [&]() {
+        const int cL = p.fcell[2 * f], cR = p.fcell[2 * f + 1];
+        if ((cR < 0) != BND) return;
+        const int s0 = p.fslot[2 * f], sR = p.fslot[2 * f + 1];
+        const int sL = s0 & 255;
+        const bool tri = (s0 >> 8) & 1;
+        if (q >= (tri ? p.qpt : p.qpq)) return;
+        const double *w = tri ? p.wt : p.wq;
+        const double c1 = p.frot[4 * f], s1 = p.frot[4 * f + 1], c2 = p.frot[4 * f + 2], s2 = p.frot[4 * f + 3];
+        const double area = p.farea[f];
+        const size_t oL = (((size_t)cL * p.nf + sL) * p.nqm + q) * NV;
+        const size_t oR = bnd ? oL : (((size_t)cR * p.nf + sR) * p.nqm + q) * NV;
+        double a[NV], bq[NV], Fb[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            R xl = dl[0][v], xr = dr[0][v];
-#pragma unroll
-            for (int u = 1; u < QB; ++u)
-                if (qb == u) {
-                    xl = dl[u][v];
-                    xr = dr[u][v];
-                }
-            a[v] = uL[v] + (double)xl;
-            bq[v] = uR[v] + (double)xr;
+            a[v] = p.U[(size_t)cL * NV + v] + (double)p.uleft[oL + v];
+            bq[v] = bnd ? 0.0 : p.U[(size_t)cR * NV + v] + (double)p.uleft[oR + v];
+            Fb[v] = lam[(size_t)cL * NV + v] - (bnd ? 0.0 : lam[(size_t)cR * NV + v]);
         }
+        double hb0[NV];
+        rotf(Fb, c1, s1, c2, s2, hb0);
         if (bnd) ghost_state(-cR, p.bc.boundtype, p.gamma, a, c1, s1, c2, s2, p.bc.inflow, p.bc.outflow, bq);
         double la[NV], ra[NV];
         rotf(a, c1, s1, c2, s2, la);
@@ -3549,36 +3539,53 @@ __global__ __launch_bounds__(256) void k_flux_vjp(FluxParams<R> p, const double 
                 double d = 0.0;
 #pragma unroll
                 for (int v = 0; v < NV; ++v) d += bb[v] * G[v].d;
-                ab[m] += d;
+#pragma unroll
+                for (int v = 0; v < NV; ++v) ab[v] += m == v ? d : 0.0;
             }
             if (bcbar && (code == 1 || code == 2 || code == 6)) {
+                // an inflow face reads the inflow state only, an outflow face
+                // the outflow state, a farfield face either
 #pragma unroll 1
-                for (int m = 0; m < 2 * NV; ++m) {
-                    Dual A[NV], G[NV], fi[NV], fo[NV];
+                for (int m = code == 2 ? NV : 0; m < (code == 1 ? NV : 2 * NV); ++m) {
+                    Dual A[NV], G[NV], fin[NV], fo[NV];
 #pragma unroll
                     for (int v = 0; v < NV; ++v) {
                         A[v] = Dual{a[v], 0.0};
-                        fi[v] = Dual{p.bc.inflow[v], m == v ? 1.0 : 0.0};
+                        fin[v] = Dual{p.bc.inflow[v], m == v ? 1.0 : 0.0};
                         fo[v] = Dual{p.bc.outflow[v], m == NV + v ? 1.0 : 0.0};
                     }
-                    ghost_state(code, p.bc.boundtype, p.gamma, A, c1, s1, c2, s2, fi, fo, G);
+                    ghost_state(code, p.bc.boundtype, p.gamma, A, c1, s1, c2, s2, fin, fo, G);
                     double d = 0.0;
 #pragma unroll
                     for (int v = 0; v < NV; ++v) d += bb[v] * G[v].d;
-                    bcacc[m] += d;
+#pragma unroll
+                    for (int e = 0; e < 2 * NV; ++e) bcacc[e] += m == e ? d : 0.0;
                 }
             }
         } else {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) obR[q * NV + v] = bb[v];
+            for (int v = 0; v < NV; ++v) ubf[oR + v] = bb[v];
         }
 #pragma unroll
-        for (int v = 0; v < NV; ++v) obL[q * NV + v] = ab[v];
-    }
-    if (bcbar && bnd) {
+        for (int v = 0; v < NV; ++v) ubf[oL + v] = ab[v];
+    };
+    if (f < p.nface) point();
+    if constexpr (BND) {
+        if (!bcbar) return;
+        __shared__ double sh[256 / WAVE][2 * NV];
 #pragma unroll
-        for (int m = 0; m < 2 * NV; ++m)
-            if (bcacc[m] != 0.0) atomic_add_f64(&bcbar[m], bcacc[m]);
+        for (int m = 0; m < 2 * NV; ++m) {
+            double x = bcacc[m];
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, WAVE);
+            if ((threadIdx.x & (WAVE - 1)) == 0) sh[threadIdx.x / WAVE][m] = x;
+        }
+        __syncthreads();
+        if (threadIdx.x < 2 * NV) {
+            double x = 0.0;
+            for (int wv = 0; wv < 256 / WAVE; ++wv) x += sh[wv][threadIdx.x];
+            if (x != 0.0) atomic_add_f64(&bcbar[threadIdx.x], x);
+        }
     }
 }
 
@@ -3857,7 +3864,8 @@ struct ucns_ctx {
     int smode = 0;      // stencils per cell of the row-stream kernel in use (0: none)
     bool needs_bc = false, have_bc = false;  // boundary codes 1/2/6 present; ucns_set_boundary called
     double *bface = nullptr;  // [nface][10] per-face INFLOW(), OUTFLOW() states (ucns_set_boundary_faces)
-    bool has_bnd_faces = false;              // any face with a ghost state (codes 1/2/3/4/6)
+    int nbface = 0;             // faces with a ghost state (codes 1/2/3/4/6)
+    int32_t *bfaces = nullptr;  // [nbface] their ids
     ucns_boundary_v1 bc{};
     int ntile = 0;
     // mesh (device)
@@ -4465,7 +4473,7 @@ int ensure_adjoint(ucns_ctx *ctx) {
 
 // the member tables of the last scatter into ubar
 void adj_gather(ucns_ctx *ctx, double *ubar) {
-    hipLaunchKernelGGL(k_adj_gather, dim3((ctx->ncell + 255) / 256), dim3(256), 0, ctx->stream, ctx->ncell,
+    hipLaunchKernelGGL(k_adj_gather, dim3((ctx->ncell + 31) / 32), dim3(256), 0, ctx->stream, ctx->ncell,
                        ctx->adj_off, ctx->adj_ent, ctx->adj_tab, ubar);
 }
 
@@ -4559,18 +4567,19 @@ int vjp_products_t(ucns_ctx *ctx, const double *lam, double *ubar, double *bcbar
     fp.wt = ctx->wquad + 64;
     fp.bc = ctx->bc;
     tstart(ctx, 1);
-    hipLaunchKernelGGL((k_flux_vjp<R, false>), dim3((ctx->nface + 255) / 256), dim3(256), 0, ctx->stream, fp, lam,
-                       ctx->adj_ubf, bcbar);
-    if (ctx->has_bnd_faces)
-        hipLaunchKernelGGL((k_flux_vjp<R, true>), dim3((ctx->nface + 255) / 256), dim3(256), 0, ctx->stream, fp, lam,
-                       ctx->adj_ubf, bcbar);
+    auto blocks = [&](int faces) { return dim3((unsigned)(((size_t)faces * ctx->nqm + 255) / 256)); };
+    hipLaunchKernelGGL((k_flux_vjp<R, false>), blocks(ctx->nface), dim3(256), 0, ctx->stream, fp,
+                       (const int32_t *)nullptr, 0, lam, ctx->adj_ubf, bcbar);
+    if (ctx->nbface)
+        hipLaunchKernelGGL((k_flux_vjp<R, true>), blocks(ctx->nbface), dim3(256), 0, ctx->stream, fp, ctx->bfaces,
+                           ctx->nbface, lam, ctx->adj_ubf, bcbar);
     tstop(ctx, 1);
     tcollect(ctx, 1, &ctx->st.ms_flux_vjp, &ctx->st.n_flux_vjp);
     if constexpr (sizeof(R) == 8) {
         if (ctx->geo_on) {
             hipLaunchKernelGGL(k_flux_geom<false>, dim3((ctx->nface + 255) / 256), dim3(256), 0, ctx->stream, fp, lam,
                                ctx->ovol, ctx->geo_area, ctx->geo_nrm, ctx->geo_ovol);
-            if (ctx->has_bnd_faces)
+            if (ctx->nbface)
                 hipLaunchKernelGGL(k_flux_geom<true>, dim3((ctx->nface + 255) / 256), dim3(256), 0, ctx->stream, fp,
                                    lam, ctx->ovol, ctx->geo_area, ctx->geo_nrm, ctx->geo_ovol);
         }
@@ -5224,7 +5233,7 @@ int ucns_create(const ucns_mesh_v2 *m, const ucns_scheme_v2 *s, ucns_ctx **out) 
     std::vector<int32_t> cinfo(nc, 0), cnb((size_t)nc * nf, -1), cface((size_t)nc * nf, 0);
     std::vector<int32_t> chnb(ctx->wenwrt == 2 ? (size_t)nc * nf : 0, 0);
     std::vector<double> chang(ctx->wenwrt == 2 ? (size_t)nc * nf * 4 : 0, 0.0);
-    std::vector<int32_t> fcell, fslot;
+    std::vector<int32_t> fcell, fslot, bfaces;
     std::vector<double> frot, farea;
     for (int i = 0; i < nc; ++i) {
         const int ifca = m->ifca[i];
@@ -5248,9 +5257,9 @@ int ucns_create(const ucns_mesh_v2 *m, const ucns_scheme_v2 *s, ucns_ctx **out) 
             if (bc == 1 || bc == 2 || bc == 3 || bc == 4 || bc == 6) {
                 // boundary face: owner only, the right state is a ghost (BOUNDARYS)
                 if (bc != 3 && bc != 4) ctx->needs_bc = true;
-                ctx->has_bnd_faces = true;
                 cnb[(size_t)i * nf + f] = -1;
                 const int id = (int)farea.size();
+                bfaces.push_back(id);
                 fcell.push_back(i);
                 fcell.push_back(-bc);
                 fslot.push_back(f | (m->types_faces[sl] == 6 ? 256 : 0));
@@ -5293,6 +5302,7 @@ int ucns_create(const ucns_mesh_v2 *m, const ucns_scheme_v2 *s, ucns_ctx **out) 
         }
     }
     ctx->nface = (int)farea.size();
+    ctx->nbface = (int)bfaces.size();
     ctx->h_cinfo_base = cinfo;
     std::vector<double> ovol(nc), minedge(nc);
     for (int i = 0; i < nc; ++i) {
@@ -5323,6 +5333,10 @@ int ucns_create(const ucns_mesh_v2 *m, const ucns_scheme_v2 *s, ucns_ctx **out) 
         (rc = dalloc(ctx, &ctx->marks_part, 2 * NPART)) || (rc = dalloc(ctx, &ctx->flag, 1)) ||
         (rc = dalloc(ctx, &ctx->stage, (size_t)nc * NV)))
         return rc;
+    if (!bfaces.empty()) {
+        if ((rc = dalloc(ctx, &ctx->bfaces, bfaces.size()))) return rc;
+        HIP_TRY(hipMemcpy(ctx->bfaces, bfaces.data(), bfaces.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    }
     if (!ctx->h_perm.empty()) {
         if ((rc = dalloc(ctx, &ctx->perm, nc))) return rc;
         HIP_TRY(hipMemcpy(ctx->perm, ctx->h_perm.data(), nc * sizeof(int32_t), hipMemcpyHostToDevice));
@@ -6235,6 +6249,7 @@ void ucns_destroy(ucns_ctx *ctx) {
     dfree(ctx->dtfix);
     dfree(ctx->dtv);
     dfree(ctx->marks_part);
+    dfree(ctx->bfaces);
     dfree(ctx->flag);
     dfree(ctx->uleft);
     for (auto &e : ctx->ev)
