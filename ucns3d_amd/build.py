@@ -14,6 +14,8 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(HERE)
@@ -27,10 +29,12 @@ FC = os.environ.get("FC", "/opt/rocm/bin/amdflang")
 
 # packed-FP32 instructions are disabled for every HIP translation unit
 HIP_FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++20", "-fPIC", "-shared",
+    "--offload-arch=gfx950", "-O3", "-std=c++20", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-munsafe-fp-atomics",
 ]
+# translation units of libucnsgpu.so, compiled side by side
+HIP_SOURCES = ["ucns_gpu.hip", "recon_muscl.hip"]
 
 
 def _run(cmd: list[str]) -> None:
@@ -52,8 +56,12 @@ def build_prep() -> str:
 def build_gpu() -> str:
     os.makedirs(LIBDIR, exist_ok=True)
     out = os.path.join(LIBDIR, "libucnsgpu.so")
-    src = os.path.join(CSRC, "ucns_gpu.hip")
-    _run([HIPCC, *HIP_FLAGS, "-I" + INCLUDE, src, "-o", out + ".tmp"])
+    with tempfile.TemporaryDirectory(dir=LIBDIR) as tmp:
+        objs = [os.path.join(tmp, src + ".o") for src in HIP_SOURCES]
+        with ThreadPoolExecutor(len(objs)) as pool:
+            list(pool.map(lambda so: _run([HIPCC, *HIP_FLAGS, "-I" + INCLUDE, "-c", os.path.join(CSRC, so[0]),
+                                           "-o", so[1]]), zip(HIP_SOURCES, objs)))
+        _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", out + ".tmp"])
     os.replace(out + ".tmp", out)
     return out
 
