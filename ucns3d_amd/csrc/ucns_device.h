@@ -15,6 +15,13 @@ namespace ucns {
 constexpr int NV = 5;
 constexpr int WAVE = 64;
 constexpr int NXCD = 8;
+// distinct stencil members of a tile held in LDS by the residual product's scatter
+#define UCNS_TILE_UQ 512
+#define UCNS_NOSLOT 0xFFFFu
+// rows of a tile's member table: 8 neighbouring cells share about 343
+// distinct members with WENO-4 on tets (5 stencils), 373 with WENO-3 on
+// hexes, 660 with WENO-4 on hexes (7 stencils of 39 members)
+constexpr int tile_uq(int ts, int imax) { return ts > 5 && imax > 19 ? 768 : UCNS_TILE_UQ; }
 constexpr int NPART = 64;  // blocks (and results) of k_marks_sum
 // monomial exponents of BASIS_REC (src/basis.f90:11-102), cubic max here
 static __constant__ int8_t c_mono[34][3] = {
@@ -409,6 +416,12 @@ struct ReconWParams {
     const R *Bc;
     const R *dmb;
     int wenoz;
+    // characteristic WENO (wenwrt 2): as in ReconParams
+    const int32_t *chnb;   // [ncell][nf]
+    const double *chang;   // [ncell][nf][4]
+    ucns_boundary_v1 bc;
+    const int32_t *cface;
+    const double *bface;
 };
 
 template <typename T>
