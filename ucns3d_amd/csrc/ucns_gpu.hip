@@ -723,8 +723,36 @@ __device__ inline void hllc_t(double gamma, const T *cl, const T *cr, T *flux) {
         flux[k] = (((1.0 + s) / 2.0) * (fl[k] + sl * (usl[k] - cl[k]))) +
                   (((1.0 - s) / 2.0) * (fr[k] + sr * (usr[k] - cr[k])));
 }
+// The FP64 solver of the flux kernels: hllc_t, term by term, with only the side
+// that sign(S_M) picks evaluated (the other is multiplied by 0 there).  The
+// kernels spend most of their vector time in FP64 divisions and square roots:
+// 11 and 5 of them here, 14 and 5 in hllc_t.
 __device__ inline void hllc64(double gamma, const double *cl, const double *cr, double *flux) {
-    hllc_t<double>(gamma, cl, cr, flux);
+    double wl[NV], wr[NV];
+    cons2prim_d(gamma, cl, wl);
+    cons2prim_d(gamma, cr, wr);
+    const double rl = wl[0], uL = wl[1], pl = wl[4], rr = wr[0], uR = wr[1], pr = wr[4];
+    const double ccl = sqrt(gamma * pl / rl), ccr = sqrt(gamma * pr / rr);
+    const double srl = sqrt(rl), srr = sqrt(rr);
+    const double cc2 = sqrt((((ccl * ccl) * srl) + ((ccr * ccr) * srr)) / (srl + srr) +
+                            (0.5 * ((srl * srr) / ((srl + srr) * (srl + srr))) * ((uR - uL) * (uR - uL))));
+    const double uu2 = ((uL * srl) + (uR * srr)) / (srl + srr);
+    const double sl = fmin(fmin(uL - ccl, uu2 - cc2), 0.0), sr = fmax(fmax(uR + ccr, uu2 + cc2), 0.0);
+    const double sm = (pr - pl + (rl * uL * (sl - uL)) - (rr * uR * (sr - uR))) / ((rl * (sl - uL)) - (rr * (sr - uR)));
+    const bool left = copysign(1.0, sm) > 0.0;
+    double ck[NV], wk[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        ck[v] = left ? cl[v] : cr[v];
+        wk[v] = left ? wl[v] : wr[v];
+    }
+    const double sk = left ? sl : sr, rk = wk[0], uk = wk[1], pk = wk[4], ek = ck[4];
+    const double fk[NV] = {rk * uk, (rk * (uk * uk)) + pk, rk * uk * wk[2], rk * uk * wk[3], uk * (ek + pk)};
+    const double mu = rk * ((sk - uk) / (sk - sm));
+    const double last = (ek / rk) + ((sm - uk) * (sm + ((pk) / (rk * (sk - uk)))));
+    const double us[NV] = {mu, mu * sm, mu * wk[2], mu * wk[3], mu * last};
+#pragma unroll
+    for (int k = 0; k < NV; ++k) flux[k] = fk[k] + sk * (us[k] - ck[k]);
 }
 
 // Reverse mode of hllc_t (FP64): given the flux cotangent hb, the cotangents
@@ -1011,6 +1039,74 @@ __global__ __launch_bounds__(256) void k_flux(FluxParams<R> p) {
     }
 #pragma unroll
     for (int v = 0; v < NV; ++v) p.fflux[(size_t)f * NV + v] = acc[v];
+}
+
+// The same with one thread per (face, quadrature point), for meshes whose
+// faces do not fill the chip and whose faces have several points: nqm times
+// the waves, and a point's chain of divisions and square roots runs beside the
+// others' instead of after them.  The points' contributions meet in LDS, where
+// thread (face, variable) adds them in point order (the order and rounding of
+// the one-thread loop).  5,184 hexahedra faces of 9 points: 18.8 -> 6.2 us; on
+// 256,000 and more faces it is slower by 3-7% (rule at the launch).
+template <typename R>
+__global__ __launch_bounds__(256) void k_flux_points(FluxParams<R> p) {
+    __shared__ double sh[256][NV + 1];  // per point: the rotated-back flux and its weight times the area
+    const int fpb = 256 / p.nqm;        // faces of a block (nqm <= 24: 6 nqm <= 96 points per cell, 4 faces at least)
+    const int f0 = blockIdx.x * fpb;
+    const int fl = threadIdx.x / p.nqm, q = threadIdx.x - fl * p.nqm;
+    const int f = f0 + fl;
+    auto point = [&]() {
+        const int s0 = p.fslot[2 * f];
+        const bool tri = (s0 >> 8) & 1;
+        if (q >= (tri ? p.qpt : p.qpq)) return;
+        const int cL = p.fcell[2 * f], cR = p.fcell[2 * f + 1];
+        const int sL = s0 & 255, sR = p.fslot[2 * f + 1];
+        const double *w = tri ? p.wt : p.wq;
+        const double c1 = p.frot[4 * f], s1 = p.frot[4 * f + 1], c2 = p.frot[4 * f + 2], s2 = p.frot[4 * f + 3];
+        const double area = p.farea[f];
+        const bool bnd = cR < 0;  // boundary face: -code
+        const size_t oL = (((size_t)cL * p.nf + sL) * p.nqm + q) * NV;
+        const size_t oR = bnd ? oL : (((size_t)cR * p.nf + sR) * p.nqm + q) * NV;
+        double a[NV], bq[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            a[v] = p.U[(size_t)cL * NV + v] + (double)p.uleft[oL + v];
+            bq[v] = bnd ? 0.0 : p.U[(size_t)cR * NV + v] + (double)p.uleft[oR + v];
+        }
+        if (bnd) {
+            const double *fin = p.bface ? p.bface + (size_t)f * 10 : p.bc.inflow;
+            const double *fout = p.bface ? p.bface + (size_t)f * 10 + 5 : p.bc.outflow;
+            ghost_state(-cR, p.bc.boundtype, p.gamma, a, c1, s1, c2, s2, fin, fout, bq);  // GET_STATES_BOUNDS
+        }
+        // ROTATEF (src/grid_t.f90:4217-4258)
+        const double la[NV] = {a[0], c1 * s2 * a[1] + s1 * s2 * a[2] + c2 * a[3],
+                               c1 * c2 * a[1] + s1 * c2 * a[2] + (-s2) * a[3], (-s1) * a[1] + c1 * a[2], a[4]};
+        const double ra[NV] = {bq[0], c1 * s2 * bq[1] + s1 * s2 * bq[2] + c2 * bq[3],
+                               c1 * c2 * bq[1] + s1 * c2 * bq[2] + (-s2) * bq[3], (-s1) * bq[1] + c1 * bq[2], bq[4]};
+        double hd[NV];
+        if (sizeof(R) == 8)
+            hllc64(p.gamma, la, ra, hd);
+        else
+            hllc32(p.gamma, la, ra, hd);
+        // ROTATEB (src/grid_t.f90:4261-4305)
+        double *o = sh[threadIdx.x];
+        o[0] = hd[0];
+        o[1] = c1 * s2 * hd[1] + c1 * c2 * hd[2] + (-s1) * hd[3];
+        o[2] = s1 * s2 * hd[1] + s1 * c2 * hd[2] + c1 * hd[3];
+        o[3] = c2 * hd[1] + (-s2) * hd[2];
+        o[4] = hd[4];
+        o[NV] = w[q] * area;
+    };
+    if (fl < fpb && f < p.nface) point();
+    __syncthreads();
+    const int nfb = min(fpb, p.nface - f0);
+    for (int e = threadIdx.x; e < nfb * NV; e += 256) {
+        const int i = e / NV, v = e - i * NV;
+        const int nq = (p.fslot[2 * (f0 + i)] >> 8) & 1 ? p.qpt : p.qpq;
+        double acc = 0.0;
+        for (int u = 0; u < nq; ++u) acc = acc + (sh[i * p.nqm + u][v] * sh[i * p.nqm + u][NV]);
+        p.fflux[(size_t)f0 * NV + e] = acc;
+    }
 }
 
 struct UpdateParams {
@@ -2842,7 +2938,17 @@ void launch_flux_t(ucns_ctx *ctx) {
     p.wt = ctx->wquad + 64;
     p.bc = ctx->bc;
     p.bface = ctx->bface;
-    hipLaunchKernelGGL((k_flux<R>), dim3((ctx->nface + 255) / 256), dim3(256), 0, ctx->stream, p);
+    // Half of the threads the chip holds at the kernel's registers (2^18): below
+    // it a thread per point wins (5,184 hexahedra faces 18.8 -> 6.2 us, 31,000
+    // channel faces 15.9 -> 9 us), well above it a thread per face (280,000
+    // channel faces 52 us against 54, 393,000 tetrahedra faces 93 against 100).
+    // Faces of one point gain nothing from it (5.7 against 7.9 us on 41,472).
+    if (ctx->nqm > 1 && ctx->nface < 131072) {
+        const int fpb = 256 / ctx->nqm;  // faces per block
+        hipLaunchKernelGGL((k_flux_points<R>), dim3((ctx->nface + fpb - 1) / fpb), dim3(256), 0, ctx->stream, p);
+    } else {
+        hipLaunchKernelGGL((k_flux<R>), dim3((ctx->nface + 255) / 256), dim3(256), 0, ctx->stream, p);
+    }
 }
 
 void tstart(ucns_ctx *ctx, int k) {
