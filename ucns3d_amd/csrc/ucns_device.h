@@ -54,13 +54,6 @@ struct ReconParams {
     const int32_t *cnb;    // [ncell][nf] face neighbours
     R *uleft;              // [ncell][nf][nqm][5]
     int *marks;            // [ncell] per block: MUSCL cells + 65536 * first-order cells (k_marks_sum)
-    // CWENO (ees 5) in the per-cell kernel: P holds the central stencil only
-    // ([ncell][imax][ideg]); the sectors' low-order pseudo-inverses, their
-    // indicators (packed) and mbar - mbar_c over their coefficients
-    const R *Pc;           // [ncell][ts-1][imax2][ideg2]
-    const R *Bc;           // [ncell][ideg2*(ideg2+1)/2]
-    const R *dmb;          // [ncell][ideg2]
-    int wenoz;
     // characteristic WENO (wenwrt 2): per cell face the neighbour (negative:
     // the boundary code) and the cell's own face angles (cos a1, sin a1, cos
     // a2, sin a2); the free-stream data of the boundary ghosts

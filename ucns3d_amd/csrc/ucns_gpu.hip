@@ -52,16 +52,11 @@ namespace {
         }                                                                                   \
     } while (0)
 
-// CWS: the CWENO layout, the sectors' rows compact (IM2 members, ID2
-// coefficients each) and the indicator packed (upper triangle by rows)
-template <typename R, int IDEG, int IMAX, int TSMAX, bool CWS = false, int ID2 = 9, int IM2 = 19>
+template <typename R, int IDEG, int IMAX, int TSMAX>
 struct ReconShared {
     static constexpr int NQMAX = 6 * 16;
-    static constexpr int DU = CWS ? IMAX + (TSMAX - 1) * IM2 : TSMAX * IMAX;
-    static constexpr int GN = CWS ? IDEG + (TSMAX - 1) * ID2 : TSMAX * IDEG;
-    static constexpr int BN = CWS ? IDEG * (IDEG + 1) / 2 : IDEG * IDEG;
     union {
-        R du[DU * NV];  // phase 1
+        R du[TSMAX * IMAX * NV];  // phase 1
         struct {
             R gh[IDEG * NV];         // combined polynomial
             R beta[TSMAX * NV];
@@ -69,27 +64,19 @@ struct ReconShared {
             R ul[NQMAX * NV];        // face-point values
         } late;
     } u;
-    R g[GN * NV];                    // per-stencil coefficients
-    R b[BN];                         // indicator, unpacked (CWS: packed)
+    R g[TSMAX * IDEG * NV];                 // per-stencil coefficients
+    R b[IDEG * IDEG];                // indicator, unpacked
     R mb[IDEG];
     double ui[NV];
-    // CWENO: the sectors' indicator (unpacked), the indicators in FP64 and
-    // the face-value shift of the sectors' low-order means
-    R bc[9 * 9];
-    double betad[TSMAX * NV];
-    R corr[NV];
 };
 
-// Fused reconstruction, one wavefront per cell.  CW: CWENO with sectors of
-// ID2 coefficients over their first IM2 members (src/reconstruct_p.f90:955-1049).
+// Fused reconstruction, one wavefront per cell: WENO-5, and shapes and face
+// rules the tiled kernels do not hold.
 // CH: characteristic-variable WENO, face by face (src/reconstruct_p.f90:497-758).
-template <typename R, int IDEG, int IMAX, int TSMAX, bool CW = false, int ID2 = 9, int IM2 = 19, bool CH = false>
-__global__ __launch_bounds__(WAVE, CW ? 2 : 1) void k_recon(ReconParams<R> p) {
-    static_assert(!CW || (ID2 <= 9 && IM2 <= IMAX), "CWENO sectors: at most 9 coefficients");
+template <typename R, int IDEG, int IMAX, int TSMAX, bool CH = false>
+__global__ __launch_bounds__(WAVE) void k_recon(ReconParams<R> p) {
     constexpr int NROW = (TSMAX * IDEG + WAVE - 1) / WAVE;
-    __shared__ ReconShared<R, IDEG, IMAX, TSMAX, CW, ID2, IM2> sh;
-    // CWENO: row of sector s >= 1's coefficient k in sh.g
-    auto crow = [](int s, int k) { return IDEG + (s - 1) * ID2 + k; };
+    __shared__ ReconShared<R, IDEG, IMAX, TSMAX> sh;
     const int lane = threadIdx.x;
     // XCD-aware order: consecutive blocks go to different XCDs, so give
     // each XCD a contiguous range of cells (its L2 then holds the
@@ -109,36 +96,12 @@ __global__ __launch_bounds__(WAVE, CW ? 2 : 1) void k_recon(ReconParams<R> p) {
 
     // ---- phase 0: dU of every stencil member (FP64, then rounded to R) ----
     const int32_t *nb = p.nbr + (size_t)cell * ts * IMAX;
-    if constexpr (CW) {
-        // the central stencil's IMAX members, then each sector's first IM2
-        for (int e = lane; e < IMAX + (admis - 1) * IM2; e += WAVE) {
-            const int m = e < IMAX ? e : ((e - IMAX) / IM2 + 1) * IMAX + (e - IMAX) % IM2;
-            const double *Un = p.U + (size_t)nb[m] * NV;
+    for (int e = lane; e < admis * IMAX; e += WAVE) {
+        const double *Un = p.U + (size_t)nb[e] * NV;
 #pragma unroll
-            for (int v = 0; v < NV; ++v) sh.u.du[e * NV + v] = (R)(Un[v] - ui[v]);
-        }
-        const R *bcp = p.Bc + (size_t)cell * (ID2 * (ID2 + 1) / 2);
-        for (int e = lane; e < ID2 * (ID2 + 1) / 2; e += WAVE) {
-            int k = 0, base = 0;
-            while (e >= base + (ID2 - k)) {
-                base += ID2 - k;
-                ++k;
-            }
-            const int l = k + (e - base);
-            sh.bc[k * ID2 + l] = bcp[e];
-            sh.bc[l * ID2 + k] = bcp[e];
-        }
-    } else {
-        for (int e = lane; e < admis * IMAX; e += WAVE) {
-            const double *Un = p.U + (size_t)nb[e] * NV;
-#pragma unroll
-            for (int v = 0; v < NV; ++v) sh.u.du[e * NV + v] = (R)(Un[v] - ui[v]);
-        }
+        for (int v = 0; v < NV; ++v) sh.u.du[e * NV + v] = (R)(Un[v] - ui[v]);
     }
-    if (CW) {
-        const R *Bc = p.B + (size_t)cell * (IDEG * (IDEG + 1) / 2);
-        for (int e = lane; e < IDEG * (IDEG + 1) / 2; e += WAVE) sh.b[e] = Bc[e];
-    } else if (p.iweno == 1) {
+    {
         const R *Bc = p.B + (size_t)cell * (IDEG * (IDEG + 1) / 2);
         for (int e = lane; e < IDEG * (IDEG + 1) / 2; e += WAVE) {
             // packed upper triangle by rows: row k holds l = k..IDEG-1
@@ -157,166 +120,42 @@ __global__ __launch_bounds__(WAVE, CW ? 2 : 1) void k_recon(ReconParams<R> p) {
     __syncthreads();
 
     // ---- phase 1: G_s = P_s dU_s, one (stencil,coefficient) row per lane ----
-    if constexpr (CW) {
-        // rows 0..IDEG-1: the central stencil; then ID2 rows per sector
-        constexpr int NROWC = (IDEG + (TSMAX - 1) * ID2 + WAVE - 1) / WAVE;
-        const int nrows = IDEG + (admis - 1) * ID2;
-        const R *Pcen = p.P + (size_t)cell * IMAX * IDEG;
-        const R *Psec = p.Pc + (size_t)cell * (ts - 1) * IM2 * ID2;
+    R acc[NROW][NV];
+    int srow[NROW];
 #pragma unroll
-        for (int t = 0; t < NROWC; ++t) {
-            const int r = lane + t * WAVE;
-            if (r >= nrows) continue;
-            R acc[NV] = {R(0), R(0), R(0), R(0), R(0)};
-            if (r < IDEG) {
-                for (int j = 0; j < IMAX; ++j) {
-                    const R pv = Pcen[(size_t)j * IDEG + r];
-                    const R *du = &sh.u.du[j * NV];
+    for (int t = 0; t < NROW; ++t) {
+        srow[t] = (lane + t * WAVE) / IDEG;
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) acc[v] += pv * du[v];
-                }
-#pragma unroll
-                for (int v = 0; v < NV; ++v) sh.g[r * NV + v] = acc[v];
-            } else {
-                const int sec = (r - IDEG) / ID2, k = (r - IDEG) % ID2;
-                const R *Ps = Psec + (size_t)sec * IM2 * ID2;
-                for (int j = 0; j < IM2; ++j) {
-                    const R pv = Ps[(size_t)j * ID2 + k];
-                    const R *du = &sh.u.du[(IMAX + sec * IM2 + j) * NV];
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) acc[v] += pv * du[v];
-                }
-#pragma unroll
-                for (int v = 0; v < NV; ++v) sh.g[crow(sec + 1, k) * NV + v] = acc[v];
-            }
-        }
-    } else {
-        R acc[NROW][NV];
-        int srow[NROW];
-#pragma unroll
-        for (int t = 0; t < NROW; ++t) {
-            srow[t] = (lane + t * WAVE) / IDEG;
-#pragma unroll
-            for (int v = 0; v < NV; ++v) acc[t][v] = R(0);
-        }
-        const int nrows = admis * IDEG;
-        const R *Pc = p.P + (size_t)cell * IMAX * ts * IDEG;
+        for (int v = 0; v < NV; ++v) acc[t][v] = R(0);
+    }
+    const int nrows = admis * IDEG;
+    const R *Pc = p.P + (size_t)cell * IMAX * ts * IDEG;
 #pragma unroll 4
-        for (int j = 0; j < IMAX; ++j) {
-            const R *Pj = Pc + (size_t)j * ts * IDEG;
-#pragma unroll
-            for (int t = 0; t < NROW; ++t) {
-                const int r = lane + t * WAVE;
-                if (r < nrows) {
-                    const R pv = Pj[r];
-                    const R *du = &sh.u.du[(srow[t] * IMAX + j) * NV];
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) acc[t][v] += pv * du[v];
-                }
-            }
-        }
+    for (int j = 0; j < IMAX; ++j) {
+        const R *Pj = Pc + (size_t)j * ts * IDEG;
 #pragma unroll
         for (int t = 0; t < NROW; ++t) {
             const int r = lane + t * WAVE;
             if (r < nrows) {
+                const R pv = Pj[r];
+                const R *du = &sh.u.du[(srow[t] * IMAX + j) * NV];
 #pragma unroll
-                for (int v = 0; v < NV; ++v) sh.g[r * NV + v] = acc[t][v];
+                for (int v = 0; v < NV; ++v) acc[t][v] += pv * du[v];
             }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NROW; ++t) {
+        const int r = lane + t * WAVE;
+        if (r < nrows) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) sh.g[r * NV + v] = acc[t][v];
         }
     }
     __syncthreads();
 
     bool reduce = (full == 0);
     const int nslot = ifca * p.nqm;
-    if constexpr (CW) {
-        // ---- CWENO: the zero polynomial (G_1 - sum_l lambda_l G_l) / lambda_1,
-        // lambda_1 = 1 - 1/LWCI1, lambda_l = (1 - lambda_1)/(ADMIS-1) ----
-        const double lam0 = 1.0 - (1.0 / p.lwci1);
-        const double laml = admis > 1 ? (1.0 - lam0) / (admis - 1) : 0.0;
-        for (int e = lane; e < IDEG * NV; e += WAVE) {
-            const int k = e / NV, v = e % NV;
-            R sl = R(0);
-            if (k < ID2)
-                for (int s = 1; s < admis; ++s) sl += (R)laml * sh.g[crow(s, k) * NV + v];
-            sh.u.late.gh[e] = (R)(1.0 / lam0) * (sh.g[e] - sl);
-        }
-        __syncthreads();
-        // indicators: the zero polynomial's with INDICATOR, a sector's with INDICATORC
-        if (lane < admis * NV) {
-            const int s = lane / NV, v = lane % NV;
-            double beta = 0.0;
-            if (s == 0) {
-                // over the packed triangle: sum_k z_k (B_kk z_k + 2 sum_{l>k} B_kl z_l)
-                int e = 0;
-                for (int k = 0; k < IDEG; ++k) {
-                    const double zk = (double)sh.u.late.gh[k * NV + v];
-                    double bg = 0.0;
-                    for (int l = k + 1; l < IDEG; ++l) bg += (double)sh.b[e + l - k] * (double)sh.u.late.gh[l * NV + v];
-                    beta += zk * ((double)sh.b[e] * zk + 2.0 * bg);
-                    e += IDEG - k;
-                }
-            } else {
-                const R *gs = &sh.g[crow(s, 0) * NV + v];
-#pragma unroll
-                for (int k = 0; k < ID2; ++k) {
-                    double bg = 0.0;
-#pragma unroll
-                    for (int l = 0; l < ID2; ++l) bg += (double)sh.bc[k * ID2 + l] * (double)gs[l * NV];
-                    beta += (double)gs[k * NV] * bg;
-                }
-            }
-            sh.betad[lane] = beta;
-        }
-        __syncthreads();
-        // weights in FP64: WENO (power 4) or WENO-Z, tau = sum_l |beta_1 - beta_l| / (ADMIS-1)
-        if (lane < admis * NV) {
-            const int s = lane / NV, v = lane % NV;
-            double tau = 0.0;
-            if (p.wenoz && admis > 1) {
-                for (int t = 1; t < admis; ++t) tau += fabs(sh.betad[v] - sh.betad[t * NV + v]);
-                tau /= (double)(admis - 1);
-            }
-            double sum = 0.0, mine = 0.0;
-            for (int t = 0; t < admis; ++t) {
-                const double lam = t == 0 ? lam0 : laml;
-                const double x = p.eps + sh.betad[t * NV + v];
-                double w;
-                if (p.wenoz) {
-                    const double r = tau / x, r2 = r * r;
-                    w = lam * (1.0 + r2 * r2);
-                } else {
-                    const double x2 = x * x;
-                    w = lam / (x2 * x2);
-                }
-                sum += w;
-                if (t == s) mine = w;
-            }
-            sh.u.late.omega[lane] = (R)(mine / sum);
-        }
-        __syncthreads();
-        // weighted polynomial on the high-order basis; the sectors' polynomials
-        // use the means of VALUEC: their weighted coefficients times
-        // (mbar - mbar_c) shift every face value alike
-        for (int e = lane; e < IDEG * NV; e += WAVE) {
-            const int k = e / NV, v = e % NV;
-            R acc = sh.u.late.omega[v] * sh.u.late.gh[e];
-            if (k < ID2)
-                for (int s = 1; s < admis; ++s) acc += sh.u.late.omega[s * NV + v] * sh.g[crow(s, k) * NV + v];
-            sh.u.late.gh[e] = acc;
-        }
-        if (lane < NV) {
-            const R *dm = p.dmb + (size_t)cell * ID2;
-            R c = R(0);
-#pragma unroll
-            for (int k = 0; k < ID2; ++k) {
-                R wg = R(0);
-                for (int s = 1; s < admis; ++s) wg += sh.u.late.omega[s * NV + lane] * sh.g[crow(s, k) * NV + lane];
-                c += dm[k] * wg;
-            }
-            sh.corr[lane] = c;
-        }
-        __syncthreads();
-    }
     if constexpr (CH) {
         // ---- characteristic WENO: per face, the eigenvectors of the averaged
         // cell / neighbour state in the face frame (WENO_NEIGHBOUR: the ghost of
@@ -418,8 +257,7 @@ __global__ __launch_bounds__(WAVE, CW ? 2 : 1) void k_recon(ReconParams<R> p) {
             __syncthreads();
         }
         reduce = reduce || (__syncthreads_or(trouble) != 0);
-    } else if (p.iweno == 1) {
-        if constexpr (!CW) {
+    } else {
         // ---- phase 2: beta_{s,v} = g^T (B g) (src/reconstruct_p.f90:995-1004) ----
         if (lane < admis * NV) {
             const int s = lane / NV, v = lane % NV;
@@ -476,7 +314,6 @@ __global__ __launch_bounds__(WAVE, CW ? 2 : 1) void k_recon(ReconParams<R> p) {
             sh.u.late.gh[e] = acc;
         }
         __syncthreads();
-        }
         // ---- phase 5: ULEFT at the face points + CHECKSOL (0.85) ----
         double wi[NV];
         cons2prim_d(p.gamma, ui, wi);
@@ -499,7 +336,6 @@ __global__ __launch_bounds__(WAVE, CW ? 2 : 1) void k_recon(ReconParams<R> p) {
                 R res = R(0);
 #pragma unroll
                 for (int k = 0; k < IDEG; ++k) res += phi[k] * sh.u.late.gh[k * NV + v];
-                if constexpr (CW) res += sh.corr[v];
                 // ULEFT is kept as the deviation from the FP64 cell average
                 uq[v] = ui[v] + (double)res;
                 sh.u.late.ul[e * NV + v] = res;
@@ -507,11 +343,7 @@ __global__ __launch_bounds__(WAVE, CW ? 2 : 1) void k_recon(ReconParams<R> p) {
             if (full && jump_test(p.gamma, wi, uq, 0.85)) trouble = 1;
         }
         reduce = reduce || (__syncthreads_or(trouble) != 0);
-    } else {
-        reduce = true;  // MUSCL scheme: every cell is non-FULL
-        __syncthreads();
     }
-
     // ---- phase 6: MUSCL + Barth-Jespersen (src/reconstruct_p.f90:2044-2280) ----
     if (reduce) {
         double umin[NV], umax[NV];
@@ -2709,8 +2541,11 @@ struct ucns_ctx {
     bool have_cweno = false;
     std::vector<double> h_cwP, h_cwB, h_cwIB;
     void *Bc = nullptr, *dmb = nullptr;
-    void *Pc = nullptr;     // per-cell kernel: the sectors' low-order pseudo-inverses [ncell][ts-1][imax2][ideg2]
-    bool cw_cell = false;   // CWENO on the per-cell kernel (WENO-5)
+    // CWENO at WENO-5 (its layouts: Cweno5Params): the sectors' low-order
+    // pseudo-inverses and members
+    void *Pc = nullptr;
+    int32_t *nbc = nullptr;
+    bool cw_cell = false;
     // library options of the scheme
     int kernels = UCNS_KERNELS_AUTO;
     int adj_keep_stages = 0;
@@ -2815,10 +2650,6 @@ int launch_recon_t(ucns_ctx *ctx) {
     p.cnb = ctx->cnb;
     p.uleft = (R *)ctx->uleft;
     p.marks = ctx->marks;
-    p.Pc = (const R *)ctx->Pc;
-    p.Bc = (const R *)ctx->Bc;
-    p.dmb = (const R *)ctx->dmb;
-    p.wenoz = ctx->wenoz;
     p.chnb = ctx->chnb;
     p.chang = ctx->chang;
     p.bc = ctx->bc;
@@ -2884,11 +2715,11 @@ int launch_recon_t(ucns_ctx *ctx) {
     if (ctx->wenwrt == 2) {
         // WENO-5, and face rules of more points than the tiled kernels hold
         if (ctx->ideg == 34 && ctx->imax == 69)
-            hipLaunchKernelGGL((k_recon<R, 34, 69, 7, false, 9, 19, true>), grid, block, 0, ctx->stream, p);
+            hipLaunchKernelGGL((k_recon<R, 34, 69, 7, true>), grid, block, 0, ctx->stream, p);
         else if (ctx->ideg == 19 && ctx->imax == 39)
-            hipLaunchKernelGGL((k_recon<R, 19, 39, 7, false, 9, 19, true>), grid, block, 0, ctx->stream, p);
+            hipLaunchKernelGGL((k_recon<R, 19, 39, 7, true>), grid, block, 0, ctx->stream, p);
         else if (ctx->ideg == 9 && ctx->imax == 19)
-            hipLaunchKernelGGL((k_recon<R, 9, 19, 7, false, 9, 19, true>), grid, block, 0, ctx->stream, p);
+            hipLaunchKernelGGL((k_recon<R, 9, 19, 7, true>), grid, block, 0, ctx->stream, p);
         else {
             ctx->err = "no characteristic reconstruction kernel for idegfree=" + std::to_string(ctx->ideg);
             return UCNS_EUNSUPPORTED;
@@ -2897,7 +2728,34 @@ int launch_recon_t(ucns_ctx *ctx) {
     }
     if (ctx->cw_cell) {
         if (ctx->ideg == 34 && ctx->imax == 69 && ctx->ideg2 == 9 && ctx->imax2 == 19) {
-            hipLaunchKernelGGL((k_recon<R, 34, 69, 7, true, 9, 19>), grid, block, 0, ctx->stream, p);
+            Cweno5Params<R> w{};
+            w.ncell = ctx->ncell;
+            w.ntile = ctx->ntile;
+            w.tiles_per_xcd = (ctx->ntile + NXCD - 1) / NXCD;
+            w.ts = ctx->ts;
+            w.nf = ctx->nf;
+            w.nqm = ctx->nqm;
+            w.qpq = ctx->qpq;
+            w.qpt = ctx->qpt;
+            w.wenoz = ctx->wenoz;
+            w.gamma = ctx->gamma;
+            w.lwci1 = ctx->lwci1;
+            w.eps = ctx->eps;
+            w.U = ctx->U;
+            w.nbr = ctx->nbr;
+            w.nbc = ctx->nbc;
+            w.P = (const R *)ctx->P;
+            w.Pc = (const R *)ctx->Pc;
+            w.B = (const R *)ctx->B;
+            w.Bc = (const R *)ctx->Bc;
+            w.dmb = (const R *)ctx->dmb;
+            w.mbar = (const R *)ctx->mbar;
+            w.qp = (const R *)ctx->qp;
+            w.cinfo = ctx->cinfo;
+            w.cnb = ctx->cnb;
+            w.uleft = (R *)ctx->uleft;
+            w.marks = ctx->marks;
+            launch_recon_cweno5(w, ctx->stream);
             return UCNS_OK;
         }
         ctx->err = "no CWENO kernel for idegfree=" + std::to_string(ctx->ideg) + " idegfree2=" +
@@ -3599,6 +3457,7 @@ int upload_real_any(ucns_ctx *ctx, void **dst, const std::vector<double> &src) {
 
 void release_prestore(ucns_ctx *ctx) {
     dfree(ctx->nbr);
+    dfree(ctx->nbc);
     dfree(ctx->P);
     dfree(ctx->rows);
     dfree(ctx->u64);
@@ -4166,14 +4025,21 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
         ctx->smode = stream_ok ? ts : 0;
     }
     ctx->ntile = (nc + 7) / 8;
-    ctx->nmark = ctx->tiled || ctx->iweno == -1 ? ctx->ntile : nc;
+    ctx->nmark = ctx->tiled || ctx->cw_cell || ctx->iweno == -1 ? ctx->ntile : nc;
     int rc = dalloc(ctx, &ctx->marks, (size_t)ctx->nmark);
     if (rc) return rc;
     HIP_TRY(hipMemset(ctx->marks, 0, (size_t)ctx->nmark * sizeof(int)));
     // stencil members without the cell itself
     //   tiled: [tile][imax][8*ts], lane position 8-cell-tile local
+    //   CWENO at WENO-5: central [tile][imax][8], sectors [tile][imax2][8*(ts-1)]
     //   plain: [cell][ts][imax]
-    std::vector<int32_t> nbr(ctx->smode ? (size_t)0 : ctx->tiled ? (size_t)ctx->ntile * IM * 8 * ts : (size_t)nc * ts * IM, 0);
+    const int IMC = ctx->cw_cell ? ctx->imax2 : 0, NS = std::max(ts - 1, 1);
+    std::vector<int32_t> nbc((size_t)ctx->ntile * IMC * 8 * NS, 0);
+    std::vector<int32_t> nbr(ctx->smode     ? (size_t)0
+                             : ctx->tiled   ? (size_t)ctx->ntile * IM * 8 * ts
+                             : ctx->cw_cell ? (size_t)ctx->ntile * IM * 8
+                                            : (size_t)nc * ts * IM,
+                             0);
     for (int i = 0; i < nc; ++i) {
         const size_t o = src_cell(ctx, i);
         for (int s = 0; s < pre->admis[o]; ++s) {
@@ -4194,6 +4060,11 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
                 } else if (ctx->tiled) {
                     const size_t TP = 8 * (size_t)ts;
                     nbr[((size_t)(i / 8) * IM + k) * TP + (size_t)(i % 8) * ts + s] = j;
+                } else if (ctx->cw_cell) {
+                    if (s == 0)
+                        nbr[((size_t)(i / 8) * IM + k) * 8 + i % 8] = j;
+                    else if (k < IMC)
+                        nbc[((size_t)(i / 8) * IMC + k) * 8 * NS + (size_t)(i % 8) * NS + s - 1] = j;
                 } else {
                     nbr[((size_t)i * ts + s) * IM + k] = j;
                 }
@@ -4203,12 +4074,16 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
     if ((rc = dalloc(ctx, &ctx->nbr, std::max<size_t>(nbr.size(), 1)))) return rc;
     if (!nbr.empty())
         HIP_TRY(hipMemcpy(ctx->nbr, nbr.data(), nbr.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    if (!nbc.empty()) {
+        if ((rc = dalloc(ctx, &ctx->nbc, nbc.size()))) return rc;
+        HIP_TRY(hipMemcpy(ctx->nbc, nbc.data(), nbc.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    }
     HIP_TRY(hipMemcpy(ctx->cinfo, cinfo.data(), nc * sizeof(int32_t), hipMemcpyHostToDevice));
-    // pseudo-inverses: staged in chunks, re-laid out on the device (CWENO on
-    // the per-cell kernel: the central stencil's only)
+    // pseudo-inverses: staged in chunks, re-laid out on the device (CWENO at
+    // WENO-5: the central stencil's only)
     const int tsP = ctx->cw_cell ? 1 : ts;
     const size_t per_cell_abi = (size_t)TSA * IM * ID, per_cell_dev = (size_t)IM * tsP * ID;
-    const size_t dev_elems = ctx->smode ? 1 : ctx->tiled ? (size_t)ctx->ntile * 8 * per_cell_dev : per_cell_dev * nc;
+    const size_t dev_elems = ctx->smode ? 1 : ctx->tiled || ctx->cw_cell ? (size_t)ctx->ntile * 8 * per_cell_dev : per_cell_dev * nc;
     rc = mixed ? dalloc(ctx, (float **)&ctx->P, dev_elems) : dalloc(ctx, (double **)&ctx->P, dev_elems);
     if (rc) return rc;
     const int sTP = 8 * ts, sD = stream_depth(mixed, ts), sPB = ID * sTP * (mixed ? 4 : 8);
@@ -4292,6 +4167,11 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
                 else
                     hipLaunchKernelGGL(k_tile_p<double>, dim3(blocks), dim3(256), 0, ctx->stream, stage,
                                        (double *)ctx->P + c0 * per_cell_dev, (int)c0, (int)cn, nc, TSA, ts, IM, ID);
+            } else if (ctx->cw_cell) {
+                if (mixed)
+                    cweno5_rows(stage, (float *)ctx->P, (int)c0, (int)cn, TSA, ctx->stream);
+                else
+                    cweno5_rows(stage, (double *)ctx->P, (int)c0, (int)cn, TSA, ctx->stream);
             } else {
                 const int blocks = (int)std::min<size_t>(4096, (cn * per_cell_dev + 255) / 256);
                 if (mixed)
@@ -4308,7 +4188,18 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
         if (host_pin) (void)hipHostFree(host_pin);
     }
     // indicators, packed upper triangle
-    if (ctx->iweno == 1) {
+    if (ctx->cw_cell) {
+        // by columns, entry by entry for the 8 cells of a tile
+        const size_t np = (size_t)ID * (ID + 1) / 2;
+        std::vector<double> bp((size_t)ctx->ntile * 8 * np, 0.0);
+        for (int i = 0; i < nc; ++i) {
+            const double *Bi = pre->indicator + src_cell(ctx, i) * ID * ID;
+            double *bt = bp.data() + (size_t)(i / 8) * np * 8 + i % 8;
+            for (int l = 0; l < ID; ++l)
+                for (int k = 0; k <= l; ++k) bt[((size_t)l * (l + 1) / 2 + k) * 8] = Bi[(size_t)k * ID + l];
+        }
+        if ((rc = upload_real_any(ctx, &ctx->B, bp))) return rc;
+    } else if (ctx->iweno == 1) {
         const size_t np = (size_t)ID * (ID + 1) / 2;
         std::vector<double> bp((size_t)nc * np);
         for (int i = 0; i < nc; ++i) {
@@ -4355,14 +4246,18 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
             }
             if ((rc = upload_real_any(ctx, &ctx->Bc, bc)) || (rc = upload_real_any(ctx, &ctx->dmb, dm))) return rc;
             if (ctx->cw_cell) {
-                // the sectors' low-order pseudo-inverses, stencils 2..ts
+                // the sectors' low-order pseudo-inverses, stencils 2..ts, as member rows
                 const int IM2 = ctx->imax2;
-                const size_t pc = (size_t)IM2 * ID2;
-                std::vector<double> P2((size_t)nc * std::max(ts - 1, 1) * pc, 0.0);
-                for (int i = 0; i < nc; ++i)
-                    for (int st = 1; st < ts; ++st)
-                        std::memcpy(P2.data() + ((size_t)i * (ts - 1) + st - 1) * pc,
-                                    ctx->h_cwP.data() + ((size_t)i * TSA + st) * pc, pc * sizeof(double));
+                const size_t pc = (size_t)IM2 * ID2, tp = (size_t)8 * NS;
+                std::vector<double> P2((size_t)ctx->ntile * pc * tp, 0.0);
+                for (int t = 0; t < ctx->ntile; ++t) {
+                    const int i0 = t * 8, nt = std::min(8, nc - i0);
+                    double *dst = P2.data() + (size_t)t * pc * tp;
+                    for (size_t e = 0; e < pc; ++e, dst += tp)
+                        for (int c = 0; c < nt; ++c)
+                            for (int st = 1; st < ts; ++st)
+                                dst[c * NS + st - 1] = ctx->h_cwP[((size_t)(i0 + c) * TSA + st) * pc + e];
+                }
                 if ((rc = upload_real_any(ctx, &ctx->Pc, P2))) return rc;
             }
         }

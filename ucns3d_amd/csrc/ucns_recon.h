@@ -24,6 +24,32 @@ void launch_scatter(const ReconWParams<float> &w, int ideg, int smode, hipStream
 void launch_recon_char(const ReconWParams<double> &p, int ideg, int smode, hipStream_t stream);
 void launch_recon_char(const ReconWParams<float> &p, int ideg, int smode, hipStream_t stream);
 
+// CWENO at WENO-5 (idegfree 34, sectors of 9 coefficients on 19 members),
+// recon_cweno5.hip.  Device layouts, for tiles of 8 cells (c: the cell in its
+// tile) and ns = ts - 1 sector stencils:
+//   nbr [tile][69][8]            central members
+//   nbc [tile][19][8 ns]         sector members, position c ns + sector
+//   P   [tile][69][34 * 8]       central rows (cweno5_rows)
+//   Pc  [tile][19][9][8 ns]      sector rows
+//   B   [tile][595][8]           packed triangle by columns: entry (k, l >= k) at l (l + 1) / 2 + k
+//   Bc  [ncell][45], dmb [ncell][9], and per cell as in ReconParams
+template <typename R>
+struct Cweno5Params {
+    int ncell, ntile, tiles_per_xcd, ts, nf, nqm, qpq, qpt, wenoz;
+    double gamma, lwci1, eps;
+    const double *U;
+    const int32_t *nbr, *nbc;
+    const R *P, *Pc, *B, *Bc, *dmb, *mbar, *qp;
+    const int32_t *cinfo, *cnb;
+    R *uleft;
+    int *marks;  // [ntile]
+};
+void launch_recon_cweno5(const Cweno5Params<double> &p, hipStream_t stream);
+void launch_recon_cweno5(const Cweno5Params<float> &p, hipStream_t stream);
+// central pseudo-inverses of cells cell0 (a multiple of 8) .. cell0+cn-1 from the ABI order into P
+void cweno5_rows(const double *src, double *dst, int cell0, int cn, int tsa, hipStream_t stream);
+void cweno5_rows(const double *src, float *dst, int cell0, int cn, int tsa, hipStream_t stream);
+
 }  // namespace ucns
 
 #endif  // UCNS_RECON_H
