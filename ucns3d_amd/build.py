@@ -34,7 +34,7 @@ HIP_FLAGS = [
     "-munsafe-fp-atomics",
 ]
 # translation units of libucnsgpu.so, compiled side by side
-HIP_SOURCES = ["ucns_gpu.hip", "recon_tiled.hip", "recon_char.hip", "recon_cweno5.hip", "recon_muscl.hip"]
+HIP_SOURCES = ["ucns_gpu.hip", "recon_tiled.hip", "recon_block.hip", "recon_cweno5.hip", "recon_muscl.hip"]
 
 
 def _run(cmd: list[str]) -> None:

@@ -409,12 +409,6 @@ struct ReconWParams {
     const R *Bc;
     const R *dmb;
     int wenoz;
-    // characteristic WENO (wenwrt 2): as in ReconParams
-    const int32_t *chnb;   // [ncell][nf]
-    const double *chang;   // [ncell][nf][4]
-    ucns_boundary_v1 bc;
-    const int32_t *cface;
-    const double *bface;
 };
 
 template <typename T>

@@ -2510,7 +2510,8 @@ struct ucns_ctx {
     double gamma = 1.4, lwci1 = 1.0, eps = 1e-11;
     bool have_prestore = false, have_state = false;
     bool tiled = false;  // WENO-4 lane-per-stencil kernel with the tiled layout
-    int smode = 0;      // stencils per cell of the row-stream kernel in use (0: none)
+    int smode = 0;      // stencils per cell where the pseudo-inverses are a row stream (0: tiled rows)
+    bool bmode = false;  // reconstruction by the block kernels (recon_block.hip)
     bool needs_bc = false, have_bc = false;  // boundary codes 1/2/6 present; ucns_set_boundary called
     double *bface = nullptr;  // [nface][10] per-face INFLOW(), OUTFLOW() states (ucns_set_boundary_faces)
     int nbface = 0;             // faces with a ghost state (codes 1/2/3/4/6)
@@ -2568,8 +2569,10 @@ struct ucns_ctx {
     double *adj_u0 = nullptr, *adj_bc = nullptr, *ckpt = nullptr, *dts = nullptr;
     void *adj_g = nullptr;  // stencil coefficients, indicators, weights of the row-stream reconstruction (R)
     double *adj_gb = nullptr;  // stencil-coefficient cotangents handed to the row stream, [ntile][ideg*5][8 ts]
-    uint16_t *adj_slot = nullptr;                      // [ntile][imax][8 ts] LDS row of each member entry
-    int32_t *adj_uq = nullptr, *adj_ucount = nullptr;  // [ntile][uq_cap], [ntile]
+    // the tiles' distinct stencil members (ensure_members): for the block
+    // reconstruction kernels and for the residual product's scatter
+    uint16_t *mem_slot = nullptr;                      // [ntile][imax][8 ts] table row of each member entry
+    int32_t *mem_uq = nullptr, *mem_count = nullptr;   // [ntile][uq_cap], [ntile]
     int uq_cap = UCNS_TILE_UQ;                         // member-table rows per tile (tile_uq(ts, imax))
     int64_t *adj_toff = nullptr, *adj_off = nullptr;  // table rows per tile, CSR offsets by cell
     int32_t *adj_ent = nullptr;                       // CSR entries: table rows (fewer than 2^31)
@@ -2625,6 +2628,25 @@ void dfree(T *&p) {
 
 int per_xcd(int ncell) { return (ncell + NXCD - 1) / NXCD; }
 
+template <typename R>
+LsqView<R> lsq_view(const ucns_ctx *ctx) {
+    LsqView<R> L{};
+    L.mode = ctx->smode ? 2 : ctx->tiled ? 1 : 0;
+    L.ts = ctx->ts;
+    L.tp = 8 * ctx->ts;
+    L.imax = ctx->imax;
+    L.ideg = ctx->ideg;
+    L.depth = stream_depth(sizeof(R) == 4, ctx->ts);
+    L.pb = ctx->ideg * L.tp * (int)sizeof(R);
+    L.rd = L.pb + L.tp * 4;
+    L.hd = L.depth * L.tp * 4;
+    L.tile_bytes = ctx->tile_bytes;
+    L.nbr = ctx->nbr;
+    L.P = (const R *)ctx->P;
+    L.rows = ctx->rows;
+    return L;
+}
+
 // kernel selection by (precision, ideg, imax)
 template <typename R>
 int launch_recon_t(ucns_ctx *ctx) {
@@ -2655,6 +2677,54 @@ int launch_recon_t(ucns_ctx *ctx) {
     p.bc = ctx->bc;
     p.cface = ctx->cface;
     p.bface = ctx->bface;
+    if (ctx->bmode) {
+        const LsqView<R> L = lsq_view<R>(ctx);
+        ReconBParams<R> w{};
+        w.ncell = ctx->ncell;
+        w.ntile = ctx->ntile;
+        w.tiles_per_xcd = (ctx->ntile + NXCD - 1) / NXCD;
+        w.nf = ctx->nf;
+        w.nqm = ctx->nqm;
+        w.qpq = ctx->qpq;
+        w.qpt = ctx->qpt;
+        w.gamma = ctx->gamma;
+        w.lwci1 = ctx->lwci1;
+        w.eps = ctx->eps;
+        w.U = ctx->U;
+        if (ctx->smode) {
+            w.rows = ctx->rows;
+            w.tile_bytes = ctx->tile_bytes;
+            w.hd = L.hd;
+            w.rd = L.rd;
+            w.depth = L.depth;
+        } else {
+            w.rows = (const unsigned char *)ctx->P;
+            w.rd = L.pb;
+            w.tile_bytes = (long long)ctx->imax * L.pb;
+            w.nbr = ctx->nbr;
+        }
+        w.imax = ctx->imax;
+        w.uq_cap = ctx->uq_cap;
+        w.uq = ctx->mem_uq;
+        w.ucount = ctx->mem_count;
+        w.slot = ctx->mem_slot;
+        w.B = (const R *)ctx->B;
+        w.mbar = (const R *)ctx->mbar;
+        w.qp = (const R *)ctx->qp;
+        w.cinfo = ctx->cinfo;
+        w.cnb = ctx->cnb;
+        w.uleft = (R *)ctx->uleft;
+        w.marks = ctx->marks;
+        w.gstore = ctx->adj_g_on ? (R *)ctx->adj_g : nullptr;
+        w.fstore = ctx->adj_g_on ? ctx->adj_flags : nullptr;
+        w.chnb = ctx->chnb;
+        w.chang = ctx->chang;
+        w.bc = ctx->bc;
+        w.cface = ctx->cface;
+        w.bface = ctx->bface;
+        launch_recon_block(w, ctx->ideg, ctx->ts, ctx->wenwrt == 2, ctx->stream);
+        return UCNS_OK;
+    }
     if (ctx->tiled) {
         ReconWParams<R> w{};
         w.ncell = ctx->ncell;
@@ -2687,15 +2757,6 @@ int launch_recon_t(ucns_ctx *ctx) {
             hipLaunchKernelGGL(k_pack64, dim3((unsigned)((n64 + 255) / 256)), dim3(256), 0, ctx->stream, n64, ctx->U,
                                ctx->u64);
             w.U64 = ctx->u64;
-        }
-        if (ctx->wenwrt == 2) {
-            w.chnb = ctx->chnb;
-            w.chang = ctx->chang;
-            w.bc = ctx->bc;
-            w.cface = ctx->cface;
-            w.bface = ctx->bface;
-            launch_recon_char(w, ctx->ideg, ctx->smode, ctx->stream);
-            return UCNS_OK;
         }
         w.gstore = ctx->adj_g_on ? (R *)ctx->adj_g : nullptr;
         w.fstore = ctx->adj_g_on ? ctx->adj_flags : nullptr;
@@ -2904,6 +2965,12 @@ int dt_kernel(ucns_ctx *ctx, double cfl, unsigned long long *out) {
 }
 
 // ---- adjoint -----------------------------------------------------------
+void release_members(ucns_ctx *ctx) {
+    dfree(ctx->mem_slot);
+    dfree(ctx->mem_uq);
+    dfree(ctx->mem_count);
+}
+
 void release_adjoint(ucns_ctx *ctx) {
     dfree(ctx->adj_ubf);
     dfree(ctx->adj_lam);
@@ -2918,13 +2985,11 @@ void release_adjoint(ucns_ctx *ctx) {
     ctx->adj_g = nullptr;
     dfree(ctx->adj_flags);
     dfree(ctx->adj_gb);
-    dfree(ctx->adj_slot);
-    dfree(ctx->adj_uq);
-    dfree(ctx->adj_ucount);
     dfree(ctx->adj_toff);
     dfree(ctx->adj_off);
     dfree(ctx->adj_ent);
     dfree(ctx->adj_tab);
+    if (!ctx->bmode) release_members(ctx);  // the block kernels' are the upload's
     ctx->ckpt_steps = 0;
     ctx->adj_ready = false;
     for (void *q : ctx->keep_ul) (void)hipFree(q);
@@ -2936,37 +3001,42 @@ void release_adjoint(ucns_ctx *ctx) {
 }
 
 template <typename R>
-LsqView<R> lsq_view(const ucns_ctx *ctx) {
-    LsqView<R> L{};
-    L.mode = ctx->smode ? 2 : ctx->tiled ? 1 : 0;
-    L.ts = ctx->ts;
-    L.tp = 8 * ctx->ts;
-    L.imax = ctx->imax;
-    L.ideg = ctx->ideg;
-    L.depth = stream_depth(sizeof(R) == 4, ctx->ts);
-    L.pb = ctx->ideg * L.tp * (int)sizeof(R);
-    L.rd = L.pb + L.tp * 4;
-    L.hd = L.depth * L.tp * 4;
-    L.tile_bytes = ctx->tile_bytes;
-    L.nbr = ctx->nbr;
-    L.P = (const R *)ctx->P;
-    L.rows = ctx->rows;
-    return L;
-}
-
-template <typename R>
 void launch_tile_members(ucns_ctx *ctx) {
     const LsqView<R> L = lsq_view<R>(ctx);
     const dim3 grid(ctx->ntile), block(WAVE);
     if (ctx->imax == 39)
         hipLaunchKernelGGL((k_tile_members<R, 39>), grid, block, 0, ctx->stream, L, ctx->ntile, ctx->ncell,
-                           ctx->cinfo, ctx->uq_cap, ctx->adj_uq, ctx->adj_ucount, ctx->adj_slot);
+                           ctx->cinfo, ctx->uq_cap, ctx->mem_uq, ctx->mem_count, ctx->mem_slot);
     else if (ctx->imax == 19)
         hipLaunchKernelGGL((k_tile_members<R, 19>), grid, block, 0, ctx->stream, L, ctx->ntile, ctx->ncell,
-                           ctx->cinfo, ctx->uq_cap, ctx->adj_uq, ctx->adj_ucount, ctx->adj_slot);
+                           ctx->cinfo, ctx->uq_cap, ctx->mem_uq, ctx->mem_count, ctx->mem_slot);
     else
         hipLaunchKernelGGL((k_tile_members<R, 8>), grid, block, 0, ctx->stream, L, ctx->ntile, ctx->ncell,
-                           ctx->cinfo, ctx->uq_cap, ctx->adj_uq, ctx->adj_ucount, ctx->adj_slot);
+                           ctx->cinfo, ctx->uq_cap, ctx->mem_uq, ctx->mem_count, ctx->mem_slot);
+}
+
+// the tiles' distinct stencil members, once per upload; all of it or nothing
+int ensure_members(ucns_ctx *ctx) {
+    if (ctx->mem_slot) return UCNS_OK;
+    ctx->uq_cap = tile_uq(ctx->ts, ctx->imax);
+    int rc = dalloc(ctx, &ctx->mem_slot, (size_t)ctx->ntile * ctx->imax * 8 * ctx->ts);
+    if (!rc) rc = dalloc(ctx, &ctx->mem_uq, (size_t)ctx->ntile * ctx->uq_cap);
+    if (!rc) rc = dalloc(ctx, &ctx->mem_count, (size_t)ctx->ntile);
+    if (rc) {
+        release_members(ctx);
+        return rc;
+    }
+    if (ctx->precision == UCNS_MIXED)
+        launch_tile_members<float>(ctx);
+    else
+        launch_tile_members<double>(ctx);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        release_members(ctx);
+        ctx->err = std::string("member tables: ") + hipGetErrorString(e);
+        return UCNS_EHIP;
+    }
+    return UCNS_OK;
 }
 
 // frees a temporary device buffer on every exit of the scope
@@ -3000,21 +3070,13 @@ int ensure_adjoint_steps(ucns_ctx *ctx) {
     }
     // the tiles' distinct stencil members (once per upload)
     if (ctx->ts <= 8 && (ctx->imax == 39 || ctx->imax == 19 || ctx->imax == 8)) {
-        if ((rc = dalloc(ctx, &ctx->adj_slot, (size_t)ctx->ntile * ctx->imax * 8 * ctx->ts))) return rc;
-        ctx->uq_cap = tile_uq(ctx->ts, ctx->imax);
-        if ((rc = dalloc(ctx, &ctx->adj_uq, (size_t)ctx->ntile * ctx->uq_cap))) return rc;
-        if ((rc = dalloc(ctx, &ctx->adj_ucount, (size_t)ctx->ntile))) return rc;
-        if (ctx->precision == UCNS_MIXED)
-            launch_tile_members<float>(ctx);
-        else
-            launch_tile_members<double>(ctx);
-        HIP_TRY(hipGetLastError());
+        if ((rc = ensure_members(ctx))) return rc;
         // table rows per tile (prefix sums on the host: set-up only).  The
         // library stream is non-blocking: every host read of what its kernels
         // wrote waits for the stream first, and every clear is queued on it.
         const int nt = ctx->ntile, nc = ctx->ncell;
         std::vector<int32_t> uc(nt);
-        HIP_TRY(hipMemcpyAsync(uc.data(), ctx->adj_ucount, nt * sizeof(int32_t), hipMemcpyDeviceToHost,
+        HIP_TRY(hipMemcpyAsync(uc.data(), ctx->mem_count, nt * sizeof(int32_t), hipMemcpyDeviceToHost,
                                ctx->stream));
         HIP_TRY(hipStreamSynchronize(ctx->stream));
         std::vector<int64_t> toff(nt + 1, 0);
@@ -3035,8 +3097,8 @@ int ensure_adjoint_steps(ucns_ctx *ctx) {
         if ((rc = dalloc(ctx, &cnt_buf.p, (size_t)nc))) return rc;
         int64_t *cnt = cnt_buf.p;
         HIP_TRY(hipMemsetAsync(cnt, 0, nc * sizeof(int64_t), ctx->stream));
-        hipLaunchKernelGGL(k_adj_csr, dim3(nt), dim3(256), 0, ctx->stream, nt, ctx->uq_cap, ctx->adj_uq,
-                           ctx->adj_ucount, ctx->adj_toff, cnt, (const int64_t *)nullptr, (int32_t *)nullptr);
+        hipLaunchKernelGGL(k_adj_csr, dim3(nt), dim3(256), 0, ctx->stream, nt, ctx->uq_cap, ctx->mem_uq,
+                           ctx->mem_count, ctx->adj_toff, cnt, (const int64_t *)nullptr, (int32_t *)nullptr);
         std::vector<int64_t> hc(nc), off(nc + 1, 0);
         HIP_TRY(hipMemcpyAsync(hc.data(), cnt, nc * sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
         HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -3049,8 +3111,8 @@ int ensure_adjoint_steps(ucns_ctx *ctx) {
         HIP_TRY(hipMemcpyAsync(ctx->adj_off, off.data(), (nc + 1) * sizeof(int64_t), hipMemcpyHostToDevice,
                                ctx->stream));
         HIP_TRY(hipMemsetAsync(cnt, 0, nc * sizeof(int64_t), ctx->stream));
-        hipLaunchKernelGGL(k_adj_csr, dim3(nt), dim3(256), 0, ctx->stream, nt, ctx->uq_cap, ctx->adj_uq,
-                           ctx->adj_ucount, ctx->adj_toff, cnt, (const int64_t *)ctx->adj_off, ctx->adj_ent);
+        hipLaunchKernelGGL(k_adj_csr, dim3(nt), dim3(256), 0, ctx->stream, nt, ctx->uq_cap, ctx->mem_uq,
+                           ctx->mem_count, ctx->adj_toff, cnt, (const int64_t *)ctx->adj_off, ctx->adj_ent);
         HIP_TRY(hipStreamSynchronize(ctx->stream));
     }
     return UCNS_OK;
@@ -3112,9 +3174,9 @@ void launch_scatter_t(ucns_ctx *ctx, double *ubar) {
     w.tile_bytes = ctx->tile_bytes;
     w.gbs = ctx->adj_gb;
     w.ubar = ubar;
-    w.slot = ctx->adj_slot;
+    w.slot = ctx->mem_slot;
     w.uq_cap = ctx->uq_cap;
-    w.ucount = ctx->adj_ucount;
+    w.ucount = ctx->mem_count;
     w.toff = ctx->adj_toff;
     w.tab = ctx->adj_tab;
     launch_scatter(w, ctx->ideg, ctx->smode, ctx->stream);
@@ -3203,10 +3265,10 @@ int vjp_products_t(ucns_ctx *ctx, const double *lam, double *ubar, double *bcbar
     vp.ubar = ubar;
     vp.gload = (ctx->smode && ctx->adj_g) ? (const R *)ctx->adj_g : nullptr;
     vp.fload = ctx->adj_flags;
-    vp.slot = ctx->adj_slot;
+    vp.slot = ctx->mem_slot;
     vp.uq_cap = ctx->uq_cap;
-    vp.uq = ctx->adj_uq;
-    vp.ucount = ctx->adj_ucount;
+    vp.uq = ctx->mem_uq;
+    vp.ucount = ctx->mem_count;
     vp.gbout = ctx->smode ? ctx->adj_gb : nullptr;
     vp.toff = ctx->adj_toff;
     vp.tab = ctx->adj_tab;
@@ -3278,7 +3340,7 @@ int vjp_products_t(ucns_ctx *ctx, const double *lam, double *ubar, double *bcbar
         return UCNS_EUNSUPPORTED;
     }
     if (ctx->smode) launch_scatter_t<R>(ctx, ubar);
-    if (ctx->adj_slot) adj_gather(ctx, ubar);
+    if (ctx->mem_slot) adj_gather(ctx, ubar);
     tstop(ctx, 0);
     tcollect(ctx, 0, &ctx->st.ms_recon_vjp, &ctx->st.n_recon_vjp);
     return UCNS_OK;
@@ -3462,6 +3524,7 @@ void release_prestore(ucns_ctx *ctx) {
     dfree(ctx->rows);
     dfree(ctx->u64);
     dfree(ctx->marks);
+    release_members(ctx);
     dfree(ctx->B);
     dfree(ctx->mbar);
     if (ctx->Bc) (void)hipFree(ctx->Bc);
@@ -4006,7 +4069,9 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
     }
     ctx->ts = ts;
     const bool mixed = ctx->precision == UCNS_MIXED;
-    ctx->tiled = (ctx->iweno == 1 && ((ID == 19 && IM == 39) || (ID == 9 && IM == 19)) &&
+    // the block kernels (recon_block.hip)
+    const bool wide = ctx->kernels == UCNS_KERNELS_AUTO && ctx->ees != 5 && ts >= 5 && ts <= 7;
+    ctx->tiled = (ctx->iweno == 1 && (ctx->wenwrt == 1 || wide) && ((ID == 19 && IM == 39) || (ID == 9 && IM == 19)) &&
                   ts <= 8 && ctx->nf * ctx->nqm <= 56);
     ctx->cw_cell = ctx->ees == 5 && !ctx->tiled;
     if (ctx->cw_cell && ID != 34) {
@@ -4025,6 +4090,10 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
         ctx->smode = stream_ok ? ts : 0;
     }
     ctx->ntile = (nc + 7) / 8;
+    // WENO-4 of at most 1,024 tiles, one per SIMD of the chip: there a wave per
+    // tile leaves SIMDs idle and its chain of rows bare (216 tiles 47 us against
+    // 31; at 3,072 tiles both take 217 us)
+    ctx->bmode = ctx->tiled && wide && (ctx->wenwrt == 2 || (ctx->smode && ID == 19 && ctx->ntile <= 1024));
     ctx->nmark = ctx->tiled || ctx->cw_cell || ctx->iweno == -1 ? ctx->ntile : nc;
     int rc = dalloc(ctx, &ctx->marks, (size_t)ctx->nmark);
     if (rc) return rc;
@@ -4274,6 +4343,7 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
                             pre->qpoints[((src_cell(ctx, i) * nfa + f) * nqa + g) * 3 + d];
         if ((rc = upload_real_any(ctx, &ctx->qp, q))) return rc;
     }
+    if (ctx->bmode && (rc = ensure_members(ctx))) return rc;
     ctx->have_prestore = true;
     ctx->st.bytes_recon_per_cell =
         (double)((size_t)IM * ts * ID * (mixed ? 4 : 8)) + (ctx->iweno == 1 ? (double)ID * (ID + 1) / 2 * (mixed ? 4 : 8) : 0) +

@@ -19,11 +19,6 @@ void launch_recon_tiled(const ReconWParams<float> &w, int ideg, int smode, bool 
 // P^T of the stencil-coefficient cotangents on the row stream
 void launch_scatter(const ReconWParams<double> &w, int ideg, int smode, hipStream_t stream);
 void launch_scatter(const ReconWParams<float> &w, int ideg, int smode, hipStream_t stream);
-// characteristic WENO-3 / WENO-4 on the tiled layouts, recon_char.hip; smode:
-// the stencils per cell of the row-stream layout, or 0
-void launch_recon_char(const ReconWParams<double> &p, int ideg, int smode, hipStream_t stream);
-void launch_recon_char(const ReconWParams<float> &p, int ideg, int smode, hipStream_t stream);
-
 // CWENO at WENO-5 (idegfree 34, sectors of 9 coefficients on 19 members),
 // recon_cweno5.hip.  Device layouts, for tiles of 8 cells (c: the cell in its
 // tile) and ns = ts - 1 sector stencils:
@@ -49,6 +44,48 @@ void launch_recon_cweno5(const Cweno5Params<float> &p, hipStream_t stream);
 // central pseudo-inverses of cells cell0 (a multiple of 8) .. cell0+cn-1 from the ABI order into P
 void cweno5_rows(const double *src, double *dst, int cell0, int cn, int tsa, hipStream_t stream);
 void cweno5_rows(const double *src, float *dst, int cell0, int cn, int tsa, hipStream_t stream);
+
+// recon_block.hip: characteristic WENO-3 / WENO-4 with 5, 6 or 7 stencils per
+// cell (ch), or WENO-4 in conserved variables with 5 or 7
+template <typename R>
+struct ReconBParams {
+    int ncell, ntile, tiles_per_xcd, nf, nqm, qpq, qpt;
+    double gamma, lwci1, eps;
+    const double *U;
+    // pseudo-inverses: tile t's row j is at rows + t tile_bytes + hd + j rd,
+    // [ideg][8 ts] R
+    const unsigned char *rows;
+    long long tile_bytes;
+    int hd, rd;
+    // distinct members of each tile [ntile][uq_cap] and, per (row, column),
+    // the index into them ([ntile][imax][8 ts], UCNS_NOSLOT past uq_cap);
+    // the members themselves behind the rows (row stream) or in nbr
+    int uq_cap, depth, imax;
+    const int32_t *uq, *ucount;
+    const uint16_t *slot;
+    const int32_t *nbr;
+    const R *B, *mbar, *qp;
+    const int32_t *cinfo, *cnb;
+    R *uleft;
+    int *marks;   // [ntile]
+    R *gstore;    // as in ReconWParams
+    int *fstore;
+    const int32_t *chnb;  // characteristic WENO, as in ReconParams
+    const double *chang;
+    ucns_boundary_v1 bc;
+    const int32_t *cface;
+    const double *bface;
+
+    // member of row j, column col
+    __device__ int member(int tile, int j, int col, int tp) const {
+        if (nbr) return nbr[((size_t)tile * imax + j) * tp + col];
+        const unsigned char *t = rows + (size_t)tile * tile_bytes;
+        const unsigned char *r = j < depth ? t + (size_t)j * tp * 4 : t + hd + (size_t)(j - depth + 1) * rd - tp * 4;
+        return ((const int32_t *)r)[col];
+    }
+};
+void launch_recon_block(const ReconBParams<double> &p, int ideg, int ts, bool ch, hipStream_t stream);
+void launch_recon_block(const ReconBParams<float> &p, int ideg, int ts, bool ch, hipStream_t stream);
 
 }  // namespace ucns
 

@@ -10,179 +10,13 @@
 
 namespace ucns {
 
-// Characteristic WENO of one tile, face by face (compute_gradcharv_smoothindicator,
-// diag_At_B_A, src/reconstruct_p.f90:497-758, 1608-1818): the eigenvectors of
-// the averaged cell / neighbour state in the face frame (WENO_NEIGHBOUR: the
-// ghost of the cell's own average on boundary faces), every stencil's
-// coefficients projected with L, indicators and weights per characteristic
-// variable, and the face's values R sum_s omega_s L p_s(x_q), with p_s(x_q)
-// the stencil's own polynomial at the point.
-//
-// Bound by FP64 vector work: lane (cell, stencil) keeps its coefficients in
-// registers and projects one characteristic column at a time, and the sum over
-// stencils is taken of a point's five values instead of the 95 weighted
-// coefficients.
-// Eigenvectors, weights and projections are in FP64 in both precisions.
-// Returns whether any of the cell's face values fails CHECKSOL.
-// 24,576 tetrahedra, WENO-4: 1289 us with one wave per cell (its lane 0 forming
-// the eigenvectors, 25 lanes the indicators), 510 us this way.
-template <typename R, int IDEG>
-__device__ __forceinline__ int char_faces(const ReconWParams<R> &p, const R (&g)[IDEG][NV],
-                                          const R (*sB)[IDEG * (IDEG + 1) / 2], int lc, int s, int cell, bool cvalid, int info, bool act, const R *qpc, const R *mb) {
-    const int ifca = ci_ifca(info), full = ci_full(info);
-    const size_t cc = cvalid ? cell : 0;
-    const double lam = s == 0 ? p.lwci1 : 1.0;
-    R *out = p.uleft + cc * p.nf * p.nqm * NV;
-    int trouble = 0;
-#pragma unroll 1
-    for (int f = 0; f < p.nf; ++f) {
-        const bool fv = cvalid && f < ifca;
-        const size_t cf = cc * p.nf + (fv ? f : 0);
-        double ui[NV];  // read again for each face: kept, it would be spilled through the least squares
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int v = 0; v < NV; ++v) ui[v] = p.U[cc * NV + v];
-        // eigenvectors (char_eigen_d's, without its zeros and ones)
-        double us, vs, ws, as, hs, q2, b, bq, oa;
-        {
-            const int nbf = p.chnb[cf];
-            const double *an = p.chang + cf * 4;
-            double ur[NV], rl[NV], rr[NV];
-            if (fv && nbf < 0) {
-                const double *bf = p.bface ? p.bface + (size_t)(p.cface[cf] - 1) * 10 : nullptr;
-                ghost_state(-nbf, p.bc.boundtype, p.gamma, ui, an[0], an[1], an[2], an[3], bf ? bf : p.bc.inflow,
-                            bf ? bf + 5 : p.bc.outflow, ur);
-            } else {
-#pragma unroll
-                for (int v = 0; v < NV; ++v) ur[v] = fv ? p.U[(size_t)nbf * NV + v] : ui[v];
-            }
-            rotf(ui, an[0], an[1], an[2], an[3], rl);
-            rotf(ur, an[0], an[1], an[2], an[3], rr);
-            const double rs = 0.5 * (rl[0] + rr[0]);
-            us = 0.5 * (rl[1] / rl[0] + rr[1] / rr[0]);
-            vs = 0.5 * (rl[2] / rl[0] + rr[2] / rr[0]);
-            ws = 0.5 * (rl[3] / rl[0] + rr[3] / rr[0]);
-            const double es = 0.5 * (rl[4] + rr[4]);
-            q2 = us * us + vs * vs + ws * ws;
-            const double ps = (p.gamma - 1.0) * (es - 0.5 * rs * q2);
-            as = sqrt(p.gamma * ps / rs);
-            hs = 0.5 * q2 + as * as / (p.gamma - 1.0);
-            b = (p.gamma - 1.0) / (as * as);
-            bq = 0.5 * b * q2;
-            oa = 1.0 / as;
-        }
-        const double l00 = 0.5 * (bq + us * oa), l01 = -0.5 * (b * us + oa), l02 = -0.5 * b * vs,
-                     l03 = -0.5 * b * ws, l04 = 0.5 * b;
-        const double l10 = 1.0 - bq, l11 = b * us, l12 = b * vs, l13 = b * ws;
-        const double l40 = 0.5 * (bq - us * oa), l41 = -0.5 * (b * us - oa);
-        auto project = [&](const double (&x)[NV], double (&c)[NV]) {
-            c[0] = x[0] * l00 + x[1] * l01 + x[2] * l02 + x[3] * l03 + x[4] * l04;
-            c[1] = x[0] * l10 + x[1] * l11 + x[2] * l12 + x[3] * l13 - x[4] * b;
-            c[2] = x[2] - x[0] * vs;
-            c[3] = x[3] - x[0] * ws;
-            c[4] = x[0] * l40 + x[1] * l41 + x[2] * l02 + x[3] * l03 + x[4] * l04;
-        };
-        // indicators and weights, one characteristic variable after the other
-        // (a column of w at a time beside the stencil's coefficients is what
-        // the registers hold; all five would spill)
-        double om[NV] = {0, 0, 0, 0, 0};
-#pragma unroll 1
-        for (int c = 0; c < NV; ++c) {
-            const double l0 = c == 0 ? l00 : c == 1 ? l10 : c == 2 ? -vs : c == 3 ? -ws : l40;
-            const double l1 = c == 0 ? l01 : c == 1 ? l11 : c == 4 ? l41 : 0.0;
-            const double l2 = c == 1 ? l12 : c == 2 ? 1.0 : c == 3 ? 0.0 : l02;
-            const double l3 = c == 1 ? l13 : c == 2 ? 0.0 : c == 3 ? 1.0 : l03;
-            const double l4 = c == 1 ? -b : c == 2 || c == 3 ? 0.0 : l04;
-            // B's address passes through an opaque value: hoisted out of the
-            // loops, its entries would take every register
-            int lb = lc;
-            asm volatile("" : "+v"(lb));
-            const R *B = sB[lb];
-            double beta = 0.0;
-            if (act) {  // all of it: arithmetic alone would sink to the weights below, without its loads
-                double w[IDEG];
-#pragma unroll
-                for (int k = 0; k < IDEG; ++k)
-                    w[k] = (double)g[k][0] * l0 + (double)g[k][1] * l1 + (double)g[k][2] * l2 + (double)g[k][3] * l3 +
-                           (double)g[k][4] * l4;
-#pragma unroll
-                for (int k = 0; k < IDEG; ++k) {
-                    double bg = 0.0;
-#pragma unroll
-                    for (int l = k + 1; l < IDEG; ++l) bg += (double)B[pidx(IDEG, k, l)] * w[l];
-                    beta += w[k] * ((double)B[pidx(IDEG, k, k)] * w[k] + 2.0 * bg);
-                }
-            }
-            // lambda/(eps+beta)^4
-            const double x = p.eps + beta;
-            const double x2 = x * x;
-            const double wt = act ? lam / (x2 * x2) : 0.0;
-            const double sum = grp_sum8(wt);
-            const double o = act ? wt / sum : 0.0;
-#pragma unroll
-            for (int e = 0; e < NV; ++e) om[e] = c == e ? o : om[e];
-        }
-        // the face's points: every lane forms its stencil's value, the group
-        // sums, lane q mod 8 keeps the point
-        const int nq = fv ? (ci_tri(info, f) ? p.qpt : p.qpq) : 0;
-#pragma unroll 1
-        for (int q0 = 0; q0 < p.nqm; q0 += 8) {
-            double mine[NV] = {0, 0, 0, 0, 0};
-#pragma unroll 1
-            for (int q = q0; q < min(q0 + 8, p.nqm); ++q) {
-                const R *xq = qpc + ((fv ? f : 0) * p.nqm + q) * 3;
-                const R x[3] = {xq[0], xq[1], xq[2]};
-                R phi[IDEG];
-                int zero = 0;
-                asm volatile("" : "+v"(zero));  // as B's address: the means stay in memory
-                basis_at<R, IDEG>(x, mb + zero, phi);
-                double pv[NV], pc[NV];
-#pragma unroll
-                for (int v = 0; v < NV; ++v) {
-                    double t = 0.0;
-#pragma unroll
-                    for (int k = 0; k < IDEG; ++k) t += (double)phi[k] * (double)g[k][v];
-                    pv[v] = t;
-                }
-                project(pv, pc);
-#pragma unroll
-                for (int c = 0; c < NV; ++c) pc[c] = grp_sum8(om[c] * pc[c]);
-                const double rv[NV] = {
-                    pc[0] + pc[1] + pc[4],
-                    (us - as) * pc[0] + us * pc[1] + (us + as) * pc[4],
-                    vs * pc[0] + vs * pc[1] + pc[2] + vs * pc[4],
-                    ws * pc[0] + ws * pc[1] + pc[3] + ws * pc[4],
-                    (hs - us * as) * pc[0] + 0.5 * q2 * pc[1] + vs * pc[2] + ws * pc[3] + (hs + us * as) * pc[4]};
-#pragma unroll
-                for (int v = 0; v < NV; ++v) mine[v] = (q & 7) == s ? rv[v] : mine[v];
-            }
-            const int q = q0 + s;
-            if (fv && q < p.nqm) {
-                const bool ok = q < nq;
-                double uq[NV];
-#pragma unroll
-                for (int v = 0; v < NV; ++v) {
-                    const R r = ok ? (R)mine[v] : R(0);
-                    out[(f * p.nqm + q) * NV + v] = r;
-                    uq[v] = ui[v] + (double)r;
-                }
-                double wi[NV];
-                cons2prim_d(p.gamma, ui, wi);
-                if (ok && full && jump_test(p.gamma, wi, uq, 0.85)) trouble = 1;
-            }
-        }
-    }
-    return trouble;
-}
-
 // STORE: also write every stencil's coefficients to p.gstore (the adjoint's forward pass).
 // qpc / mb: the cell's face points and basis means, in HBM or staged in LDS
 // by loads still in flight (QWAIT: wait for them before the face points).
 // STG: the face values pass through stg (LDS, 8 x 8 x NV values, free once
 // the indicators are formed) and leave as coalesced words.
-template <typename R, int IDEG, int NQL, bool STORE = false, bool CW = false, bool QWAIT = false, bool STG = false,
-          bool CH = false>
-__device__ __forceinline__ void recon_late(const ReconWParams<R> &p, R (&g)[IDEG][NV], const double (&ui_)[NV],
+template <typename R, int IDEG, int NQL, bool STORE = false, bool CW = false, bool QWAIT = false, bool STG = false>
+__device__ __forceinline__ void recon_late(const ReconWParams<R> &p, R (&g)[IDEG][NV], const double (&ui)[NV],
                                            const R (*sB)[IDEG * (IDEG + 1) / 2], R (*sG0)[IDEG * NV], int lc, int s,
                                            int cell, bool cvalid, int info, bool act, const R *qpc, const R *mb,
                                            R *stg = nullptr) {
@@ -205,22 +39,6 @@ __device__ __forceinline__ void recon_late(const ReconWParams<R> &p, R (&g)[IDEG
     }
     __syncthreads();
 
-    const int nslot = ifca * p.nqm;
-    R *out = p.uleft + (size_t)(cvalid ? cell : 0) * p.nf * p.nqm * NV;
-    double wi[NV], ui[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) ui[v] = ui_[v];
-    int trouble = 0;
-    if constexpr (CH) {
-        if constexpr (QWAIT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        trouble = char_faces<R, IDEG>(p, g, sB, lc, s, cell, cvalid, info, act, qpc, mb);
-        if (cvalid) {
-#pragma unroll
-            for (int v = 0; v < NV; ++v) ui[v] = p.U[(size_t)cell * NV + v];
-        }
-    }
-    cons2prim_d(p.gamma, ui, wi);
-    if constexpr (!CH) {
     R om[NV];
     R corr[NV] = {R(0), R(0), R(0), R(0), R(0)};  // CWENO: the sectors' low-order means
     if constexpr (CW) {
@@ -359,7 +177,12 @@ __device__ __forceinline__ void recon_late(const ReconWParams<R> &p, R (&g)[IDEG
     // Values are stored as they are formed.  A cell that passes CHECKSOL
     // cannot fail CHECKSOLX (its 0.95 jumps imply the 0.85 ones), so only
     // the MUSCL branch below re-tests and overwrites its face points.
+    const int nslot = ifca * p.nqm;
     if constexpr (QWAIT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    R *out = p.uleft + (size_t)(cvalid ? cell : 0) * p.nf * p.nqm * NV;
+    double wi[NV];
+    cons2prim_d(p.gamma, ui, wi);
+    int trouble = 0;
 #pragma unroll 1
     for (int q = s; q < NQL * 8; q += 8) {
         const int f = q / p.nqm, qq = q - f * p.nqm;
@@ -410,7 +233,6 @@ __device__ __forceinline__ void recon_late(const ReconWParams<R> &p, R (&g)[IDEG
             asm volatile("" ::: "memory");
         }
     }
-    }  // !CH
     const int any_trouble = grp_or8(trouble);  // every lane takes part in the shuffle
     const bool reduce = cvalid && (!full || any_trouble);
     bool first = false;
@@ -502,7 +324,7 @@ __device__ __forceinline__ void recon_late(const ReconWParams<R> &p, R (&g)[IDEG
     if (STORE && s == 0 && cvalid) p.fstore[cell] = (reduce ? 1 : 0) | (first ? 2 : 0);
 }
 
-template <typename R, int IDEG, int IMAX, int NQL, int D, bool CW = false, bool CH = false>
+template <typename R, int IDEG, int IMAX, int NQL, int D, bool CW = false>
 __device__ __forceinline__ void recon_w_body(const ReconWParams<R> &p) {
     constexpr int NP = IDEG * (IDEG + 1) / 2;
     __shared__ R sB[8][NP];
@@ -584,7 +406,7 @@ __device__ __forceinline__ void recon_w_body(const ReconWParams<R> &p) {
         }
     }
     const size_t cq = cvalid ? cell : 0;
-    recon_late<R, IDEG, NQL, false, CW, false, false, CH>(p, g, ui, sB, sG0, lc, s, cell, cvalid, info, act,
+    recon_late<R, IDEG, NQL, false, CW>(p, g, ui, sB, sG0, lc, s, cell, cvalid, info, act,
                                         p.qp + cq * p.nf * p.nqm * 3, p.mbar + cq * IDEG);
 }
 
@@ -655,7 +477,7 @@ constexpr int free_lds(int ring, int need, int a0, int a1, int b0, int b1, int c
     return -1;
 }
 
-template <typename R, int IDEG, int IMAX, int NQL, int TS, int DEPTH, bool STORE = false, bool CH = false>
+template <typename R, int IDEG, int IMAX, int NQL, int TS, int DEPTH, bool STORE = false>
 __device__ __forceinline__ void recon_s_body(const ReconWParams<R> &p) {
     using SS = StreamShape<R, IDEG, IMAX, TS, DEPTH>;
     constexpr int NP = SS::NP, TP = SS::TP;
@@ -679,10 +501,6 @@ __device__ __forceinline__ void recon_s_body(const ReconWParams<R> &p) {
                  : "+v"(info), "+v"(ui[0]), "+v"(ui[1]), "+v"(ui[2]), "+v"(ui[3]), "+v"(ui[4])
                  :
                  : "memory");
-    // CH: the face loop takes every register, and a cell state kept in them
-    // would be spilled through this loop
-    __shared__ double sUi[CH ? 8 : 1][NV];
-    if (CH && s < NV) sUi[CH ? lc : 0][s] = s == 0 ? ui[0] : s == 1 ? ui[1] : s == 2 ? ui[2] : s == 3 ? ui[3] : ui[4];
     const int admis = ci_admis(info);
     const bool act = cvalid && s < admis;
     const int rl = act ? lc * TS + s : 0;
@@ -753,11 +571,8 @@ __device__ __forceinline__ void recon_s_body(const ReconWParams<R> &p) {
             const double2 a = *(const double2 *)st;
             const double2 c = *(const double2 *)(st + 2);
             const double u4 = st[4];
-            double uc[NV];
-#pragma unroll
-            for (int v = 0; v < NV; ++v) uc[v] = CH ? sUi[CH ? lc : 0][v] : ui[v];
-            const R du[NV] = {(R)(a.x - uc[0]), (R)(a.y - uc[1]), (R)(c.x - uc[2]), (R)(c.y - uc[3]),
-                              (R)(u4 - uc[4])};
+            const R du[NV] = {(R)(a.x - ui[0]), (R)(a.y - ui[1]), (R)(c.x - ui[2]), (R)(c.y - ui[3]),
+                              (R)(u4 - ui[4])};
             const R *row = (const R *)slot + rl;
             R pc[IDEG];
 #pragma unroll
@@ -841,9 +656,9 @@ __device__ __forceinline__ void recon_s_body(const ReconWParams<R> &p) {
     // 20.8 -> 20.1 ms, 64^3 x 6 tetrahedra 10.86 -> 10.71); in FP32 the
     // direct stores measured as fast or faster (hexahedra 10.8 ms direct,
     // 11.6 staged)
-    constexpr bool STG = sizeof(R) == 8 && !CH;
+    constexpr bool STG = sizeof(R) == 8;
     static_assert(!STG || 8 * 8 * NV * (int)sizeof(R) <= SS::B1 - SS::B0, "face-value staging exceeds the B block");
-    recon_late<R, IDEG, NQL, STORE, false, (QO >= 0), STG, CH>(p, g, ui, sB, sG0, lc, s, cell, cvalid, info, act, qpc, mb,
+    recon_late<R, IDEG, NQL, STORE, false, (QO >= 0), STG>(p, g, ui, sB, sG0, lc, s, cell, cvalid, info, act, qpc, mb,
                                                            (R *)(ring + SS::B0));
 }
 
