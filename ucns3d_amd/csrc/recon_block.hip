@@ -310,7 +310,8 @@ __global__ __launch_bounds__(NW *WAVE, OCC) void k_recon_block(ReconBParams<R> p
                 sj = *(const uint16_t *)(St + (size_t)(j * TP * 2) + os);
                 const char *row = Pt + (size_t)j * p.rd;
 #pragma unroll
-                for (int k = 0; k < KW; ++k) pr[k] = *(const R *)(row + ol + k * TP * (int)sizeof(R));
+                for (int k = 0; k < KW; ++k)
+                    pr[k] = __builtin_nontemporal_load((const R *)(row + ol + k * TP * (int)sizeof(R)));
             };
             auto add = [&](const R (&pr)[KW], const double *u) {
                 R du[NV];

@@ -374,7 +374,7 @@ __device__ __forceinline__ void recon_w_body(const ReconWParams<R> &p) {
                 for (int v = 0; v < NV; ++v) ub[d][v] = p.U[(size_t)n * NV + v];
                 const R *Pj = Pt + (size_t)d * IDEG * TP;
 #pragma unroll
-                for (int k = 0; k < IDEG; ++k) pb[d][k] = Pj[k * TP];
+                for (int k = 0; k < IDEG; ++k) pb[d][k] = __builtin_nontemporal_load(Pj + k * TP);
             }
 #pragma unroll 1
             for (int j0 = 0; j0 < IMAX; j0 += D) {
@@ -394,7 +394,7 @@ __device__ __forceinline__ void recon_w_body(const ReconWParams<R> &p) {
                             for (int v = 0; v < NV; ++v) ub[d][v] = p.U[(size_t)n * NV + v];
                             const R *Pj = Pt + (size_t)jn * IDEG * TP;
 #pragma unroll
-                            for (int k = 0; k < IDEG; ++k) pb[d][k] = Pj[k * TP];
+                            for (int k = 0; k < IDEG; ++k) pb[d][k] = __builtin_nontemporal_load(Pj + k * TP);
                         }
 #pragma unroll
                         for (int k = 0; k < IDEG; ++k)
