@@ -176,17 +176,19 @@ static void launch(const ReconWParams<R> &w, int ideg, int smode, bool cweno, hi
     const bool few = w.nf * w.nqm <= 24;
 #define UCNS_LAUNCH(...) hipLaunchKernelGGL((__VA_ARGS__), grid, block, 0, stream, w)
     if (smode) {
-        // (ideg, imax, face-point slots, stencils): WENO-4 tets / hexes, WENO-3 tets / hexes
+        // (ideg, imax, face-point slots, stencils): WENO-4 tets / hexes, WENO-3 tets / prisms and pyramids / hexes
         if constexpr (sizeof(R) == 8) {
             if (w.gstore) {
                 if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_sg64<19, 39, 3, 5>);
                 else if (ideg == 19) UCNS_LAUNCH(k_recon_sg64<19, 39, 7, 7>);
                 else if (smode == 5) UCNS_LAUNCH(k_recon_sg64<9, 19, 3, 5>);
+                else if (smode == 6) UCNS_LAUNCH(k_recon_sg64<9, 19, 3, 6>);
                 else UCNS_LAUNCH(k_recon_sg64<9, 19, 3, 7>);
             } else {
                 if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_s64<19, 39, 3, 5>);
                 else if (ideg == 19) UCNS_LAUNCH(k_recon_s64<19, 39, 7, 7>);
                 else if (smode == 5) UCNS_LAUNCH(k_recon_s64<9, 19, 3, 5>);
+                else if (smode == 6) UCNS_LAUNCH(k_recon_s64<9, 19, 3, 6>);
                 else UCNS_LAUNCH(k_recon_s64<9, 19, 3, 7>);
             }
         } else {
@@ -194,11 +196,13 @@ static void launch(const ReconWParams<R> &w, int ideg, int smode, bool cweno, hi
                 if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_sg32<19, 39, 3, 5>);
                 else if (ideg == 19) UCNS_LAUNCH(k_recon_sg32<19, 39, 7, 7>);
                 else if (smode == 5) UCNS_LAUNCH(k_recon_sg32<9, 19, 3, 5>);
+                else if (smode == 6) UCNS_LAUNCH(k_recon_sg32<9, 19, 3, 6>);
                 else UCNS_LAUNCH(k_recon_sg32<9, 19, 3, 7>);
             } else {
                 if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_s32<19, 39, 3, 5>);
                 else if (ideg == 19) UCNS_LAUNCH(k_recon_s32<19, 39, 7, 7>);
                 else if (smode == 5) UCNS_LAUNCH(k_recon_s32<9, 19, 3, 5>);
+                else if (smode == 6) UCNS_LAUNCH(k_recon_s32<9, 19, 3, 6>);
                 else UCNS_LAUNCH(k_recon_s32<9, 19, 3, 7>);
             }
         }
@@ -238,6 +242,7 @@ void launch_scatter(const ReconWParams<double> &w, int ideg, int smode, hipStrea
     if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_scatter_s64<19, 39, 5>);
     else if (ideg == 19) UCNS_LAUNCH(k_scatter_s64<19, 39, 7>);
     else if (smode == 5) UCNS_LAUNCH(k_scatter_s64<9, 19, 5>);
+    else if (smode == 6) UCNS_LAUNCH(k_scatter_s64<9, 19, 6>);
     else UCNS_LAUNCH(k_scatter_s64<9, 19, 7>);
 }
 void launch_scatter(const ReconWParams<float> &w, int ideg, int smode, hipStream_t stream) {
@@ -245,6 +250,7 @@ void launch_scatter(const ReconWParams<float> &w, int ideg, int smode, hipStream
     if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_scatter_s32<19, 39, 5>);
     else if (ideg == 19) UCNS_LAUNCH(k_scatter_s32<19, 39, 7>);
     else if (smode == 5) UCNS_LAUNCH(k_scatter_s32<9, 19, 5>);
+    else if (smode == 6) UCNS_LAUNCH(k_scatter_s32<9, 19, 6>);
     else UCNS_LAUNCH(k_scatter_s32<9, 19, 7>);
 }
 #undef UCNS_LAUNCH
