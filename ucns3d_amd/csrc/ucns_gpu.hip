@@ -3341,7 +3341,7 @@ int vjp_products_t(ucns_ctx *ctx, const double *lam, double *ubar, double *bcbar
         ctx->err = "no residual product for idegfree=" + std::to_string(ctx->ideg);
         return UCNS_EUNSUPPORTED;
     }
-    if (ctx->smode) launch_scatter_t<R>(ctx, ubar);
+    if (ctx->smode && !geo_done) launch_scatter_t<R>(ctx, ubar);  // k_recon_vjp scatters by itself
     if (ctx->mem_slot) adj_gather(ctx, ubar);
     tstop(ctx, 0);
     tcollect(ctx, 0, &ctx->st.ms_recon_vjp, &ctx->st.n_recon_vjp);
@@ -4862,7 +4862,9 @@ int ucns_rk3_adjoint_geometry(ucns_ctx *ctx, int32_t nsteps, double dt_fixed, co
     }
     int rc = ready(ctx);
     if (rc) return rc;
-    if (ctx->precision != UCNS_FP64 || ctx->smode) {
+    // k_recon_vjp reads any layout of the pseudo-inverses (LsqView); it takes
+    // the row stream of 6 stencils, not those of 5 and 7
+    if (ctx->precision != UCNS_FP64 || (ctx->smode && ctx->smode != 6)) {
         ctx->err = "ucns_rk3_adjoint_geometry: needs an FP64 context on the register kernels "
                    "(precision UCNS_FP64; kernels UCNS_KERNELS_REGISTER where the row-stream kernels would run)";
         return UCNS_EUNSUPPORTED;
