@@ -950,6 +950,8 @@ struct UpdateParams {
     const double *minedge;
     double *U, *U2;
     double *rhs_out;         // optional [ncell][5]
+    double *u64;             // optional: the new state as 64-byte records (k_pack64's), for the next reconstruction
+    double *copy;            // optional: a copy of the new state, [ncell][5]
     const double *dt;        // this step's dt: one value, or (dt_slots) the slots it is the least of
     int dt_slots;
     unsigned long long *dt_next;  // the next step's slots: cleared to +inf in stage 2, atomic-min targets in stage 3
@@ -1044,6 +1046,17 @@ __global__ __launch_bounds__(256) void k_update(UpdateParams p) {
             }
 #pragma unroll
             for (int v = 0; v < NV; ++v) u[v] = un[v];
+            if (p.u64) {
+                double2 *r64 = (double2 *)(p.u64 + (size_t)i * 8);
+                r64[0] = make_double2(un[0], un[1]);
+                r64[1] = make_double2(un[2], un[3]);
+                r64[2] = make_double2(un[4], 0.0);
+                r64[3] = make_double2(0.0, 0.0);
+            }
+            if (p.copy) {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) p.copy[(size_t)i * NV + v] = un[v];
+            }
             if (p.stage == 3 && p.dt_next) {
                 double w[NV];
                 cons2prim_d(p.gamma, un, w);
@@ -2337,7 +2350,9 @@ __global__ __launch_bounds__(256) void k_flux_geom(FluxParams<double> p, const d
     if (!BND) atomic_add_f64(&govol[cR], -area * eR / ovol[cR]);
 }
 
-// the state [ncell][5] as 64-byte records [ncell][8] (the last three zero)
+// the state [ncell][5] as 64-byte records [ncell][8] (the last three zero):
+// the first reconstruction of a march; the later ones find the records that
+// k_update wrote
 __global__ __launch_bounds__(256) void k_pack64(size_t n64, const double *U, double *U64) {
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n64) return;
@@ -2355,32 +2370,48 @@ __global__ void k_zero_f64(double *p, size_t n) {
 //   stage 3: u = 1/3 u0 + 2/3 u2 - 2/3 dt R(u2)/V   -> u2_bar, u0_bar
 //   stage 2: u2 = 3/4 u0 + 1/4 u1 - 1/4 dt R(u1)/V  -> u1_bar, u0_bar
 //   stage 1: u1 = u0 - dt R(u0)/V                    -> u0_bar
-// k_rk3_adj_w forms w = -c dt ybar / V (the cotangent handed to the residual
-// product) for the stage whose output cotangent is ybar; k_rk3_adj_acc then
-// adds a ybar and the product to the cotangents of the stage's inputs.
-__global__ void k_rk3_adj_w(int ncell, const double *ybar, const double *ovol, const double *dt, double c, double *w) {
+// w = -c dt ybar / V is the cotangent handed to the residual product of the
+// stage whose output cotangent is ybar.  k_rk3_adj_w forms it for the last
+// stage; k_rk3_adj_stage then adds a ybar and the product to the cotangents of
+// a stage's inputs, and forms w for the stage before it.  Both clear the
+// product's sum for the stage that follows: four launches of 4-5 us a stage
+// (clear, w, inputs, and a copy of u0_bar a step) are one.
+__global__ void k_rk3_adj_w(int ncell, const double *ybar, const double *ovol, const double *dt, double c, double *w,
+                            double *jt) {
     const size_t n = (size_t)ncell * NV;
-    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x)
+    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x) {
         w[e] = -(c * *dt) * ybar[e] * ovol[e / NV];
+        jt[e] = 0.0;
+    }
 }
 // the cotangents of one stage's inputs from its output cotangent y and the
 // residual product jt = (dR/du)^T w:
 //   stage 3: x = 2/3 y + jt (x = u2_bar), u0_bar = 1/3 y
 //   stage 2: x = 1/4 y + jt (x = u1_bar), u0_bar += 3/4 y   (x may alias y)
-//   stage 1: u0_bar += y + jt
-__global__ void k_rk3_adj_stage(int ncell, int stage, const double *y, const double *jt, double *x, double *u0) {
+//   stage 1: a = u0_bar + y + jt (the step's input)
+// and from them w of the stage before (dt null: there is none)
+__global__ void k_rk3_adj_stage(int ncell, int stage, const double *y, double *jt, double *x, double *u0, double *a,
+                                const double *ovol, const double *dt, double c, double *w) {
     const size_t n = (size_t)ncell * NV;
     const double to4 = 3.0 / 4.0, oo4 = 1.0 / 4.0, to3 = 2.0 / 3.0, oo3 = 1.0 / 3.0;
     for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x) {
         const double ye = y[e], je = jt[e];
+        double yn;  // the output cotangent of the stage before
         if (stage == 3) {
-            x[e] = to3 * ye + je;
+            yn = to3 * ye + je;
+            x[e] = yn;
             u0[e] = oo3 * ye;
         } else if (stage == 2) {
             u0[e] += to4 * ye;
-            x[e] = oo4 * ye + je;
+            yn = oo4 * ye + je;
+            x[e] = yn;
         } else {
-            u0[e] += ye + je;
+            yn = u0[e] + (ye + je);
+            a[e] = yn;
+        }
+        if (dt) {
+            w[e] = -(c * *dt) * yn * ovol[e / NV];
+            jt[e] = 0.0;
         }
     }
 }
@@ -2647,9 +2678,10 @@ LsqView<R> lsq_view(const ucns_ctx *ctx) {
     return L;
 }
 
-// kernel selection by (precision, ideg, imax)
+// kernel selection by (precision, ideg, imax); packed: the last update wrote
+// the state's 64-byte records
 template <typename R>
-int launch_recon_t(ucns_ctx *ctx) {
+int launch_recon_t(ucns_ctx *ctx, bool packed = false) {
     ReconParams<R> p{};
     p.ncell = ctx->ncell;
     p.nf = ctx->nf;
@@ -2754,8 +2786,9 @@ int launch_recon_t(ucns_ctx *ctx) {
         if (ctx->smode) {
             // the row-stream kernels gather the member states from 64-byte records
             const size_t n64 = (size_t)ctx->ncell * 8;
-            hipLaunchKernelGGL(k_pack64, dim3((unsigned)((n64 + 255) / 256)), dim3(256), 0, ctx->stream, n64, ctx->U,
-                               ctx->u64);
+            if (!packed)
+                hipLaunchKernelGGL(k_pack64, dim3((unsigned)((n64 + 255) / 256)), dim3(256), 0, ctx->stream, n64,
+                                   ctx->U, ctx->u64);
             w.U64 = ctx->u64;
         }
         w.gstore = ctx->adj_g_on ? (R *)ctx->adj_g : nullptr;
@@ -2887,9 +2920,9 @@ void tcollect(ucns_ctx *ctx, int k, double *acc, int64_t *n) {
 }
 
 // reconstruction + face fluxes of the current state (ULEFT and face fluxes on device)
-int residual_kernels(ucns_ctx *ctx) {
+int residual_kernels(ucns_ctx *ctx, bool packed = false) {
     tstart(ctx, 0);
-    int rc = ctx->precision == UCNS_MIXED ? launch_recon_t<float>(ctx) : launch_recon_t<double>(ctx);
+    int rc = ctx->precision == UCNS_MIXED ? launch_recon_t<float>(ctx, packed) : launch_recon_t<double>(ctx, packed);
     if (rc) return rc;
     tstop(ctx, 0);
     tcollect(ctx, 0, &ctx->st.ms_recon, &ctx->st.n_recon);
@@ -2903,8 +2936,9 @@ int residual_kernels(ucns_ctx *ctx) {
     return UCNS_OK;
 }
 
+// more: another stage follows, so the row-stream kernels' records are written too
 int update_kernel(ucns_ctx *ctx, int stage, const double *dt, bool dt_slots, unsigned long long *dt_next, double cfl,
-                  double *rhs_out) {
+                  double *rhs_out, bool more = false, double *copy = nullptr) {
     UpdateParams p{};
     p.ncell = ctx->ncell;
     p.nf = ctx->nf;
@@ -2918,6 +2952,8 @@ int update_kernel(ucns_ctx *ctx, int stage, const double *dt, bool dt_slots, uns
     p.U = ctx->U;
     p.U2 = ctx->U2;
     p.rhs_out = rhs_out;
+    p.u64 = more && ctx->smode && !ctx->bmode ? ctx->u64 : nullptr;
+    p.copy = copy;
     p.dt = dt;
     p.dt_slots = dt_slots;
     p.dt_next = dt_next;
@@ -3197,16 +3233,16 @@ int vjp_recon_t(ucns_ctx *ctx) {
 }
 
 // the products of one residual at the state of the last vjp_recon_t: ubar
-// (zeroed here) = the flux product, the reconstruction product and, in
+// (zeroed here unless the caller did) = the flux product, the reconstruction product and, in
 // row-stream mode, the scatter of P^T g_bar (adj_gb) through the member tables
 template <typename R>
-int vjp_products_t(ucns_ctx *ctx, const double *lam, double *ubar, double *bcbar) {
+int vjp_products_t(ucns_ctx *ctx, const double *lam, double *ubar, double *bcbar, bool zeroed = false) {
     const int nfq = ctx->nf * ctx->nqm;
     if (ctx->ts > 8 || nfq > 56) {
         ctx->err = "the residual product needs at most 8 stencils and 56 face points per cell";
         return UCNS_EUNSUPPORTED;
     }
-    zero_dev(ctx, ubar, (size_t)ctx->ncell * NV);
+    if (!zeroed) zero_dev(ctx, ubar, (size_t)ctx->ncell * NV);
     FluxParams<R> fp{};
     fp.nface = ctx->nface;
     fp.nf = ctx->nf;
@@ -3425,25 +3461,29 @@ struct KeptStage {
     }
 };
 
-// one SSP-RK3 step forward from ctx->U with the stage states stored; stages
+// step it of nsteps, SSP-RK3 forward from ctx->U with the stage states stored; stages
 // 3 it + stage - 1 >= keep0 also keep their reconstruction
-int rk3_step_ckpt(ucns_ctx *ctx, int it, const double *dt, unsigned long long *next, double cfl, int keep0) {
+int rk3_step_ckpt(ucns_ctx *ctx, int it, int nsteps, const double *dt, unsigned long long *next, double cfl,
+                  int keep0) {
     const size_t n = (size_t)ctx->ncell * NV;
     for (int stage = 1; stage <= 3; ++stage) {
         const int q = 3 * it + stage - 1;
-        HIP_TRY(hipMemcpyAsync(ctx->ckpt + (size_t)q * n, ctx->U, n * sizeof(double), hipMemcpyDeviceToDevice,
-                               ctx->stream));
+        // the stages after the first find their state stored by the update
+        if (q == 0)
+            HIP_TRY(hipMemcpyAsync(ctx->ckpt, ctx->U, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
         int rc;
         if (q >= keep0) {
             KeptStage k(ctx, q - keep0);
             ctx->adj_g_on = ctx->smode != 0;
-            rc = residual_kernels(ctx);
+            rc = residual_kernels(ctx, q > 0);
             ctx->adj_g_on = false;
         } else {
-            rc = residual_kernels(ctx);
+            rc = residual_kernels(ctx, q > 0);
         }
         if (rc) return rc;
-        update_kernel(ctx, stage, dt, next != nullptr, next, cfl, nullptr);
+        const bool more = q + 1 < 3 * nsteps;
+        update_kernel(ctx, stage, dt, next != nullptr, next, cfl, nullptr, more,
+                      more ? ctx->ckpt + (size_t)(q + 1) * n : nullptr);
     }
     return UCNS_OK;
 }
@@ -3452,7 +3492,7 @@ int rk3_step_ckpt(ucns_ctx *ctx, int it, const double *dt, unsigned long long *n
 // the final state on entry and of the initial state on return.  Stages are
 // reversed in the order (step n: 3, 2, 1), each at its stored state, with
 //   w = -c dt ybar / V, jt = (dR/du)^T w, and k_rk3_adj_stage combining ybar
-//   and jt into the cotangents of the stage's inputs.
+//   and jt into the cotangents of the stage's inputs and the next w.
 // In row-stream mode the scatter of a stage's reconstruction product rides on
 // the forward reconstruction of the next stage reversed, so each reversed
 // stage streams the pseudo-inverses once.
@@ -3473,20 +3513,22 @@ int rk3_reverse_t(ucns_ctx *ctx, int nsteps, double *abar, double *bcbar, int ke
         for (int stage = 3; stage >= 1 && rc == UCNS_OK; --stage) {
             ctx->U = ctx->ckpt + ((size_t)3 * it + stage - 1) * n;
             const double *y = stage == 3 ? a : x;
-            hipLaunchKernelGGL(k_rk3_adj_w, dim3(blocks), dim3(256), 0, ctx->stream, ctx->ncell, y, ctx->ovol, dt,
-                               cst[stage], w);
+            if (it == nsteps - 1 && stage == 3)
+                hipLaunchKernelGGL(k_rk3_adj_w, dim3(blocks), dim3(256), 0, ctx->stream, ctx->ncell, y, ctx->ovol,
+                                   dt, cst[stage], w, jt);
             const int q = 3 * it + stage - 1;
             if (q >= keep0) {
                 KeptStage k(ctx, q - keep0);
-                if ((rc = vjp_products_t<R>(ctx, w, jt, bcbar))) break;
+                if ((rc = vjp_products_t<R>(ctx, w, jt, bcbar, true))) break;
             } else {
                 if ((rc = vjp_recon_t<R>(ctx))) break;
-                if ((rc = vjp_products_t<R>(ctx, w, jt, bcbar))) break;
+                if ((rc = vjp_products_t<R>(ctx, w, jt, bcbar, true))) break;
             }
-            // this stage's product is complete: fold it into its input cotangents
+            // this stage's product is complete: fold it into its input
+            // cotangents, and form the cotangent of the stage before
+            const double *ndt = stage > 1 ? dt : it > 0 ? dt - 1 : nullptr;
             hipLaunchKernelGGL(k_rk3_adj_stage, dim3(blocks), dim3(256), 0, ctx->stream, ctx->ncell, stage, y, jt, x,
-                               u0);
-            if (stage == 1) (void)hipMemcpyAsync(a, u0, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream);
+                               u0, a, ctx->ovol, ndt, cst[stage > 1 ? stage - 1 : 3], w);
         }
     }
     ctx->U = ustate;
@@ -4635,8 +4677,8 @@ int ucns_rk3_steps(ucns_ctx *ctx, int32_t nsteps, double cfl, double dt_fixed, d
         const double *dt = fixed ? ctx->dtfix : (const double *)(ctx->dtv + cur * DT_SLOTS * DT_STRIDE);
         unsigned long long *next = fixed ? nullptr : ctx->dtv + (1 - cur) * DT_SLOTS * DT_STRIDE;
         for (int stage = 1; stage <= 3; ++stage) {
-            if ((rc = residual_kernels(ctx))) return rc;
-            update_kernel(ctx, stage, dt, !fixed, next, cfl, nullptr);
+            if ((rc = residual_kernels(ctx, it > 0 || stage > 1))) return rc;
+            update_kernel(ctx, stage, dt, !fixed, next, cfl, nullptr, it + 1 < nsteps || stage < 3);
         }
         HIP_TRY(hipGetLastError());
         if (!fixed) cur = 1 - cur;
@@ -4727,7 +4769,7 @@ static int rk3_adjoint_impl(ucns_ctx *ctx, int32_t nsteps, double cfl, double dt
             HIP_TRY(hipMemcpyAsync(ctx->dts + it, dt, sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
         else
             hipLaunchKernelGGL(k_dt_value, dim3(1), dim3(WAVE), 0, ctx->stream, dt, ctx->dts + it);
-        if ((rc = rk3_step_ckpt(ctx, it, dt, next, cfl, keep0))) return rc;
+        if ((rc = rk3_step_ckpt(ctx, it, nsteps, dt, next, cfl, keep0))) return rc;
         HIP_TRY(hipGetLastError());
         if (!fixed) cur = 1 - cur;
     }
