@@ -1,13 +1,18 @@
 """Kernels that are chosen by a rule on the mesh, each at the sizes where its
-split can go wrong: against the oracle, or against the kernels that the rule
-leaves (another summation order in FP64: differences of a few hundred roundings
-of 1.1e-16, held to 1e-12 of the largest value; products behind a march 1e-10)."""
+split can go wrong: tiles and blocks with a remainder, tables that overflow,
+both sides of a rule's line.  Against the oracle at the parity bars
+(reconstruction 1e-12, residual 1e-11, relative L2 per variable), or against
+the kernels that the rule leaves (another order of FP64 sums: a few hundred
+roundings of 1.1e-16, held to 1e-12 of the largest value; cotangents behind a
+march to 1e-10)."""
 import numpy as np
 import pytest
 
-from ucns3d_amd.case import PRISM, Case, CaseSpec, reduced
+from oracle.oracle import Oracle
+from shuffle import shuffled_structs
+from ucns3d_amd.case import HEX, PRISM, TET, Case, CaseSpec, reduced
 from ucns3d_amd.native import UCNS_FP64, UCNS_KERNELS_REGISTER
-from ucns3d_amd.solver import Solver
+from ucns3d_amd.solver import Solver, UcnsError
 
 pytestmark = pytest.mark.gpu
 
@@ -17,6 +22,109 @@ def close(a, b, tol):
     assert np.isfinite(a).all()
     d = np.abs(a - b).max()
     assert d <= tol * np.abs(b).max(), (d, np.abs(b).max())
+
+
+def rel_l2(a, b):
+    """relative L2 per variable, the momenta against the whole momentum"""
+    a, b = a.reshape(-1, 5), b.reshape(-1, 5)
+    num, den = np.sqrt(((a - b) ** 2).sum(0)), np.sqrt((b ** 2).sum(0))
+    den[1:4] = np.sqrt((den[1:4] ** 2).sum())
+    return num / den
+
+
+# cell counts that are no multiple of a tile (8 cells) or of a block (32)
+REMAINDERS = {
+    "hex-muscl-125": CaseSpec("r-muscl", HEX, 5, "muscl", jitter=0.1, seed=3),
+    "hex-weno4-729": CaseSpec("r-hex4", HEX, 9, "weno4", jitter=0.1, seed=3),
+    "hex-weno4-char-729": CaseSpec("r-hex4c", HEX, 9, "weno4", jitter=0.1, seed=3, wenwrt=2),
+    "tet-weno4-char-750": CaseSpec("r-tet4c", TET, 5, "weno4", jitter=0.1, seed=3, wenwrt=2),
+    "prism-weno3-686": CaseSpec("r-prism3", PRISM, 7, "weno3", jitter=0.1, seed=3),
+    "tet-cweno5-2058": CaseSpec("r-tet5", TET, 7, "weno5", jitter=0.1, seed=3, ees=5),
+}
+
+
+@pytest.mark.parametrize("name", list(REMAINDERS))
+def test_remainders_against_the_oracle(name):
+    case = Case(REMAINDERS[name])
+    assert case.ncell == int(name.split("-")[-1]) and case.ncell % 8 and case.ncell % 32
+    u = case.init_state()
+    orc = Oracle(case)
+    r_ref, cnt = orc.residual(u)
+    print(f"[remainder] {name}", flush=True)
+    s = Solver(case, UCNS_FP64)
+    s.set_state(u)
+    err = rel_l2(s.residual(), r_ref)
+    st = s.stats()
+    s.close()
+    print("  residual", err)
+    assert (st["n_reduced_last"], st["n_firstorder_last"]) == (cnt[0], cnt[1])
+    assert np.all(err <= 1e-11), err
+
+
+# tiles whose distinct members exceed the table in LDS (512 rows; 768 with 7
+# stencils of 39 members): 8 cells far apart, in the caller's order
+OVERFLOW = {
+    "hex-weno4": CaseSpec("o-hex4", HEX, 11, "weno4", jitter=0.1, seed=5),
+    "tet-weno4-char": CaseSpec("o-tet4c", TET, 7, "weno4", jitter=0.1, seed=5, wenwrt=2),
+    "prism-weno3": CaseSpec("o-prism3", PRISM, 9, "weno3", jitter=0.1, seed=5),
+}
+
+
+@pytest.mark.parametrize("name", list(OVERFLOW))
+def test_tiles_past_the_member_table(name):
+    case = Case(OVERFLOW[name])
+    u = case.init_state() * (1 + 1e-3 * np.random.default_rng(2).uniform(-1, 1, (case.ncell, 5)))
+    sh = np.random.default_rng(4).permutation(case.ncell).astype(np.int64)
+    keep, st = shuffled_structs(case, sh)
+    w = np.random.default_rng(6).standard_normal(u.shape)
+    print(f"[member table] {name} ncell={case.ncell}", flush=True)
+    a = Solver(case, UCNS_FP64)
+    b = Solver(case, UCNS_FP64, structs=st)
+    a.set_state(u)
+    b.set_state(u[sh])
+    close(b.reconstruct(), a.reconstruct()[sh], 1e-12)
+    if case.spec.wenwrt == 1:  # the products do not cover characteristic variables
+        close(b.residual_vjp(w[sh])[0], a.residual_vjp(w)[0][sh], 1e-10)
+    a.close()
+    b.close()
+
+
+# marches on one-point faces: fluxes and update in one kernel up to 32,768
+# cells; a timed context keeps the two kernels
+@pytest.mark.parametrize("n", [3, 5, 31, 33])
+def test_march_on_one_point_faces(n):
+    case = Case(CaseSpec("f-muscl", HEX, n, "muscl", jitter=0.1, seed=3))
+    u = case.init_state()
+    out = []
+    for timed in (False, True):
+        print(f"[one-point march] ncell={case.ncell} timed={timed}", flush=True)
+        s = Solver(case, UCNS_FP64)
+        if timed:
+            s.reset_stats()
+        s.set_state(u)
+        t = s.rk3_steps(3, cfl=0.5)
+        out.append((s.get_state(), t))
+        s.close()
+    (a, ta), (b, tb) = out
+    close(a, b, 1e-12)
+    assert abs(ta - tb) <= 1e-12 * tb
+
+
+# the last value of a state, with one block per 1,024 values and with more
+# values than the 256 blocks take in one trip
+@pytest.mark.parametrize("n", [3, 38])
+def test_non_finite_last_value(n):
+    case = Case(CaseSpec("nf-muscl", HEX, n, "muscl", seed=3))
+    u = case.init_state()
+    print(f"[non-finite last value] ncell={case.ncell}", flush=True)
+    s = Solver(case, UCNS_FP64)
+    s.set_state(u)
+    s.rk3_steps(0, dt_fixed=1e-3)
+    u[-1, 4] = np.inf
+    s.set_state(u)
+    with pytest.raises(UcnsError, match="non-finite"):
+        s.rk3_steps(0, dt_fixed=1e-3)
+    s.close()
 
 
 @pytest.mark.parametrize("spec", [CaseSpec("geo-prism", PRISM, 3, "weno3", jitter=0.1, seed=13), reduced("c4", 3)],
