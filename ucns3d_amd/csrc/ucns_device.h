@@ -22,7 +22,11 @@ constexpr int NXCD = 8;
 // distinct members with WENO-4 on tets (5 stencils), 373 with WENO-3 on
 // hexes, 660 with WENO-4 on hexes (7 stencils of 39 members)
 constexpr int tile_uq(int ts, int imax) { return ts > 5 && imax > 19 ? 768 : UCNS_TILE_UQ; }
-constexpr int NPART = 64;  // blocks (and results) of k_marks_sum
+constexpr int NPART = 256;  // blocks (and results) of k_finish
+struct HostResult {
+    int part[NPART][4];  // per block: reduced cells, first-order cells, non-finite values, 0
+    double t;
+};
 // monomial exponents of BASIS_REC (src/basis.f90:11-102), cubic max here
 static __constant__ int8_t c_mono[34][3] = {
     {1, 0, 0}, {0, 1, 0}, {0, 0, 1},

@@ -2531,29 +2531,46 @@ __global__ void k_rk3_adj_stage(int ncell, int stage, const double *y, double *j
 }
 
 __global__ void k_fill_u64(unsigned long long *p, unsigned long long v) { p[threadIdx.x] = v; }
-// sums of the blocks' troubled-cell marks into part[gridDim.x][2]
-__global__ __launch_bounds__(256) void k_marks_sum(const int *marks, int n, int *part) {
-    __shared__ int sh[2][256 / WAVE];
-    int a = 0, b = 0;
+// the time and the fixed step of a march
+__global__ void k_set2(double *p, double a, double *q, double b) {
+    if (threadIdx.x == 0) {
+        *p = a;
+        *q = b;
+    }
+}
+// What a call hands back to the host, written straight into pinned host memory
+// (one launch and one wait where a clear, two sums and three copies through
+// pageable memory held the stream for 100 us after a march): the sums of the
+// blocks' troubled-cell marks, whether u holds a non-finite value (nu = 0: not
+// looked at), and the time.
+__global__ __launch_bounds__(256) void k_finish(const int *marks, int n, const double *u, size_t nu, const double *t,
+                                                HostResult *out) {
+    __shared__ int sh[3][256 / WAVE];
+    int a = 0, b = 0, bad = 0;
     for (int e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) {
         a += marks[e] & 65535;
         b += marks[e] >> 16;
     }
+    for (size_t e = blockIdx.x * 256 + threadIdx.x; e < nu; e += gridDim.x * 256)
+        if (!isfinite(u[e])) bad = 1;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         a += __shfl_xor(a, o, WAVE);
         b += __shfl_xor(b, o, WAVE);
+        bad |= __shfl_xor(bad, o, WAVE);
     }
     if ((threadIdx.x & (WAVE - 1)) == 0) {
         sh[0][threadIdx.x / WAVE] = a;
         sh[1][threadIdx.x / WAVE] = b;
+        sh[2][threadIdx.x / WAVE] = bad;
     }
     __syncthreads();
-    if (threadIdx.x < 2) {
-        int t = 0;
-        for (int w = 0; w < 256 / WAVE; ++w) t += sh[threadIdx.x][w];
-        part[blockIdx.x * 2 + threadIdx.x] = t;
+    if (threadIdx.x < 3) {
+        int v = 0;
+        for (int w = 0; w < 256 / WAVE; ++w) v += sh[threadIdx.x][w];
+        out->part[blockIdx.x][threadIdx.x] = v;
     }
+    if (t && blockIdx.x == 0 && threadIdx.x == 0) out->t = *t;
 }
 
 // Per-cell 5-vectors across the ABI: the caller's cell o = perm[c] (o = c
@@ -2576,14 +2593,6 @@ __global__ __launch_bounds__(256) void k_cells_out(int ncell, const int32_t *per
 #pragma unroll
     for (int v = 0; v < NV; ++v)
         dst[layout == UCNS_LAYOUT_AOS ? o * NV + v : (size_t)v * ncell + o] = src[(size_t)c * NV + v];
-}
-
-__global__ void k_nonfinite(const double *u, size_t n, int *flag) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int bad = 0;
-    for (; i < n; i += (size_t)gridDim.x * blockDim.x)
-        if (!isfinite(u[i])) bad = 1;
-    if (bad) atomicOr(flag, 1);
 }
 
 // [cells][ts_in][imax][ideg] (FP64, ABI) -> [cells][imax][ts_out][ideg] (R)
@@ -2707,9 +2716,9 @@ struct ucns_ctx {
     int4 *fadj = nullptr;      // face records by cell of k_flux_update (null: it does not run)
     double *U = nullptr, *U2 = nullptr, *fflux = nullptr, *rhs = nullptr, *t = nullptr, *dtfix = nullptr;
     unsigned long long *dtv = nullptr;  // [2][DT_SLOTS * DT_STRIDE] ping-pong dt slots
-    int *marks = nullptr, *marks_part = nullptr;  // troubled cells per reconstruction block; their sums [NPART][2]
+    int *marks = nullptr;          // troubled cells per reconstruction block
+    HostResult *result = nullptr;  // pinned host memory, written by k_finish
     int nmark = 0;
-    int *flag = nullptr;
     // adjoint (allocated on first use): face-point cotangents, state-sized
     // work arrays, the free-stream cotangent, stage checkpoints and step dts
     double *adj_ubf = nullptr, *adj_lam = nullptr, *adj_ubar = nullptr, *adj_x = nullptr, *adj_a = nullptr;
@@ -3130,21 +3139,38 @@ int fused_step(ucns_ctx *ctx, const double *dt, bool dt_slots, unsigned long lon
     return UCNS_OK;
 }
 
-// the troubled-cell counts of the last reconstruction into the statistics;
-// waits for the stream
-int collect_counts(ucns_ctx *ctx) {
-    int part[2 * NPART];
-    hipLaunchKernelGGL(k_marks_sum, dim3(NPART), dim3(256), 0, ctx->stream, ctx->marks, ctx->nmark, ctx->marks_part);
+int finish_blocks(const ucns_ctx *ctx, size_t nu) {
+    return (int)std::min<size_t>(NPART, std::max<size_t>(1, (std::max<size_t>(ctx->nmark, nu) + 1023) / 1024));
+}
+
+// queues the result of a call; the stream is waited for before it is read
+int queue_result(ucns_ctx *ctx, size_t nu, const double *t) {
+    hipLaunchKernelGGL(k_finish, dim3(finish_blocks(ctx, nu)), dim3(256), 0, ctx->stream, ctx->marks, ctx->nmark,
+                       ctx->U, nu, t, ctx->result);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(part, ctx->marks_part, sizeof(part), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    return UCNS_OK;
+}
+
+// the troubled-cell counts of the last reconstruction into the statistics;
+// true if the state was found non-finite
+bool read_result(ucns_ctx *ctx, size_t nu) {
     int64_t red = 0, fst = 0;
-    for (int b = 0; b < NPART; ++b) {
-        red += part[2 * b];
-        fst += part[2 * b + 1];
+    int bad = 0;
+    for (int b = 0; b < finish_blocks(ctx, nu); ++b) {
+        red += ctx->result->part[b][0];
+        fst += ctx->result->part[b][1];
+        bad += ctx->result->part[b][2];
     }
     ctx->st.n_reduced_last = red;
     ctx->st.n_firstorder_last = fst;
+    return bad != 0;
+}
+
+int collect_counts(ucns_ctx *ctx) {
+    const int rc = queue_result(ctx, 0, nullptr);
+    if (rc) return rc;
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    read_result(ctx, 0);
     return UCNS_OK;
 }
 
@@ -4199,9 +4225,9 @@ int ucns_create(const ucns_mesh_v2 *m, const ucns_scheme_v2 *s, ucns_ctx **out) 
         (rc = dalloc(ctx, &ctx->U2, (size_t)nc * NV)) || (rc = dalloc(ctx, &ctx->rhs, (size_t)nc * NV)) ||
         (rc = dalloc(ctx, &ctx->fflux, (size_t)ctx->nface * NV)) || (rc = dalloc(ctx, &ctx->t, 1)) ||
         (rc = dalloc(ctx, &ctx->dtfix, 1)) || (rc = dalloc(ctx, &ctx->dtv, 2 * DT_SLOTS * DT_STRIDE)) ||
-        (rc = dalloc(ctx, &ctx->marks_part, 2 * NPART)) || (rc = dalloc(ctx, &ctx->flag, 1)) ||
         (rc = dalloc(ctx, &ctx->stage, (size_t)nc * NV)))
         return rc;
+    HIP_TRY(hipHostMalloc((void **)&ctx->result, sizeof(HostResult), hipHostMallocDefault));
     if (!bfaces.empty()) {
         if ((rc = dalloc(ctx, &ctx->bfaces, bfaces.size()))) return rc;
         HIP_TRY(hipMemcpy(ctx->bfaces, bfaces.data(), bfaces.size() * sizeof(int32_t), hipMemcpyHostToDevice));
@@ -4792,8 +4818,10 @@ static int residual_to(ucns_ctx *ctx, double *rhs_out, int32_t layout, bool host
     if ((rc = residual_kernels(ctx))) return rc;
     update_kernel(ctx, 0, nullptr, false, nullptr, 0.0, ctx->rhs);
     HIP_TRY(hipGetLastError());
-    if ((rc = collect_counts(ctx))) return rc;
-    if (rhs_out) return cells_out(ctx, ctx->rhs, layout, rhs_out, host);
+    if (!rhs_out) return collect_counts(ctx);
+    if ((rc = queue_result(ctx, 0, nullptr))) return rc;
+    if ((rc = cells_out(ctx, ctx->rhs, layout, rhs_out, host))) return rc;  // waits for the stream
+    read_result(ctx, 0);
     return UCNS_OK;
 }
 
@@ -4822,10 +4850,12 @@ int ucns_residual_noalloc(ucns_ctx *ctx, double *rhs_dev, int32_t layout) {
     ctx->fflux = (double *)((unsigned char *)ctx->scratch + UCNS_SCRATCH_HEAD);
     rc = residual_kernels(ctx);
     if (rc == UCNS_OK) update_kernel(ctx, 0, nullptr, false, nullptr, 0.0, ctx->rhs);
-    if (rc == UCNS_OK) rc = collect_counts(ctx);
+    if (rc == UCNS_OK) rc = queue_result(ctx, 0, nullptr);
+    if (rc == UCNS_OK) rc = cells_out(ctx, ctx->rhs, layout, rhs_dev, false);  // waits for the stream
     ctx->fflux = own_fflux;
     if (rc) return rc;
-    return cells_out(ctx, ctx->rhs, layout, rhs_dev, false);
+    read_result(ctx, 0);
+    return UCNS_OK;
 }
 
 int ucns_residual_device(ucns_ctx *ctx, double *rhs_dev, int32_t layout) {
@@ -4843,9 +4873,8 @@ int ucns_rk3_steps(ucns_ctx *ctx, int32_t nsteps, double cfl, double dt_fixed, d
     if (rc) return rc;
     HIP_TRY(hipSetDevice(ctx->device));
     const double t0 = t_io ? *t_io : 0.0;
-    HIP_TRY(hipMemcpyAsync(ctx->t, &t0, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
     const bool fixed = dt_fixed > 0;
-    if (fixed) HIP_TRY(hipMemcpyAsync(ctx->dtfix, &dt_fixed, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    hipLaunchKernelGGL(k_set2, dim3(1), dim3(WAVE), 0, ctx->stream, ctx->t, t0, ctx->dtfix, dt_fixed);
     int cur = 0;
     if (!fixed && nsteps > 0) dt_kernel(ctx, cfl, ctx->dtv);
     for (int it = 0; it < nsteps; ++it) {
@@ -4860,16 +4889,12 @@ int ucns_rk3_steps(ucns_ctx *ctx, int32_t nsteps, double cfl, double dt_fixed, d
         HIP_TRY(hipGetLastError());
         if (!fixed) cur = 1 - cur;
     }
-    HIP_TRY(hipMemsetAsync(ctx->flag, 0, sizeof(int), ctx->stream));
-    hipLaunchKernelGGL(k_nonfinite, dim3(1024), dim3(256), 0, ctx->stream, ctx->U, (size_t)ctx->ncell * NV,
-                       ctx->flag);
-    int flag = 0;
-    double t1 = t0;
-    HIP_TRY(hipMemcpyAsync(&flag, ctx->flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipMemcpyAsync(&t1, ctx->t, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    if ((rc = collect_counts(ctx))) return rc;  // waits for the copies above
-    if (t_io) *t_io = t1;
-    if (flag) {
+    const size_t nu = (size_t)ctx->ncell * NV;
+    if ((rc = queue_result(ctx, nu, ctx->t))) return rc;
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    const bool bad = read_result(ctx, nu);
+    if (t_io) *t_io = ctx->result->t;
+    if (bad) {
         ctx->err = "non-finite state after the RK3 steps";
         return UCNS_ENONFINITE;
     }
@@ -4934,9 +4959,8 @@ static int rk3_adjoint_impl(ucns_ctx *ctx, int32_t nsteps, double cfl, double dt
     }
     const int keep0 = 3 * nsteps - adj_keep(ctx, 3 * nsteps);
     const double t0 = t_io ? *t_io : 0.0;
-    HIP_TRY(hipMemcpyAsync(ctx->t, &t0, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
     const bool fixed = dt_fixed > 0;
-    if (fixed) HIP_TRY(hipMemcpyAsync(ctx->dtfix, &dt_fixed, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    hipLaunchKernelGGL(k_set2, dim3(1), dim3(WAVE), 0, ctx->stream, ctx->t, t0, ctx->dtfix, dt_fixed);
     int cur = 0;
     if (!fixed) dt_kernel(ctx, cfl, ctx->dtv);
     for (int it = 0; it < nsteps; ++it) {
@@ -4952,11 +4976,9 @@ static int rk3_adjoint_impl(ucns_ctx *ctx, int32_t nsteps, double cfl, double dt
     }
     zero_dev(ctx, ctx->adj_bc, 2 * NV);
     if ((rc = rk3_reverse(ctx, nsteps, a_dev, ctx->adj_bc, keep0))) return rc;
-    HIP_TRY(hipGetLastError());
-    double t1 = t0;
-    HIP_TRY(hipMemcpyAsync(&t1, ctx->t, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    if ((rc = queue_result(ctx, 0, ctx->t))) return rc;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
-    if (t_io) *t_io = t1;
+    if (t_io) *t_io = ctx->result->t;
     return UCNS_OK;
 }
 
@@ -5179,9 +5201,9 @@ void ucns_destroy(ucns_ctx *ctx) {
     dfree(ctx->t);
     dfree(ctx->dtfix);
     dfree(ctx->dtv);
-    dfree(ctx->marks_part);
+    if (ctx->result) (void)hipHostFree(ctx->result);
+    ctx->result = nullptr;
     dfree(ctx->bfaces);
-    dfree(ctx->flag);
     dfree(ctx->uleft);
     for (auto &e : ctx->ev)
         if (e) (void)hipEventDestroy(e);
