@@ -874,12 +874,11 @@ __global__ __launch_bounds__(256) void k_flux(FluxParams<R> p) {
 }
 
 // The same with one thread per (face, quadrature point), for meshes whose
-// faces do not fill the chip and whose faces have several points: nqm times
+// faces have several points: nqm times
 // the waves, and a point's chain of divisions and square roots runs beside the
 // others' instead of after them.  The points' contributions meet in LDS, where
 // thread (face, variable) adds them in point order (the order and rounding of
-// the one-thread loop).  5,184 hexahedra faces of 9 points: 18.8 -> 6.2 us; on
-// 256,000 and more faces it is slower by 3-7% (rule at the launch).
+// the one-thread loop).  5,184 hexahedra faces of 9 points: 18.8 -> 6.2 us.
 template <typename R>
 __global__ __launch_bounds__(256) void k_flux_points(FluxParams<R> p) {
     __shared__ double sh[256][NV + 1];  // per point: the rotated-back flux and its weight times the area
@@ -3021,12 +3020,12 @@ FluxParams<R> flux_params(const ucns_ctx *ctx) {
 template <typename R>
 void launch_flux_t(ucns_ctx *ctx) {
     const FluxParams<R> p = flux_params<R>(ctx);
-    // Half of the threads the chip holds at the kernel's registers (2^18): below
-    // it a thread per point wins (5,184 hexahedra faces 18.8 -> 6.2 us, 31,000
-    // channel faces 15.9 -> 9 us), well above it a thread per face (280,000
-    // channel faces 52 us against 54, 393,000 tetrahedra faces 93 against 100).
-    // Faces of one point gain nothing from it (5.7 against 7.9 us on 41,472).
-    if (ctx->nqm > 1 && ctx->nface < 131072) {
+    // A thread per point where faces have several: 5,184 hexahedra faces 18.8 ->
+    // 6.2 us, 31,000 channel faces 15.9 -> 9 us; marches on 169,000 (channel) to
+    // 393,000 (tetrahedra) faces take the same time within 0.3% either way, on
+    // 69,000 hexahedra in mixed precision 2.66 -> 2.62 ms.  Faces of one point gain
+    // nothing from it (5.7 against 7.9 us on 41,472).
+    if (ctx->nqm > 1) {
         const int fpb = 256 / ctx->nqm;  // faces per block
         hipLaunchKernelGGL((k_flux_points<R>), dim3((ctx->nface + fpb - 1) / fpb), dim3(256), 0, ctx->stream, p);
     } else {
