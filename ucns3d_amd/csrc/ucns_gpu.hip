@@ -2249,26 +2249,27 @@ __global__ void k_adj_csr(int ntile, int cap, const int32_t *uq, const int32_t *
 // free-stream values) from forward-mode passes of the same templated code the
 // primal runs, one pass per input; F_bar is pulled back through ROTATEB
 // (whose transpose is ROTATEF) and ROTATEF (transpose ROTATEB).
-// BND: the launch over boundary faces (ghost-state Jacobians by forward
-// mode); the other launch takes the interior and periodic faces, whose
-// kernel then carries none of the boundary code's registers
 //
-// One thread per (face, quadrature point): the points are independent, their
-// writes are contiguous across lanes, and a small mesh still fills the chip
-// (one thread per face left 121 blocks for a 14,000-cell channel).  The
-// boundary launch runs over the list of boundary faces, so its waves are
-// full, and reduces the ten free-stream cotangents in the block before its
-// atomics (same-address atomics retire one per 12 ns).
-// 14,000-cell channel: interior 19.4 -> 10.6 us, boundary 113.7 -> 20.6 us;
-// 24,576 tetrahedra: 34.9 -> 22.4 us.
+// One thread per interior (face, quadrature point): the points are independent,
+// their writes are contiguous across lanes, and a small mesh still fills the
+// chip (one thread per face left 121 blocks for a 14,000-cell channel).
+// Boundary faces, by list, come in the first blocks of the same launch (meshes
+// without any get a kernel without their registers) with 16 lanes per point: a
+// lane per ghost-state input, where one thread ran the 15 passes one after the
+// other.  The block reduces the free-stream cotangents before its atomics
+// (same-address atomics retire one per 12 ns).
+// 14,000-cell channel: a thread per face 19.4 us and, boundary, 113.7; a thread
+// per point 10.6 and 20.6; this launch 19.5.  24,576 tetrahedra: 34.9 -> 22.4 us.
+constexpr int BLANES = 16;
 template <typename R, bool BND>
-__global__ __launch_bounds__(256) void k_flux_vjp(FluxParams<R> p, const int32_t *bfaces, int nbface,
-                                                  const double *lam, double *ubf, double *bcbar) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void flux_vjp_block(const FluxParams<R> &p, int block, const int32_t *bfaces, int nbface,
+                                               const double *lam, double *ubf, double *bcbar) {
+    const int t = (block * 256 + (int)threadIdx.x) / (BND ? BLANES : 1);
     const int fi = t / p.nqm, q = t - fi * p.nqm;
     const int f = BND ? (fi < nbface ? bfaces[fi] : p.nface) : fi;
     constexpr bool bnd = BND;
-    double bcacc[2 * NV] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const int m = threadIdx.x & (BLANES - 1);
+    double bcd = 0.0;  // boundary: this lane's free-stream cotangent
     auto point = [&]() {
         const int cL = p.fcell[2 * f], cR = p.fcell[2 * f + 1];
         if ((cR < 0) != BND) return;
@@ -2304,64 +2305,68 @@ __global__ __launch_bounds__(256) void k_flux_vjp(FluxParams<R> p, const int32_t
         rotb(lab, c1, s1, c2, s2, ab);
         rotb(rab, c1, s1, c2, s2, bb);
         if (bnd) {
-            const int code = -cR;
-#pragma unroll 1
-            for (int m = 0; m < NV; ++m) {
-                Dual A[NV], G[NV];
+            // lane m: the derivative along the cell's value m (m < 5), the inflow
+            // state's m - 5 (an outflow face does not read it) or the outflow
+            // state's m - 10 (an inflow face does not); the lanes of a point
+            // repeat everything up to here
+            const int code = -cR, e = m - NV;
+            const bool fs = bcbar && (code == 1 || code == 2 || code == 6) && e < 2 * NV && (e < NV ? code != 2 : code != 1);
+            double d = 0.0;
+            if (m < NV || fs) {
+                Dual A[NV], G[NV], fin[NV], fo[NV];
 #pragma unroll
-                for (int v = 0; v < NV; ++v) A[v] = Dual{a[v], m == v ? 1.0 : 0.0};
-                ghost_state(code, p.bc.boundtype, p.gamma, A, c1, s1, c2, s2, p.bc.inflow, p.bc.outflow, G);
-                double d = 0.0;
+                for (int v = 0; v < NV; ++v) {
+                    A[v] = Dual{a[v], m == v ? 1.0 : 0.0};
+                    fin[v] = Dual{p.bc.inflow[v], e == v ? 1.0 : 0.0};
+                    fo[v] = Dual{p.bc.outflow[v], e == NV + v ? 1.0 : 0.0};
+                }
+                ghost_state(code, p.bc.boundtype, p.gamma, A, c1, s1, c2, s2, fin, fo, G);
 #pragma unroll
                 for (int v = 0; v < NV; ++v) d += bb[v] * G[v].d;
-#pragma unroll
-                for (int v = 0; v < NV; ++v) ab[v] += m == v ? d : 0.0;
             }
-            if (bcbar && (code == 1 || code == 2 || code == 6)) {
-                // an inflow face reads the inflow state only, an outflow face
-                // the outflow state, a farfield face either
-#pragma unroll 1
-                for (int m = code == 2 ? NV : 0; m < (code == 1 ? NV : 2 * NV); ++m) {
-                    Dual A[NV], G[NV], fin[NV], fo[NV];
+            if (m < NV) {
+                double am = ab[0];
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) {
-                        A[v] = Dual{a[v], 0.0};
-                        fin[v] = Dual{p.bc.inflow[v], m == v ? 1.0 : 0.0};
-                        fo[v] = Dual{p.bc.outflow[v], m == NV + v ? 1.0 : 0.0};
-                    }
-                    ghost_state(code, p.bc.boundtype, p.gamma, A, c1, s1, c2, s2, fin, fo, G);
-                    double d = 0.0;
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) d += bb[v] * G[v].d;
-#pragma unroll
-                    for (int e = 0; e < 2 * NV; ++e) bcacc[e] += m == e ? d : 0.0;
-                }
+                for (int v = 1; v < NV; ++v) am = m == v ? ab[v] : am;
+                ubf[oL + m] = am + d;
+            } else {
+                bcd = d;
             }
         } else {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) ubf[oR + v] = bb[v];
+            for (int v = 0; v < NV; ++v) {
+                ubf[oR + v] = bb[v];
+                ubf[oL + v] = ab[v];
+            }
         }
-#pragma unroll
-        for (int v = 0; v < NV; ++v) ubf[oL + v] = ab[v];
     };
     if (f < p.nface) point();
     if constexpr (BND) {
         if (!bcbar) return;
-        __shared__ double sh[256 / WAVE][2 * NV];
-#pragma unroll
-        for (int m = 0; m < 2 * NV; ++m) {
-            double x = bcacc[m];
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, WAVE);
-            if ((threadIdx.x & (WAVE - 1)) == 0) sh[threadIdx.x / WAVE][m] = x;
-        }
+        __shared__ double sh[256 / WAVE][BLANES];
+        bcd += __shfl_xor(bcd, 16, WAVE);
+        bcd += __shfl_xor(bcd, 32, WAVE);
+        if ((threadIdx.x & (WAVE - 1)) < BLANES) sh[threadIdx.x / WAVE][m] = bcd;
         __syncthreads();
         if (threadIdx.x < 2 * NV) {
             double x = 0.0;
-            for (int wv = 0; wv < 256 / WAVE; ++wv) x += sh[wv][threadIdx.x];
+            for (int wv = 0; wv < 256 / WAVE; ++wv) x += sh[wv][NV + threadIdx.x];
             if (x != 0.0) atomic_add_f64(&bcbar[threadIdx.x], x);
         }
     }
+}
+
+// EDGES: the first nbblock blocks take the boundary faces
+template <typename R, bool EDGES>
+__global__ __launch_bounds__(256) void k_flux_vjp(FluxParams<R> p, const int32_t *bfaces, int nbface, int nbblock,
+                                                  const double *lam, double *ubf, double *bcbar) {
+    if constexpr (EDGES) {
+        if ((int)blockIdx.x < nbblock) {
+            flux_vjp_block<R, true>(p, blockIdx.x, bfaces, nbface, lam, ubf, bcbar);
+            return;
+        }
+    }
+    flux_vjp_block<R, false>(p, blockIdx.x - nbblock, bfaces, nbface, lam, ubf, bcbar);
 }
 
 // Geometry cotangents of one residual product lam . R(U) on the face side
@@ -3451,12 +3456,14 @@ int vjp_products_t(ucns_ctx *ctx, const double *lam, double *ubar, double *bcbar
     fp.wt = ctx->wquad + 64;
     fp.bc = ctx->bc;
     tstart(ctx, 1);
-    auto blocks = [&](int faces) { return dim3((unsigned)(((size_t)faces * ctx->nqm + 255) / 256)); };
-    hipLaunchKernelGGL((k_flux_vjp<R, false>), blocks(ctx->nface), dim3(256), 0, ctx->stream, fp,
-                       (const int32_t *)nullptr, 0, lam, ctx->adj_ubf, bcbar);
+    const int nint = (int)(((size_t)ctx->nface * ctx->nqm + 255) / 256);
+    const int nbblock = (int)(((size_t)ctx->nbface * ctx->nqm * BLANES + 255) / 256);
     if (ctx->nbface)
-        hipLaunchKernelGGL((k_flux_vjp<R, true>), blocks(ctx->nbface), dim3(256), 0, ctx->stream, fp, ctx->bfaces,
-                           ctx->nbface, lam, ctx->adj_ubf, bcbar);
+        hipLaunchKernelGGL((k_flux_vjp<R, true>), dim3(nbblock + nint), dim3(256), 0, ctx->stream, fp, ctx->bfaces,
+                           ctx->nbface, nbblock, lam, ctx->adj_ubf, bcbar);
+    else
+        hipLaunchKernelGGL((k_flux_vjp<R, false>), dim3(nint), dim3(256), 0, ctx->stream, fp,
+                           (const int32_t *)nullptr, 0, 0, lam, ctx->adj_ubf, bcbar);
     tstop(ctx, 1);
     tcollect(ctx, 1, &ctx->st.ms_flux_vjp, &ctx->st.n_flux_vjp);
     if constexpr (sizeof(R) == 8) {
