@@ -71,18 +71,19 @@ def recon_bytes_per_cell(case, precision: int) -> float:
 
 
 def recon_kernel_name(case, precision: int) -> str:
-    """the reconstruction kernel the library launches: the row-stream
-    kernels for 5 or 7 stencils (tetrahedra, hexahedra), the
-    register-prefetch ones for other stencil counts"""
+    """the reconstruction kernel the library launches: the row-stream kernels for
+    WENO-4 with 5 or 7 stencils (tetrahedra, hexahedra) and WENO-3 with 5 to 7,
+    the register-prefetch ones for other stencil counts"""
     ts = int(case.array("admis").max())
     nv = (case.array("face_nodes").reshape(case.ncell, -1, 4) >= 0).sum(2)
     nf = int((nv > 0).sum(1).max())
     nqm = max(case.qp_quad if (nv == 4).any() else 0, case.qp_tri if (nv == 3).any() else 0)
     nfq = nf * nqm
-    if case.ideg == 34:  # WENO-5: the per-cell kernel (CWENO: its compact-layout variant)
+    if case.ideg == 34:  # WENO-5: the per-cell kernel (CWENO: a block of waves per tile)
         r = "float" if precision else "double"
-        return f"k_recon<{r},34,69,7{',true,9,19' if case.spec.ees == 5 else ''}>"
-    stream = ((ts == 5 and nfq <= 24) or (ts == 7 and nfq > 24)) if case.ideg == 19 else (ts in (5, 7) and nfq <= 24)
+        occ = 5 if precision and case.ncell > 8 * 768 else 4
+        return f"k_recon_cweno5<{r},{occ}>" if case.spec.ees == 5 else f"k_recon<{r},34,69,7>"
+    stream = ((ts == 5 and nfq <= 24) or (ts == 7 and nfq > 24)) if case.ideg == 19 else (5 <= ts <= 7 and nfq <= 24)
     nql = 3 if nfq <= 24 else 7
     if stream:
         return f"k_recon_{'s32' if precision else 's64'}<{case.ideg},{case.imax},{nql},{ts}>"

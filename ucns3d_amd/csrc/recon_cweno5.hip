@@ -32,8 +32,9 @@ constexpr int NW = 5, NT = NW * WAVE;
 constexpr int GC = ID * NV, GSEC = ID2 * NV;  // coefficients of a central, of a sector polynomial
 static_assert(8 * ID <= NT, "a thread per (coefficient, cell)");
 
-template <typename R>
-__global__ __launch_bounds__(NT, 4) void k_recon_cweno5(Cweno5Params<R> p) {
+// OCC: waves per SIMD
+template <typename R, int OCC>
+__global__ __launch_bounds__(NT, OCC) void k_recon_cweno5(Cweno5Params<R> p) {
     // members' differences (central, then half of the sectors' at a time),
     // then the sectors' coefficients [c][6][45]: three blocks a CU in FP64
     constexpr int HJ = (IM2 + 1) / 2;
@@ -451,7 +452,16 @@ __global__ void k_cweno5_rows(const double *src, R *dst, int cell0, int cn, int 
 
 template <typename R>
 void launch(const Cweno5Params<R> &p, hipStream_t stream) {
-    hipLaunchKernelGGL(k_recon_cweno5<R>, dim3(p.tiles_per_xcd * NXCD), dim3(NT), 0, stream, p);
+    const dim3 grid(p.tiles_per_xcd * NXCD), block(NT);
+    // At 4 waves per SIMD three blocks fit a CU (in FP64 the LDS holds no more).
+    // The mixed kernel fits a fourth at 5, with 116 bytes of scratch a lane: worth
+    // it once the chip's 768 blocks are taken.  Blast box in mixed precision, 2
+    // steps: 307 tiles 0.385 ms with 4 waves and 0.412 with 5, 1,370 tiles 1.18
+    // and 0.98, 3,030 tiles 2.24 and 1.79; 6 waves (188 bytes) 1.82.
+    if (sizeof(R) == 4 && p.ntile > 3 * 256)
+        hipLaunchKernelGGL((k_recon_cweno5<R, sizeof(R) == 4 ? 5 : 4>), grid, block, 0, stream, p);
+    else
+        hipLaunchKernelGGL((k_recon_cweno5<R, 4>), grid, block, 0, stream, p);
 }
 template <typename R>
 void rows(const double *src, R *dst, int cell0, int cn, int tsa, hipStream_t stream) {
