@@ -1,20 +1,24 @@
 // libucnsgpu.so -- MI355X (gfx950) residual + SSP-RK3 path behind include/ucns.h.
 //
 // Per RK stage three kernels run on the library stream:
-//   k_recon   one wavefront per cell: stencil LSQ contraction (P_s dU_s),
-//             smoothness indicators and WENO weights, the weighted
-//             polynomial at every face Gauss point, CHECKSOL -> MUSCL/Barth
-//             -> CHECKSOLX, ULEFT written once per cell
-//             (ARBITRARY_ORDER, src/reconstruct_p.f90:2954-3015)
-//   k_flux    one thread per unique face: rotate, HLLC, rotate back at each
-//             Gauss point; the area-weighted sum is written once per face
+//   reconstruction  stencil LSQ contraction (P_s dU_s), smoothness indicators
+//             and WENO weights, the weighted polynomial at every face Gauss
+//             point, CHECKSOL -> MUSCL/Barth -> CHECKSOLX, ULEFT written once
+//             per cell (ARBITRARY_ORDER, src/reconstruct_p.f90:2954-3015):
+//             recon_tiled.hip (a wave per tile of 8 cells), recon_block.hip
+//             and recon_cweno5.hip (a block of waves per tile),
+//             recon_muscl.hip (8 lanes per cell), k_recon here (a wave per cell)
+//   fluxes    per unique face: rotate, HLLC, rotate back at each Gauss point;
+//             the area-weighted sum is written once per face
 //             (CALCULATE_FLUXESHI_CONVECTIVE, src/flux_p.f90:478-1030, which
 //             solves every face twice; here each face is solved once and
-//             scattered atomic-free by the gather below)
+//             scattered atomic-free by the gather below): k_flux_points, or
+//             k_flux where faces have one point
 //   k_update  one thread per cell: RHS = signed sum of its faces' fluxes, the
 //             Shu-Osher stage update (RUNGE_KUTTA3, src/time_p.f90:885-1027),
 //             and after the last stage the next dt as a min-reduction
 //             (CALCULATE_CFL, src/time_p.f90:27-116)
+// Small meshes of one-point faces run fluxes and update as one (k_flux_update).
 // Device layouts are chosen for coalescing and differ from the ABI layouts;
 // ucns_upload_prestore converts.  FP64 everywhere in UCNS_FP64; in UCNS_MIXED
 // the stencil matrices, indicators, Gauss points, reconstruction, weights and
@@ -3028,9 +3032,11 @@ void launch_flux_t(ucns_ctx *ctx) {
     // A thread per point where faces have several: 5,184 hexahedra faces 18.8 ->
     // 6.2 us, 31,000 channel faces 15.9 -> 9 us; marches on 169,000 (channel) to
     // 393,000 (tetrahedra) faces take the same time within 0.3% either way, on
-    // 69,000 hexahedra in mixed precision 2.66 -> 2.62 ms.  Faces of one point gain
-    // nothing from it (5.7 against 7.9 us on 41,472).
-    if (ctx->nqm > 1) {
+    // 69,000 hexahedra in mixed precision 2.66 -> 2.62 ms.  From a million faces
+    // on, where the face values no longer stay in the caches, a thread per face is
+    // the faster one (1,080,000 channel faces 147 us against 185, mixed 91 against
+    // 136).  Faces of one point gain nothing from it (5.7 against 7.9 us on 41,472).
+    if (ctx->nqm > 1 && ctx->nface < 524288) {
         const int fpb = 256 / ctx->nqm;  // faces per block
         hipLaunchKernelGGL((k_flux_points<R>), dim3((ctx->nface + fpb - 1) / fpb), dim3(256), 0, ctx->stream, p);
     } else {
