@@ -1897,24 +1897,35 @@ __global__ __launch_bounds__(WAVE) void k_recon_vjp(VjpParams<R> p) {
 // scatter.  On the WENO path every step is per variable (indicators and
 // weights are), so a lane holds one variable's column of G_s at a time; B G_s
 // runs over the packed triangle of B once per variable.
+// Bound by latency at two or three waves per SIMD (registers), and by the issue of
+// the face-point pass: with each lane taking a quarter of the coefficients at
+// every other point, the monomials of run-time exponents had been most of its
+// instructions.  Adjoint of 2 steps on 24,576 tetrahedra 3.34 -> 3.13 ms, on
+// 3,375 hexahedra 1.19 -> 1.05 ms, of 3 steps on a 14,000-cell channel 1.76 ->
+// 1.71 ms.
 template <typename R, int IDEG, int NQL, int TS>
-__global__ __launch_bounds__(WAVE) void k_recon_vjp_s(VjpParams<R> p) {
+__global__ __launch_bounds__(WAVE, IDEG == 9 ? 3 : 2) void k_recon_vjp_s(VjpParams<R> p) {
     constexpr int NP = IDEG * (IDEG + 1) / 2;
-    constexpr int KL = (IDEG + 3) / 4;  // coefficients per lane in the face-point pass
-    constexpr int QU = 3;               // face points in flight per lane (and group)
+    constexpr int KL = (IDEG + 7) / 8;  // coefficients per lane in the face-point pass
+    constexpr int BL = (8 * NP + WAVE - 1) / WAVE;
+    // the face-point pass's basis values and cotangents, then the indicators
+    constexpr int PHI = 8 * 8 * IDEG * (int)sizeof(R), PASS = PHI + 8 * 8 * NV * 8, BB = 8 * NP * (int)sizeof(R);
     constexpr int TP = 8 * TS;
     constexpr unsigned KS = NV * TP;    // stride of one coefficient row (elements)
     __shared__ double sGb[8][IDEG * NV];  // cotangent of the combined coefficients
-    __shared__ R sB[8][NP];               // the tile's indicator matrices
+    __shared__ __align__(16) char sRaw[PASS > BB ? PASS : BB];
+    R(*sB)[NP] = (R(*)[NP])sRaw;                      // the tile's indicator matrices
+    R(*sPhi)[8][IDEG] = (R(*)[8][IDEG])sRaw;          // 8 points of each cell: basis values
+    double(*sUb)[8][NV] = (double(*)[8][NV])(sRaw + PHI);  // and cotangents (0 where there is no point)
     const int lane = threadIdx.x, lc = lane >> 3, s = lane & 7;
     const int b = blockIdx.x;
     const int tile = (b % NXCD) * p.tiles_per_xcd + b / NXCD;
     if (tile >= p.ntile) return;
-    {
-        const int nvc = min(8, p.ncell - tile * 8);
-        const R *Bt = p.B + (size_t)tile * 8 * NP;
-        for (int e = lane; e < nvc * NP; e += WAVE) (&sB[0][0])[e] = Bt[e];
-    }
+    // the indicators wait in registers: their LDS serves the face points first
+    R br[BL];
+    const int nB = min(8, p.ncell - tile * 8) * NP;
+#pragma unroll
+    for (int t = 0; t < BL; ++t) br[t] = p.B[(size_t)tile * 8 * NP + min(lane + t * WAVE, nB - 1)];
     const int cell = tile * 8 + lc;
     const bool cvalid = cell < p.ncell;
     const int cs = cvalid ? cell : 0;
@@ -1932,78 +1943,72 @@ __global__ __launch_bounds__(WAVE) void k_recon_vjp_s(VjpParams<R> p) {
     };
 
     // ---- cotangent of the combined coefficients, sum_q phi_q ubar_q, and of
-    // the cell average through a_q = U_i + ULEFT(q).  The 8 lanes of a cell
-    // are two groups of 4: group g takes the face points of parity g, lane i
-    // of a group the coefficients i, i+4, i+8, ...; the groups' sums meet by
-    // one exchange ----
+    // the cell average through a_q = U_i + ULEFT(q), 8 face points of each cell
+    // at a time: lane s evaluates the basis at point s and leaves it in LDS with
+    // the point's cotangent, then takes coefficients s, s+8, s+16 over the eight ----
     double usum[NV] = {0, 0, 0, 0, 0};
     {
-        const int g = s >> 2, il = s & 3;
         double ab[KL][NV];
-        R mk[KL];
-        int ex[KL][3];
 #pragma unroll
-        for (int t = 0; t < KL; ++t) {
-            const int k = il + 4 * t;
-            mk[t] = k < IDEG ? mb[k] : R(0);
-#pragma unroll
-            for (int d = 0; d < 3; ++d) ex[t][d] = k < IDEG ? c_mono[k][d] : 0;
+        for (int t = 0; t < KL; ++t)
 #pragma unroll
             for (int v = 0; v < NV; ++v) ab[t][v] = 0.0;
-        }
+        const int nq8 = p.nf * p.nqm;
+        R x[3];
+        double ub[NV];
+        auto fetch = [&](int q) {  // indices stay in the cell's block
+            const int qc = max(0, min(q, nslot - 1));
+#pragma unroll
+            for (int d = 0; d < 3; ++d) x[d] = qpc[qc * 3 + d];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) ub[v] = ubc[qc * NV + v];
+        };
+        fetch(s);
 #pragma unroll 1
-        for (int q0 = 0; q0 < nslot; q0 += 2 * QU) {
-            // QU points' loads are issued before any is used (indices stay in
-            // the cell's block: q < nslot <= nf nqm)
-            R xq[QU][3];
-            double ub[QU][NV];
+        for (int q0 = 0; q0 < nq8; q0 += 8) {
+            const bool ok = qvalid(q0 + s);
+            {
+                R phi[IDEG];
+                basis_at<R, IDEG>(x, mb, phi);
 #pragma unroll
-            for (int u = 0; u < QU; ++u) {
-                const int q = min(q0 + 2 * u + g, nslot - 1);
-#pragma unroll
-                for (int d = 0; d < 3; ++d) xq[u][d] = qpc[q * 3 + d];
-#pragma unroll
-                for (int v = 0; v < NV; ++v) ub[u][v] = ubc[q * NV + v];
+                for (int k = 0; k < IDEG; ++k) sPhi[lc][s][k] = phi[k];
             }
 #pragma unroll
-            for (int u = 0; u < QU; ++u) {
-                const int q = q0 + 2 * u + g;
-                const bool ok = q < nslot && qvalid(q);
-                const R x0 = xq[u][0], x1 = xq[u][1], x2 = xq[u][2];
-                const R x0s = x0 * x0, x1s = x1 * x1, x2s = x2 * x2;
-                const R x0c = x0s * x0, x1c = x1s * x1, x2c = x2s * x2;
+            for (int v = 0; v < NV; ++v) {
+                const double u = ok ? ub[v] : 0.0;
+                sUb[lc][s][v] = u;
+                usum[v] += u;
+            }
+            fetch(q0 + 8 + s);
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
                 double uv[NV];
 #pragma unroll
-                for (int v = 0; v < NV; ++v) {
-                    uv[v] = ok ? ub[u][v] : 0.0;
-                    usum[v] += uv[v];
-                }
+                for (int v = 0; v < NV; ++v) uv[v] = sUb[lc][u][v];
 #pragma unroll
                 for (int t = 0; t < KL; ++t) {
-                    const double ph = (double)(pw(x0, x0s, x0c, ex[t][0]) * pw(x1, x1s, x1c, ex[t][1]) *
-                                                   pw(x2, x2s, x2c, ex[t][2]) - mk[t]);
+                    const double ph = (double)sPhi[lc][u][min(s + 8 * t, IDEG - 1)];
 #pragma unroll
                     for (int v = 0; v < NV; ++v) ab[t][v] += ph * uv[v];
                 }
             }
+            __syncthreads();
         }
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            usum[v] += __shfl_xor(usum[v], 4, WAVE);
+        for (int v = 0; v < NV; ++v) usum[v] = grp_sum8(usum[v]);
 #pragma unroll
-            for (int t = 0; t < KL; ++t) ab[t][v] += __shfl_xor(ab[t][v], 4, WAVE);
-        }
-        if (g == 0) {
+        for (int t = 0; t < KL; ++t) {
+            const int k = s + 8 * t;
+            if (k < IDEG) {
 #pragma unroll
-            for (int t = 0; t < KL; ++t) {
-                const int k = il + 4 * t;
-                if (k < IDEG) {
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) sGb[lc][k * NV + v] = ab[t][v];
-                }
+                for (int v = 0; v < NV; ++v) sGb[lc][k * NV + v] = ab[t][v];
             }
         }
     }
+#pragma unroll
+    for (int t = 0; t < BL; ++t)
+        if (lane + t * WAVE < nB) sB[0][lane + t * WAVE] = br[t];
     __syncthreads();  // sGb, sB
 
     const bool reduce = cvalid && (fl & 1), first = (fl & 2) != 0;
