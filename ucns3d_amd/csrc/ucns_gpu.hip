@@ -563,6 +563,11 @@ __device__ inline void hllc_t(double gamma, const T *cl, const T *cr, T *flux) {
 // that sign(S_M) picks evaluated (the other is multiplied by 0 there).  The
 // kernels spend most of their vector time in FP64 divisions and square roots:
 // 11 and 5 of them here, 14 and 5 in hllc_t.
+// The other side's terms vanish unless they are not finite: where its wave speed
+// is S_M (a division by S - S_M: every component) or its own normal velocity (by
+// S - u: the energy), which a state without a sound speed (p <= 0) can bring
+// about, hllc_t's 0 times infinity makes the flux NaN.  It does here too, so that
+// such a state still ends a march as non-finite.
 __device__ inline void hllc64(double gamma, const double *cl, const double *cr, double *flux) {
     double wl[NV], wr[NV];
     cons2prim_d(gamma, cl, wl);
@@ -589,6 +594,12 @@ __device__ inline void hllc64(double gamma, const double *cl, const double *cr, 
     const double us[NV] = {mu, mu * sm, mu * wk[2], mu * wk[3], mu * last};
 #pragma unroll
     for (int k = 0; k < NV; ++k) flux[k] = fk[k] + sk * (us[k] - ck[k]);
+    const double so = left ? sr : sl, uo = left ? uR : uL;
+    if (so == sm || so == uo) {
+        flux[4] = (double)NAN;
+#pragma unroll
+        for (int k = 0; k < NV - 1; ++k) flux[k] = so == sm ? (double)NAN : flux[k];
+    }
 }
 
 // Reverse mode of hllc_t (FP64): given the flux cotangent hb, the cotangents
