@@ -5,13 +5,15 @@ both sides of a rule's line.  Against the oracle at the parity bars
 the kernels that the rule leaves (another order of FP64 sums: a few hundred
 roundings of 1.1e-16, held to 1e-12 of the largest value; cotangents behind a
 march to 1e-10)."""
+import dataclasses
+
 import numpy as np
 import pytest
 
 from oracle.oracle import Oracle
 from shuffle import shuffled_structs
-from ucns3d_amd.case import HEX, PRISM, TET, Case, CaseSpec, reduced
-from ucns3d_amd.native import UCNS_FP64, UCNS_KERNELS_REGISTER
+from ucns3d_amd.case import HEX, HYBRID, PRISM, TET, Case, CaseSpec, reduced
+from ucns3d_amd.native import UCNS_FP64, UCNS_KERNELS_REGISTER, UCNS_MIXED
 from ucns3d_amd.solver import Solver, UcnsError
 
 pytestmark = pytest.mark.gpu
@@ -183,3 +185,41 @@ def test_states_without_a_sound_speed(name):
     with pytest.raises(UcnsError, match="non-finite"):
         s.rk3_steps(1, dt_fixed=1e-3)
     s.close()
+
+
+# triangles of a mesh with quadrilaterals leave slots of the face-point array
+# without a point; nothing may depend on what the caller left there
+UNUSED = {
+    "channel-weno3": reduced("c4", 3),
+    "channel-weno3-char": dataclasses.replace(reduced("c4", 3), wenwrt=2),
+    "hybrid-weno3": CaseSpec("u-hybrid", HYBRID, 6, "weno3", jitter=0.1, seed=3),
+    "blast-cweno5": reduced("c5", 10),
+}
+
+
+@pytest.mark.parametrize("precision", [UCNS_FP64, UCNS_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("name", list(UNUSED))
+def test_slots_without_a_face_point(name, precision):
+    spec = UNUSED[name]
+    case = Case(spec)
+    u = case.init_state()
+    w = np.random.default_rng(3).standard_normal(u.shape)
+    q = case.array("qpoints").reshape(case.ncell, case.nface_max, -1, 3)
+    nv = (case.array("face_nodes").reshape(case.ncell, -1, 4) >= 0).sum(2)
+    nq = np.where(nv == 4, case.qp_quad, np.where(nv == 3, case.qp_tri, 0))
+    unused = np.arange(q.shape[2]) >= nq[:, :, None]
+    assert (unused & (nq > 0)[:, :, None]).any()
+    out = []
+    for fill in (0.0, np.nan):
+        q[unused] = fill
+        print(f"[unused slots] {name} ncell={case.ncell} precision={precision} fill={fill}", flush=True)
+        s = Solver(case, precision)
+        fs = spec.freestream() if spec.mach > 0 else np.array([1.0, 0.0, 0.0, 0.0, 2.5])
+        s.set_boundary(1 if spec.mach > 0 else 0, fs, fs)
+        s.set_state(u)
+        r = s.residual()
+        out.append((r, None if spec.wenwrt == 2 or spec.ees == 5 else s.residual_vjp(w)[0]))
+        s.close()
+    assert np.isfinite(out[0][0]).all() and np.array_equal(out[0][0], out[1][0])
+    if out[0][1] is not None:  # sums of atomics: another order on every run
+        close(out[1][1], out[0][1], 1e-12)

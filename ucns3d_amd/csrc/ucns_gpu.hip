@@ -1979,8 +1979,10 @@ __global__ __launch_bounds__(WAVE, IDEG == 9 ? 3 : 2) void k_recon_vjp_s(VjpPara
         for (int q0 = 0; q0 < nq8; q0 += 8) {
             const bool ok = qvalid(q0 + s);
             {
+                // a slot without a point holds whatever the caller left there
+                const R xp[3] = {ok ? x[0] : R(0), ok ? x[1] : R(0), ok ? x[2] : R(0)};
                 R phi[IDEG];
-                basis_at<R, IDEG>(x, mb, phi);
+                basis_at<R, IDEG>(xp, mb, phi);
 #pragma unroll
                 for (int k = 0; k < IDEG; ++k) sPhi[lc][s][k] = phi[k];
             }
