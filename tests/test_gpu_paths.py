@@ -5,6 +5,7 @@ both sides of a rule's line.  Against the oracle at the parity bars
 the kernels that the rule leaves (another order of FP64 sums: a few hundred
 roundings of 1.1e-16, held to 1e-12 of the largest value; cotangents behind a
 march to 1e-10)."""
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -223,3 +224,30 @@ def test_slots_without_a_face_point(name, precision):
     assert np.isfinite(out[0][0]).all() and np.array_equal(out[0][0], out[1][0])
     if out[0][1] is not None:  # sums of atomics: another order on every run
         close(out[1][1], out[0][1], 1e-12)
+
+
+# iweno 1 with the linear polynomial of the central stencil: one stencil, so a
+# weight of 1 whatever the indicator, and the limiter only where CHECKSOL asks
+@pytest.mark.parametrize("precision,tol", [(UCNS_FP64, 1e-11), (UCNS_MIXED, 1e-5)], ids=["fp64", "mixed"])
+def test_linear_weno(precision, tol):
+    case = Case(CaseSpec("l-weno", HEX, 5, "muscl", jitter=0.1, seed=3))
+    mesh, scheme, pre = structs = case.structs(precision)
+    scheme.iweno = 1
+    ind = np.tile(np.eye(3), (case.ncell, 1, 1))
+    full = (np.arange(case.ncell) % 3 > 0).astype(np.int32)
+    pre.indicator = ind.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+    pre.full = full.ctypes.data_as(ctypes.POINTER(ctypes.c_int32))
+    u = case.init_state()
+    orc = Oracle(case)
+    orc.m, orc.s, orc.p = structs
+    r_ref, cnt = orc.residual(u)
+    print(f"[linear WENO] ncell={case.ncell} precision={precision}", flush=True)
+    s = Solver(case, precision, structs=structs)
+    s.set_state(u)
+    err = rel_l2(s.residual(), r_ref)
+    st = s.stats()
+    s.close()
+    print("  residual", err, "MUSCL cells", cnt[0])
+    assert 0 < cnt[0] < case.ncell
+    assert (st["n_reduced_last"], st["n_firstorder_last"]) == (cnt[0], cnt[1])
+    assert np.all(err <= tol), err

@@ -74,8 +74,9 @@ struct ReconShared {
     double ui[NV];
 };
 
-// Fused reconstruction, one wavefront per cell: WENO-5, and shapes and face
-// rules the tiled kernels do not hold.
+// Fused reconstruction, one wavefront per cell: WENO-5, the linear central
+// polynomial without the limiter (iweno 1, idegfree 3), and shapes and face rules
+// the tiled kernels do not hold.
 // CH: characteristic-variable WENO, face by face (src/reconstruct_p.f90:497-758).
 template <typename R, int IDEG, int IMAX, int TSMAX, bool CH = false>
 __global__ __launch_bounds__(WAVE) void k_recon(ReconParams<R> p) {
@@ -3013,6 +3014,8 @@ int launch_recon_t(ucns_ctx *ctx, bool packed = false) {
         hipLaunchKernelGGL((k_recon<R, 34, 69, 7>), grid, block, 0, ctx->stream, p);
     else if (ctx->ideg == 9 && ctx->imax == 19)
         hipLaunchKernelGGL((k_recon<R, 9, 19, 7>), grid, block, 0, ctx->stream, p);
+    else if (ctx->ideg == 3 && ctx->imax == 8 && ctx->ts == 1)  // linear, unlimited where CHECKSOL lets it
+        hipLaunchKernelGGL((k_recon<R, 3, 8, 1>), grid, block, 0, ctx->stream, p);
     else {
         ctx->err = "no reconstruction kernel for idegfree=" + std::to_string(ctx->ideg) +
                    " imax=" + std::to_string(ctx->imax);
