@@ -251,3 +251,71 @@ def test_linear_weno(precision, tol):
     assert 0 < cnt[0] < case.ncell
     assert (st["n_reduced_last"], st["n_firstorder_last"]) == (cnt[0], cnt[1])
     assert np.all(err <= tol), err
+
+
+# The geometry product forms the stencil coefficients again: it neither stores
+# nor keeps the row stream's, so a march keeps as many stages as on the register
+# kernels, and holds no more device memory
+def test_geometry_product_keeps_no_coefficients():
+    import torch
+    spec = reduced("c4", 9)
+    case = Case(spec)
+    steps, fs = 3, spec.freestream()
+    nv = (case.array("face_nodes").reshape(case.ncell, -1, 4) >= 0).sum(2)
+    face_values = case.ncell * int((nv > 0).sum(1).max()) * max(case.qp_quad, case.qp_tri) * 5 * 8
+    gib = 1.01 * 3 * steps * face_values / 2.0 ** 30  # every stage's, and nothing beside them
+    w = np.random.default_rng(3).standard_normal((case.ncell, 5))
+    u = case.init_state()
+
+    def context(**kw):
+        s = Solver(case, UCNS_FP64, adj_keep_gib=gib, **kw)
+        s.set_boundary(1, fs, fs)
+        s.set_state(u)
+        s.reset_stats()
+        return s
+
+    out = []
+    for kw in ({"kernels": UCNS_KERNELS_REGISTER}, {}):
+        print(f"[geometry product, kept stages] ncell={case.ncell} {kw}", flush=True)
+        s = context(**kw)
+        free = torch.cuda.mem_get_info()[0]
+        g = s.rk3_adjoint_geometry(steps, w, 1e-3)[0]
+        out.append((g, s.stats()["n_recon_adj"], free - torch.cuda.mem_get_info()[0]))
+        s.close()
+    (g_reg, again_reg, mem_reg), (g_row, again_row, mem_row) = out
+    print("  stages reconstructed again", again_reg, again_row, "bytes held", mem_reg, mem_row)
+    assert again_reg == 0 and again_row == 0
+    assert mem_row <= mem_reg + (8 << 20)  # allocations come in 2 MiB pieces
+    close(g_row, g_reg, 1e-10)
+
+
+# products that store and geometry products in turn, in one context whose budget
+# holds only some stages of the first kind
+def test_geometry_and_ordinary_adjoints_in_turn():
+    spec = reduced("c4", 6)
+    case = Case(spec)
+    fs = spec.freestream()
+    w = np.random.default_rng(3).standard_normal((case.ncell, 5))
+    u = case.init_state()
+
+    def call(s, kind):
+        s.set_state(u)
+        return (s.rk3_adjoint_geometry(2, w, 1e-3) if kind == "geometry" else s.rk3_adjoint(2, w, dt_fixed=1e-3))[0]
+
+    def context(gib):
+        s = Solver(case, UCNS_FP64, adj_keep_gib=gib)
+        s.set_boundary(1, fs, fs)
+        return s
+
+    ref = {}
+    for kind in ("geometry", "ordinary"):
+        s = context(0.0)
+        ref[kind] = call(s, kind)
+        s.close()
+    for order in (("ordinary", "geometry", "ordinary"), ("geometry", "ordinary", "geometry", "geometry")):
+        for gib in (0.02, 0.05, 1.0):
+            print(f"[adjoints in turn] ncell={case.ncell} {order} {gib} GiB", flush=True)
+            s = context(gib)
+            for kind in order:
+                close(call(s, kind), ref[kind], 1e-10)
+            s.close()

@@ -2766,8 +2766,8 @@ struct ucns_ctx {
     int fail_alloc_in = 0;   // > 0: the fail_alloc_in-th device allocation from now fails (ucns_debug_fail_alloc)
     size_t ckpt_steps = 0;
     // the last stages of a march keep their forward reconstruction for the
-    // reverse sweep: face values, and in row-stream mode the stencil
-    // coefficients, indicators, weights (as adj_g) and flags
+    // reverse sweep: face values, and where the product reads them (adj_stores)
+    // the stencil coefficients, indicators, weights (as adj_g) and flags
     std::vector<void *> keep_ul, keep_g;
     std::vector<int *> keep_f;
     // geometry cotangents of ucns_rk3_adjoint_geometry (device, FP64, live
@@ -3304,6 +3304,26 @@ struct DevTemp {
     ~DevTemp() { dfree(p); }
 };
 
+// whether the residual product reads what the forward reconstruction stored
+// (k_recon_vjp_s); the geometry product (k_recon_vjp) forms it again
+bool adj_stores(const ucns_ctx *ctx) { return ctx->smode && !ctx->geo_on; }
+
+// elements of adj_g: the coefficients, indicators and weights of every stencil
+size_t adj_g_elems(const ucns_ctx *ctx) { return (size_t)ctx->ntile * (ctx->ideg + 2) * NV * 8 * ctx->ts; }
+
+// the stored forward of one stage, and the coefficients' cotangents
+int ensure_stored(ucns_ctx *ctx) {
+    if (ctx->adj_gb) return UCNS_OK;
+    int rc;
+    if ((rc = dalloc(ctx, &ctx->adj_flags, (size_t)ctx->ncell))) return rc;
+    if (ctx->precision == UCNS_MIXED)
+        rc = dalloc(ctx, (float **)&ctx->adj_g, adj_g_elems(ctx));
+    else
+        rc = dalloc(ctx, (double **)&ctx->adj_g, adj_g_elems(ctx));
+    if (rc) return rc;
+    return dalloc(ctx, &ctx->adj_gb, (size_t)ctx->ntile * ctx->ideg * NV * 8 * ctx->ts);
+}
+
 int ensure_adjoint_steps(ucns_ctx *ctx) {
     const size_t n = (size_t)ctx->ncell * NV;
     int rc;
@@ -3314,18 +3334,6 @@ int ensure_adjoint_steps(ucns_ctx *ctx) {
     if ((rc = dalloc(ctx, &ctx->adj_a, n))) return rc;
     if ((rc = dalloc(ctx, &ctx->adj_u0, n))) return rc;
     if ((rc = dalloc(ctx, &ctx->adj_bc, 2 * NV))) return rc;
-    if (ctx->smode) {
-        const size_t ng = (size_t)ctx->ntile * (ctx->ideg + 2) * NV * 8 * ctx->ts;
-        if ((rc = dalloc(ctx, &ctx->adj_flags, (size_t)ctx->ncell))) return rc;
-        if (ctx->precision == UCNS_MIXED)
-            rc = dalloc(ctx, (float **)&ctx->adj_g, ng);
-        else
-            rc = dalloc(ctx, (double **)&ctx->adj_g, ng);
-        if (rc) return rc;
-    }
-    if (ctx->smode) {
-        if ((rc = dalloc(ctx, &ctx->adj_gb, (size_t)ctx->ntile * ctx->ideg * NV * 8 * ctx->ts))) return rc;
-    }
     // the tiles' distinct stencil members (once per upload)
     if (ctx->ts <= 8 && (ctx->imax == 39 || ctx->imax == 19 || ctx->imax == 8)) {
         if ((rc = ensure_members(ctx))) return rc;
@@ -3397,9 +3405,12 @@ int ensure_adjoint(ucns_ctx *ctx) {
         ctx->err = "the adjoint takes uniform boundary states (ucns_set_boundary), not per-face ones";
         return UCNS_EUNSUPPORTED;
     }
-    if (ctx->adj_ready) return UCNS_OK;
-    release_adjoint(ctx);
-    const int rc = ensure_adjoint_steps(ctx);
+    int rc = UCNS_OK;
+    if (!ctx->adj_ready) {
+        release_adjoint(ctx);
+        rc = ensure_adjoint_steps(ctx);
+    }
+    if (rc == UCNS_OK && adj_stores(ctx)) rc = ensure_stored(ctx);
     if (rc != UCNS_OK) {
         release_adjoint(ctx);
         return rc;
@@ -3445,7 +3456,7 @@ void launch_scatter_t(ucns_ctx *ctx, double *ubar) {
 // weights and the cell flags
 template <typename R>
 int vjp_recon_t(ucns_ctx *ctx) {
-    ctx->adj_g_on = ctx->smode && ctx->adj_g;
+    ctx->adj_g_on = adj_stores(ctx);
     tstart(ctx, 3);
     const int rc = launch_recon_t<R>(ctx);
     tstop(ctx, 3);
@@ -3523,13 +3534,13 @@ int vjp_products_t(ucns_ctx *ctx, const double *lam, double *ubar, double *bcbar
     vp.cnb = ctx->cnb;
     vp.ubf = ctx->adj_ubf;
     vp.ubar = ubar;
-    vp.gload = (ctx->smode && ctx->adj_g) ? (const R *)ctx->adj_g : nullptr;
+    vp.gload = adj_stores(ctx) ? (const R *)ctx->adj_g : nullptr;
     vp.fload = ctx->adj_flags;
     vp.slot = ctx->mem_slot;
     vp.uq_cap = ctx->uq_cap;
     vp.uq = ctx->mem_uq;
     vp.ucount = ctx->mem_count;
-    vp.gbout = ctx->smode ? ctx->adj_gb : nullptr;
+    vp.gbout = adj_stores(ctx) ? ctx->adj_gb : nullptr;
     vp.toff = ctx->adj_toff;
     vp.tab = ctx->adj_tab;
     vp.gP = ctx->geo_P;
@@ -3630,50 +3641,67 @@ int residual_vjp_dev(ucns_ctx *ctx, const double *lam, double *ubar, double *bcb
 // most nstage): the scheme's adj_keep_stages caps the count (0: no cap,
 // < 0: none), adj_keep_gib the bytes (never more than the free device memory
 // less 4 GiB).
-// Buffers only grow; a failed allocation leaves the count at what was had.
+// A failed allocation leaves the count at what was had.
 int adj_keep(ucns_ctx *ctx, int nstage) {
     const size_t esz = ctx->precision == UCNS_MIXED ? 4 : 8;
+    const bool st = adj_stores(ctx);
     const size_t ul = (size_t)ctx->ncell * ctx->nf * ctx->nqm * NV * esz;
-    const size_t g = ctx->smode ? (size_t)ctx->ntile * (ctx->ideg + 2) * NV * 8 * ctx->ts * esz : 0;
-    const size_t fl = ctx->smode ? (size_t)ctx->ncell * sizeof(int) : 0;
-    const size_t per = ul + g + fl;
+    const size_t g = adj_g_elems(ctx) * esz, fl = (size_t)ctx->ncell * sizeof(int);
+    const size_t per = ul + (st ? g + fl : 0);
+    auto held = [&](size_t nul, size_t ng) { return nul * ul + ng * (g + fl); };
     long want = nstage;
     if (ctx->adj_keep_stages < 0) return 0;
     if (ctx->adj_keep_stages > 0) want = std::min<long>(want, ctx->adj_keep_stages);
     size_t budget = (size_t)(ctx->adj_keep_gib * (double)(1ull << 30));
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) == hipSuccess) {
-        const size_t have = fr + ctx->keep_ul.size() * per, margin = 4ull << 30;
+        const size_t have = fr + held(ctx->keep_ul.size(), ctx->keep_g.size()), margin = 4ull << 30;
         budget = std::min(budget, have > margin ? have - margin : 0);
     }
     want = std::min<long>(want, (long)(budget / per));
-    while ((long)ctx->keep_ul.size() < want) {
-        void *a = nullptr, *b = nullptr;
-        int *c = nullptr;
-        if (hipMalloc(&a, ul) != hipSuccess) break;
-        if (ctx->smode && (hipMalloc(&b, g) != hipSuccess || hipMalloc((void **)&c, fl) != hipSuccess)) {
-            (void)hipFree(a);
-            if (b) (void)hipFree(b);
-            break;
+    // calls that store and geometry calls share the face values: what one of them
+    // holds beyond the other's budget is given back
+    const size_t n = (size_t)want;
+    if (held(std::max(ctx->keep_ul.size(), n), st ? std::max(ctx->keep_g.size(), n) : ctx->keep_g.size()) > budget) {
+        for (; ctx->keep_ul.size() > n; ctx->keep_ul.pop_back()) (void)hipFree(ctx->keep_ul.back());
+        for (; ctx->keep_g.size() > (st ? n : 0); ctx->keep_g.pop_back(), ctx->keep_f.pop_back()) {
+            (void)hipFree(ctx->keep_g.back());
+            (void)hipFree(ctx->keep_f.back());
         }
-        ctx->keep_ul.push_back(a);
-        ctx->keep_g.push_back(b);
-        ctx->keep_f.push_back(c);
+    }
+    size_t got = 0;  // stages in place
+    for (; got < n; ++got) {
+        if (ctx->keep_ul.size() == got) {
+            void *a = nullptr;
+            if (hipMalloc(&a, ul) != hipSuccess) break;
+            ctx->keep_ul.push_back(a);
+        }
+        if (st && ctx->keep_g.size() == got) {
+            void *b = nullptr;
+            int *c = nullptr;
+            if (hipMalloc(&b, g) != hipSuccess) break;
+            if (hipMalloc((void **)&c, fl) != hipSuccess) {
+                (void)hipFree(b);
+                break;
+            }
+            ctx->keep_g.push_back(b);
+            ctx->keep_f.push_back(c);
+        }
     }
     (void)hipGetLastError();  // a refused allocation only lowers the count
-    return (int)std::min<long>(want, (long)ctx->keep_ul.size());
+    return (int)got;
 }
 
 // Point the reconstruction's outputs (face values; stencil coefficients and
-// flags in row-stream mode) at kept stage b, and back to the context's own
-// buffers on destruction.
+// flags where the product reads them) at kept stage b, and back to the context's
+// own buffers on destruction.
 struct KeptStage {
     ucns_ctx *ctx;
     void *ul, *g;
     int *f;
     KeptStage(ucns_ctx *c, int b) : ctx(c), ul(c->uleft), g(c->adj_g), f(c->adj_flags) {
         ctx->uleft = ctx->keep_ul[b];
-        if (ctx->smode) {
+        if (adj_stores(c)) {
             ctx->adj_g = ctx->keep_g[b];
             ctx->adj_flags = ctx->keep_f[b];
         }
@@ -3698,7 +3726,7 @@ int rk3_step_ckpt(ucns_ctx *ctx, int it, int nsteps, const double *dt, unsigned 
         int rc;
         if (q >= keep0) {
             KeptStage k(ctx, q - keep0);
-            ctx->adj_g_on = ctx->smode != 0;
+            ctx->adj_g_on = adj_stores(ctx);
             rc = residual_kernels(ctx, q > 0);
             ctx->adj_g_on = false;
         } else {
@@ -5144,17 +5172,20 @@ int ucns_rk3_adjoint_geometry(ucns_ctx *ctx, int32_t nsteps, double dt_fixed, co
         return UCNS_EUNSUPPORTED;
     }
     HIP_TRY(hipSetDevice(ctx->device));
+    // from here on every product is the geometry product; its arrays go with the call
+    struct Scope {
+        ucns_ctx *ctx;
+        explicit Scope(ucns_ctx *c) : ctx(c) { c->geo_on = true; }
+        ~Scope() { release_geometry(ctx); }
+    } scope(ctx);
     if ((rc = ensure_adjoint(ctx))) return rc;
     const size_t nc = ctx->ncell;
-    release_geometry(ctx);
     if ((rc = dalloc(ctx, &ctx->geo_P, nc * ctx->ts * ctx->imax * ctx->ideg)) ||
         (rc = dalloc(ctx, &ctx->geo_B, nc * ctx->ideg * ctx->ideg)) || (rc = dalloc(ctx, &ctx->geo_M, nc * ctx->ideg)) ||
         (rc = dalloc(ctx, &ctx->geo_Q, nc * ctx->nf * ctx->nqm * 3)) ||
         (rc = dalloc(ctx, &ctx->geo_area, (size_t)ctx->nface)) ||
-        (rc = dalloc(ctx, &ctx->geo_nrm, (size_t)ctx->nface * 3)) || (rc = dalloc(ctx, &ctx->geo_ovol, nc))) {
-        release_geometry(ctx);
+        (rc = dalloc(ctx, &ctx->geo_nrm, (size_t)ctx->nface * 3)) || (rc = dalloc(ctx, &ctx->geo_ovol, nc)))
         return rc;
-    }
     zero_dev(ctx, ctx->geo_P, nc * ctx->ts * ctx->imax * ctx->ideg);
     zero_dev(ctx, ctx->geo_B, nc * ctx->ideg * ctx->ideg);
     zero_dev(ctx, ctx->geo_M, nc * ctx->ideg);
@@ -5162,17 +5193,13 @@ int ucns_rk3_adjoint_geometry(ucns_ctx *ctx, int32_t nsteps, double dt_fixed, co
     zero_dev(ctx, ctx->geo_area, (size_t)ctx->nface);
     zero_dev(ctx, ctx->geo_nrm, (size_t)ctx->nface * 3);
     zero_dev(ctx, ctx->geo_ovol, nc);
-    if ((rc = cells_in(ctx, uN_bar, true, layout, ctx->adj_a)) == UCNS_OK) {
-        ctx->geo_on = true;
+    if ((rc = cells_in(ctx, uN_bar, true, layout, ctx->adj_a)) == UCNS_OK)
         rc = rk3_adjoint_impl(ctx, nsteps, 0.0, dt_fixed, ctx->adj_a, t_io);
-        ctx->geo_on = false;
-    }
     double bc[2 * NV];
     if (rc == UCNS_OK && hipMemcpyAsync(bc, ctx->adj_bc, sizeof(bc), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess)
         rc = UCNS_EHIP;
     if (rc == UCNS_OK) rc = cells_out(ctx, ctx->adj_a, layout, u0_bar, true);
     if (rc == UCNS_OK) rc = geo_to_caller(ctx, gbar);
-    release_geometry(ctx);
     if (rc == UCNS_EHIP && ctx->err.empty()) ctx->err = "ucns_rk3_adjoint_geometry: HIP error";
     if (rc) return rc;
     if (bc_bar) std::memcpy(bc_bar, bc, sizeof(bc));
