@@ -319,3 +319,34 @@ def test_geometry_and_ordinary_adjoints_in_turn():
             for kind in order:
                 close(call(s, kind), ref[kind], 1e-10)
             s.close()
+
+
+# The rule for the block kernels in conserved variables: at most 512 tiles (768 in
+# mixed precision), and no tile past the member table.  A context on them builds
+# the member tables (three allocations) at its upload, one on the row stream with
+# its first adjoint
+@pytest.mark.parametrize("precision,n,shuffled,block", [
+    (UCNS_FP64, 15, False, True), (UCNS_FP64, 15, True, False), (UCNS_FP64, 16, False, True),
+    (UCNS_FP64, 17, False, False), (UCNS_MIXED, 17, False, True), (UCNS_MIXED, 17, True, False),
+    (UCNS_MIXED, 19, False, False)])
+def test_rule_of_the_block_kernels(precision, n, shuffled, block):
+    case = Case(CaseSpec("b-hex4", HEX, n, "weno4", jitter=0.1, seed=5))
+    u = case.init_state()
+    w = np.random.default_rng(6).standard_normal(u.shape)
+    sh = np.random.default_rng(4).permutation(case.ncell) if shuffled else np.arange(case.ncell)
+    keep, st = shuffled_structs(case, sh.astype(np.int64), precision)
+    print(f"[block rule] ncell={case.ncell} precision={precision} shuffled={shuffled}", flush=True)
+    s = Solver(case, precision, structs=st)
+    s.set_state(u[sh])
+    made = 0
+    while True:  # one allocation more on every try, until the set-up succeeds
+        s.debug_fail_alloc(made + 1)
+        try:
+            s.residual_vjp(w[sh])
+            break
+        except UcnsError as e:
+            assert "injected" in str(e)
+            made += 1
+    s.close()
+    # 7 work arrays, the 3 of the stored forward, 5 of the tables' index by cell
+    assert made == (15 if block else 18), made

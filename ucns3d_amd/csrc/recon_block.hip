@@ -3,8 +3,8 @@
 // (src/gradients.f90:253-497, src/reconstruct_p.f90:497-758, 920-1199,
 // 2044-2280, 3126-3406).
 //
-// A wave per tile (ucns_tiled.h) streams at the card's rate once a thousand and
-// more tiles are in flight, but a tile's rows, and the phases behind them, run
+// A wave per tile (ucns_tiled.h) streams at the card's rate once some thousand
+// tiles are in flight, but a tile's rows, and the phases behind them, run
 // one after the other in it.  Here they spread over four waves:
 //   - a wave takes IDEG / NW of the coefficients of all 8 TS (cell, stencil)
 //     columns (lane = column), so two or three blocks fit a CU;
@@ -20,7 +20,8 @@
 // WENO-4, 1,728 hexahedra (216 tiles): 47 us with a wave per tile, 31 us this
 // way; 3,072 tiles of tetrahedra 216 and 218 us; 24,576 tiles 1389 and 1518 us
 // (the four waves' index reads, LDS gathers and barriers), so the wave per tile
-// keeps the large meshes.
+// keeps the larger meshes (the line, and its measurements, are in
+// ucns_upload_prestore).
 #include "ucns_recon.h"
 
 namespace ucns {

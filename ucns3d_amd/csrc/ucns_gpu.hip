@@ -4399,10 +4399,17 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
         ctx->smode = stream_ok ? ts : 0;
     }
     ctx->ntile = (nc + 7) / 8;
-    // WENO-4 of at most 1,024 tiles, one per SIMD of the chip: there a wave per
-    // tile leaves SIMDs idle and its chain of rows bare (216 tiles 47 us against
-    // 31; at 3,072 tiles both take 217 us)
-    ctx->bmode = ctx->tiled && wide && (ctx->wenwrt == 2 || (ctx->smode && ID == 19 && ctx->ntile <= 1024));
+    // WENO-4 of few tiles: there a wave per tile leaves SIMDs idle and its chain of
+    // rows bare.  The line is where the blocks no longer all run at once (two a CU
+    // in FP64 on hexahedra).  A march's stage in us, row stream and block kernels:
+    //   FP64   hexahedra    216 tiles 55.6, 39.4;  512 61.1, 58.9;  615 74.5, 83.2;  1,000 95.4, 111.5
+    //          tetrahedra   162 45.8, 31.3;        384 47.5, 42.0;  547 51.3, 53.1;    999 68.4, 77.1
+    //   mixed  hexahedra    216 45.4, 32.8;        512 49.4, 43.1;  729 54.5, 55.5;    858 62.4, 64.3
+    //          tetrahedra   162 39.3, 27.4;        384 40.2, 31.2;  750 42.8, 39.9;    999 46.4, 47.1
+    // (a mesh of hexahedra, pyramids and prisms in FP64, 648 tiles: 84.0, 81.1; the
+    // member tables have a say in it below)
+    ctx->bmode = ctx->tiled && wide &&
+                 (ctx->wenwrt == 2 || (ctx->smode && ID == 19 && ctx->ntile <= (mixed ? 768 : 512)));
     ctx->nmark = ctx->tiled || ctx->cw_cell || ctx->iweno == -1 ? ctx->ntile : nc;
     int rc = dalloc(ctx, &ctx->marks, (size_t)ctx->nmark);
     if (rc) return rc;
@@ -4653,6 +4660,23 @@ int ucns_upload_prestore(ucns_ctx *ctx, const ucns_prestore_v1 *pre) {
         if ((rc = upload_real_any(ctx, &ctx->qp, q))) return rc;
     }
     if (ctx->bmode && (rc = ensure_members(ctx))) return rc;
+    if (ctx->bmode && ctx->wenwrt == 1) {
+        // A tile with more distinct members than the table in LDS holds (cells in
+        // an order without locality) has no rows in flight in the block kernel,
+        // and one such tile holds the launch up: 3,375 shuffled hexahedra in FP64
+        // take 88.6 us a stage on it, 61.7 on the row stream, which gathers every
+        // member and does not care (mixed 75.0 and 50.1).  The characteristic
+        // kernel has no such stand-in and stays (2,058 shuffled tetrahedra 72 us,
+        // 136 with one wave per cell).
+        std::vector<int32_t> uc(ctx->ntile);
+        HIP_TRY(hipMemcpyAsync(uc.data(), ctx->mem_count, uc.size() * sizeof(int32_t), hipMemcpyDeviceToHost,
+                               ctx->stream));
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        if (*std::max_element(uc.begin(), uc.end()) > ctx->uq_cap) {
+            ctx->bmode = false;
+            release_members(ctx);
+        }
+    }
     ctx->have_prestore = true;
     ctx->st.bytes_recon_per_cell =
         (double)((size_t)IM * ts * ID * (mixed ? 4 : 8)) + (ctx->iweno == 1 ? (double)ID * (ID + 1) / 2 * (mixed ? 4 : 8) : 0) +
