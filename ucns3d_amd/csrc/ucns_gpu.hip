@@ -2284,10 +2284,19 @@ __global__ void k_adj_csr(int ntile, int cap, const int32_t *uq, const int32_t *
 // 14,000-cell channel: a thread per face 19.4 us and, boundary, 113.7; a thread
 // per point 10.6 and 20.6; this launch 19.5.  24,576 tetrahedra: 34.9 -> 22.4 us.
 constexpr int BLANES = 16;
+// the (face, point) number of a thread, at `lanes` threads per point: a launch may
+// hold more than 2^31 threads (from 134 million boundary points on), the points
+// stay below that
+__host__ __device__ constexpr int vjp_point(int block, int thread, int lanes) {
+    return (int)(((long long)block * 256 + thread) / lanes);
+}
+static_assert(vjp_point(0, 255, BLANES) == 15 && vjp_point(8388607, 255, BLANES) == 134217727 &&
+              vjp_point(8388608, 0, BLANES) == 134217728 && vjp_point(134217727, 255, BLANES) == 2147483647 &&
+              vjp_point(8388607, 255, 1) == 2147483647);
 template <typename R, bool BND>
 __device__ __forceinline__ void flux_vjp_block(const FluxParams<R> &p, int block, const int32_t *bfaces, int nbface,
                                                const double *lam, double *ubf, double *bcbar) {
-    const int t = (block * 256 + (int)threadIdx.x) / (BND ? BLANES : 1);
+    const int t = vjp_point(block, threadIdx.x, BND ? BLANES : 1);
     const int fi = t / p.nqm, q = t - fi * p.nqm;
     const int f = BND ? (fi < nbface ? bfaces[fi] : p.nface) : fi;
     constexpr bool bnd = BND;
