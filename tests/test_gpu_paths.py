@@ -350,3 +350,95 @@ def test_rule_of_the_block_kernels(precision, n, shuffled, block):
     s.close()
     # 7 work arrays, the 3 of the stored forward, 5 of the tables' index by cell
     assert made == (15 if block else 18), made
+
+
+# MUSCL in mixed precision: a step against the FP64 oracle (1e-5), on one-point
+# faces with fluxes and update in one kernel (32,768 cells are the most it takes)
+# and on meshes it does not take
+@pytest.mark.parametrize("spec", [CaseSpec("mm-125", HEX, 5, "muscl", jitter=0.1, seed=3),
+                                  CaseSpec("mm-32768", HEX, 32, "muscl", jitter=0.1, seed=3),
+                                  CaseSpec("mm-35937", HEX, 33, "muscl", jitter=0.1, seed=3),
+                                  CaseSpec("mm-prism", PRISM, 7, "muscl", jitter=0.1, seed=3)], ids=lambda s: s.name)
+def test_muscl_in_mixed_precision(spec):
+    case = Case(spec)
+    u = case.init_state()
+    print(f"[mixed MUSCL] {spec.name} ncell={case.ncell}", flush=True)
+    s = Solver(case, UCNS_MIXED)
+    s.set_state(u)
+    s.rk3_steps(1, cfl=0.5)
+    err = rel_l2(s.get_state(), Oracle(case).rk3(u, 1, cfl=0.5)[0])
+    s.close()
+    print("  rel L2", err)
+    assert np.all(err <= 1e-5), err
+
+
+# The one-kernel march forms a face's flux in both of its cells: the two must hold
+# the same bits, so a periodic march conserves to the rounding of its updates (of
+# the order 1e-16 a cell and stage; FP32 fluxes that differed would leave 1e-9)
+@pytest.mark.parametrize("precision", [UCNS_FP64, UCNS_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("n", [5, 32])
+def test_one_point_march_conserves(n, precision):
+    case = Case(CaseSpec("cons-muscl", HEX, n, "muscl", jitter=0.1, seed=3))
+    u = case.init_state()
+    vol = np.ctypeslib.as_array(case.structs()[0].totvolume, shape=(case.ncell,))[:, None]
+    print(f"[conservation] ncell={case.ncell} precision={precision}", flush=True)
+    s = Solver(case, precision)
+    s.set_state(u)
+    s.rk3_steps(3, cfl=0.5)
+    gap = np.abs((vol * (s.get_state() - u)).sum(0)) / np.abs(vol * u).sum(0).max()
+    s.close()
+    print("  gap", gap)
+    assert np.all(gap <= 1e-13), gap
+
+
+# the largest mesh of the one-kernel march, against the two kernels
+def test_largest_march_on_one_point_faces():
+    case = Case(CaseSpec("f-muscl-32", HEX, 32, "muscl", jitter=0.1, seed=3))
+    assert case.ncell == 32768
+    u = case.init_state()
+    out = []
+    for timed in (False, True):
+        print(f"[one-point march] ncell={case.ncell} timed={timed}", flush=True)
+        s = Solver(case, UCNS_FP64)
+        if timed:
+            s.reset_stats()
+        s.set_state(u)
+        t = s.rk3_steps(3, cfl=0.5)
+        out.append((s.get_state(), t, s.stats()["n_flux"]))
+        s.close()
+    (a, ta, na), (b, tb, nb) = out
+    assert (na, nb) == (0, 9)
+    close(a, b, 1e-12)
+    assert abs(ta - tb) <= 1e-12 * tb
+
+
+# per-face boundary states in the one-kernel march
+@pytest.mark.parametrize("precision,tol", [(UCNS_FP64, 1e-12), (UCNS_MIXED, 1e-5)], ids=["fp64", "mixed"])
+def test_jet_inflow_on_one_point_faces(precision, tol):
+    from oracle import oracle
+    from test_boundary import face_centres
+    from test_gpu_boundary import P0, prim2cons
+    case = Case(CaseSpec("jet-muscl", HEX, 9, "muscl", jitter=0.1, seed=9, bc=(1, 2, 4, 4, 3, 3)))
+    outer = prim2cons(1.0, 0.5, 0.0, 0.0, P0)
+    jet = prim2cons(1.4, 2.0, 0.2, -0.1, 0.9 * P0)
+    inside = np.linalg.norm(face_centres(case)[..., 1:] - 0.5 * case.spec.length, axis=-1) < 0.3 * case.spec.length
+    states = np.where(inside[..., None], jet, outer)
+    u = case.init_state()
+    print(f"[one-point jet] ncell={case.ncell} precision={precision}", flush=True)
+    oracle.set_boundary(1, outer, outer)
+    oracle.set_boundary_faces(states, None)
+    try:
+        ref = Oracle(case).rk3(u, 1, cfl=0.4)[0]
+    finally:
+        oracle.set_boundary_faces(None, None)
+    uniform = Oracle(case).rk3(u, 1, cfl=0.4)[0]
+    s = Solver(case, precision)
+    s.set_boundary(1, outer, outer)
+    s.set_boundary_faces(states, None)
+    s.set_state(u)
+    s.rk3_steps(1, cfl=0.4)
+    err = rel_l2(s.get_state(), ref)
+    s.close()
+    print("  rel L2", err)
+    assert np.all(err <= tol), err
+    assert rel_l2(uniform, ref).max() > 1e-4  # the jet is seen
