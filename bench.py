@@ -71,23 +71,37 @@ def recon_bytes_per_cell(case, precision: int) -> float:
 
 
 def recon_kernel_name(case, precision: int) -> str:
-    """the reconstruction kernel the library launches: the row-stream kernels for
-    WENO-4 with 5 or 7 stencils (tetrahedra, hexahedra) and WENO-3 with 5 to 7,
-    the register-prefetch ones for other stencil counts"""
+    """the reconstruction kernel the library launches for a case in its own
+    order (a WENO-4 mesh whose tiles overflow the block kernels' member table,
+    cells in an order without locality, is not looked for)"""
     ts = int(case.array("admis").max())
     nv = (case.array("face_nodes").reshape(case.ncell, -1, 4) >= 0).sum(2)
     nf = int((nv > 0).sum(1).max())
     nqm = max(case.qp_quad if (nv == 4).any() else 0, case.qp_tri if (nv == 3).any() else 0)
     nfq = nf * nqm
-    if case.ideg == 34:  # WENO-5: the per-cell kernel (CWENO: a block of waves per tile)
-        r = "float" if precision else "double"
-        occ = 5 if precision and case.ncell > 8 * 768 else 4
-        return f"k_recon_cweno5<{r},{occ}>" if case.spec.ees == 5 else f"k_recon<{r},34,69,7>"
+    ntile = (case.ncell + 7) // 8
+    r = "float" if precision else "double"
+    if case.iweno == -1:
+        return f"k_recon_muscl<{r}>"
+    if case.ideg == 34 and case.spec.ees == 5:  # a block of waves per tile
+        return f"k_recon_cweno5<{r},{5 if precision and ntile > 768 else 4}>"
+    tiled = case.ideg in (9, 19) and nfq <= 56
+    if case.spec.wenwrt == 2:
+        if tiled and 5 <= ts <= 7:
+            return f"k_recon_block<{r},{case.ideg},{case.imax},{ts}>"
+        return f"k_recon<{r},{case.ideg},{case.imax},7,true>"
+    if not tiled:  # WENO-5, and face rules the tiled kernels do not hold
+        return f"k_recon<{r},{case.ideg},{case.imax},7>"
+    bits = 32 if precision else 64
+    nql = 3 if nfq <= 24 or case.ideg == 9 else 7
+    if case.spec.ees == 5:
+        return f"k_recon_cw{bits}<{case.ideg},{case.imax},{nql}>"
+    # WENO-4 with 5 or 7 stencils (tetrahedra, hexahedra) and WENO-3 with 5 to 7: the
+    # row stream, or for WENO-4 on few tiles the block kernels
     stream = ((ts == 5 and nfq <= 24) or (ts == 7 and nfq > 24)) if case.ideg == 19 else (5 <= ts <= 7 and nfq <= 24)
-    nql = 3 if nfq <= 24 else 7
-    if stream:
-        return f"k_recon_{'s32' if precision else 's64'}<{case.ideg},{case.imax},{nql},{ts}>"
-    return f"k_recon_{'w32' if precision else 'w64'}<{case.ideg},{case.imax},{nql}>"
+    if stream and case.ideg == 19 and ntile <= (768 if precision else 512):
+        return f"k_recon_block<{r},{case.ideg},{case.imax},{ts}>"
+    return f"k_recon_{'s' if stream else 'w'}{bits}<{case.ideg},{case.imax},{nql}{f',{ts}' if stream else ''}>"
 
 
 def committed_traffic(kernel: str, config: str):
