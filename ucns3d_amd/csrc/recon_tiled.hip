@@ -7,9 +7,23 @@
 
 namespace ucns {
 
-template <int IDEG, int IMAX, int NQL, int TS>
+// NT: the rows are loaded non-temporally.  That is the faster way up to some 1.3
+// million cells, and for WENO-3 and in mixed precision at every size measured.  A
+// march of WENO-4 in FP64 past that takes as long with them as with ordinary loads,
+// or longer, by where the allocator placed the rows (two contexts created in turn get one
+// placement each).  ms a step, ordinary loads and non-temporal, in either:
+//   tetrahedra 1,170,672 cells   25.3, 25.5   22.7, 23.0
+//              1,361,886         29.6, 29.7   29.0, 30.8
+//              1,971,054         42.9, 43.1   41.8, 44.6
+//   hexahedra  1,259,712         40.6, 40.4   36.8, 36.4
+//              1,560,896         50.4, 50.5   50.3, 51.3
+//              2,097,152         68.0, 68.9   67.5, 69.2
+// Why the second placement and the larger mesh do not suit them is not known; on
+// another card the two kinds took the same time in both.
+constexpr int NT_CELLS = 1310720;
+template <int IDEG, int IMAX, int NQL, int TS, bool NT = true>
 __global__ __launch_bounds__(WAVE) void k_recon_s64(ReconWParams<double> p) {
-    recon_s_body<double, IDEG, IMAX, NQL, TS, stream_depth(false, TS)>(p);
+    recon_s_body<double, IDEG, IMAX, NQL, TS, stream_depth(false, TS), false, NT>(p);
 }
 // Scatter of a residual product on the row stream, without the
 // reconstruction: lane (cell, stencil) holds its g_bar (p.gbs) and streams
@@ -185,8 +199,11 @@ static void launch(const ReconWParams<R> &w, int ideg, int smode, bool cweno, hi
                 else if (smode == 6) UCNS_LAUNCH(k_recon_sg64<9, 19, 3, 6>);
                 else UCNS_LAUNCH(k_recon_sg64<9, 19, 3, 7>);
             } else {
-                if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_s64<19, 39, 3, 5>);
-                else if (ideg == 19) UCNS_LAUNCH(k_recon_s64<19, 39, 7, 7>);
+                const bool nt = w.ncell <= NT_CELLS;
+                if (ideg == 19 && smode == 5 && nt) UCNS_LAUNCH(k_recon_s64<19, 39, 3, 5>);
+                else if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_s64<19, 39, 3, 5, false>);
+                else if (ideg == 19 && nt) UCNS_LAUNCH(k_recon_s64<19, 39, 7, 7>);
+                else if (ideg == 19) UCNS_LAUNCH(k_recon_s64<19, 39, 7, 7, false>);
                 else if (smode == 5) UCNS_LAUNCH(k_recon_s64<9, 19, 3, 5>);
                 else if (smode == 6) UCNS_LAUNCH(k_recon_s64<9, 19, 3, 6>);
                 else UCNS_LAUNCH(k_recon_s64<9, 19, 3, 7>);

@@ -477,7 +477,7 @@ constexpr int free_lds(int ring, int need, int a0, int a1, int b0, int b1, int c
     return -1;
 }
 
-template <typename R, int IDEG, int IMAX, int NQL, int TS, int DEPTH, bool STORE = false>
+template <typename R, int IDEG, int IMAX, int NQL, int TS, int DEPTH, bool STORE = false, bool NT = true>
 __device__ __forceinline__ void recon_s_body(const ReconWParams<R> &p) {
     using SS = StreamShape<R, IDEG, IMAX, TS, DEPTH>;
     constexpr int NP = SS::NP, TP = SS::TP;
@@ -511,7 +511,7 @@ __device__ __forceinline__ void recon_s_body(const ReconWParams<R> &p) {
         const char *src = T + SS::HD + (size_t)j * SS::RD;
         char *dst = ring + (j % DEPTH) * SS::SB;
 #pragma unroll
-        for (int c = 0; c < SS::NCH; ++c) dma_chunk(src + c * 1024, dst + c * 1024, lane, SS::RD - c * 1024);
+        for (int c = 0; c < SS::NCH; ++c) dma_chunk<NT>(src + c * 1024, dst + c * 1024, lane, SS::RD - c * 1024);
     };
     // piece q = lane + 64 c of a row is bytes [16 (q % 3), +16) of column
     // q / 3's record; pieces past the TP columns re-read cell 0.  Every lane
@@ -541,13 +541,13 @@ __device__ __forceinline__ void recon_s_body(const ReconWParams<R> &p) {
 #pragma unroll
         for (int c = 0; c < SS::NBC; ++c) {
             const int valid = bb - c * 1024;
-            dma_chunk(valid > 0 ? src + c * 1024 : src, dst + c * 1024, lane, valid > 0 ? valid : 16);
+            dma_chunk<NT>(valid > 0 ? src + c * 1024 : src, dst + c * 1024, lane, valid > 0 ? valid : 16);
         }
     };
 
 
     // prologue: header, then (row, states) pairs for rows 0..DEPTH-1
-    dma_chunk(T, ring + DEPTH * SS::SB, lane, SS::HD);
+    dma_chunk<NT>(T, ring + DEPTH * SS::SB, lane, SS::HD);
     issue_row(0);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(SS::NCH) : "memory");  // header landed
 #pragma unroll
@@ -633,7 +633,7 @@ __device__ __forceinline__ void recon_s_body(const ReconWParams<R> &p) {
 #pragma unroll 1
             for (int c = 0; c < nch; ++c) {
                 const int valid = bytes - c * 1024;
-                dma_chunk(valid > 0 ? (const char *)src + c * 1024 : (const char *)src, ring + off + c * 1024, lane,
+                dma_chunk<NT>(valid > 0 ? (const char *)src + c * 1024 : (const char *)src, ring + off + c * 1024, lane,
                           valid > 0 ? valid : 16);
             }
         };
