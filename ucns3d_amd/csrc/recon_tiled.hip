@@ -7,21 +7,41 @@
 
 namespace ucns {
 
-// NT: the rows are loaded non-temporally.  That is the faster way up to some 1.3
-// million cells, and for WENO-3 and in mixed precision at every size measured.  A
-// march of WENO-4 in FP64 past that takes as long with them as with ordinary loads,
-// or longer, by where the allocator placed the rows (two contexts created in turn get one
-// placement each).  ms a step, ordinary loads and non-temporal, in either:
-//   tetrahedra 1,170,672 cells   25.3, 25.5   22.7, 23.0
-//              1,361,886         29.6, 29.7   29.0, 30.8
-//              1,971,054         42.9, 43.1   41.8, 44.6
-//   hexahedra  1,259,712         40.6, 40.4   36.8, 36.4
-//              1,560,896         50.4, 50.5   50.3, 51.3
-//              2,097,152         68.0, 68.9   67.5, 69.2
-// Why the second placement and the larger mesh do not suit them is not known; on
-// another card the two kinds took the same time in both.
-constexpr int NT_CELLS = 1310720;
-template <int IDEG, int IMAX, int NQL, int TS, bool NT = true>
+// Whether a march's reconstruction loads its pseudo-inverses (`bytes` of them in a
+// launch) non-temporally, so that they do not evict the states and face values that
+// the next kernels read (ucns_device.h).  That is the faster way, except
+//   - where they fit the 256 MB of the memory-side cache: as ordinary lines they
+//     stay there from one stage to the next.  us a stage, ordinary and
+//     non-temporal, row stream: 32,768 hexahedra WENO-3 mixed (157 MB) 65.6, 84.9;
+//     4,913 WENO-4 FP64 (204 MB) 64.8, 75.2; 7,986 tetrahedra WENO-4 FP64 (237 MB)
+//     64.2, 69.3; 12,167 hexahedra WENO-4 mixed (252 MB) 89.2, 89.9; 54,872 WENO-3
+//     mixed (263 MB) 129.3, 127.1.  Register kernels, WENO-4: 2,058 pyramids mixed
+//     (37 MB) 61.7, 58.3; 4,374 FP64 (156 MB) 77.6, 82.1; 11,664 prisms mixed (207
+//     MB) 82.3, 97.0; and CWENO on WENO-3, 24,576 tetrahedra (84 MB) 50.3, 60.4;
+//   - WENO-4 in FP64 past some 1.3 million cells, which takes as long with them as
+//     with ordinary loads, or longer, by where the allocator placed the rows (two
+//     contexts created in turn get one placement each).  ms a step, ordinary and
+//     non-temporal, in either:
+//       tetrahedra 1,170,672 cells   25.3, 25.5   22.7, 23.0
+//                  1,361,886         29.6, 29.7   29.0, 30.8
+//                  1,971,054         42.9, 43.1   41.8, 44.6
+//       hexahedra  1,259,712         40.6, 40.4   36.8, 36.4
+//                  1,560,896         50.4, 50.5   50.3, 51.3
+//                  2,097,152         68.0, 68.9   67.5, 69.2
+//     Why the second placement and the larger mesh do not suit them is not known;
+//     on another card the two kinds took the same time in both.
+// The kernels of the residual products always load non-temporally: a reversed
+// stage streams its rows twice with the stored coefficients between.
+template <typename R>
+static bool stream_nt(const ReconWParams<R> &w, int ideg, int smode) {
+    const long long mib = 1 << 20;
+    const long long bytes =
+        smode ? w.ntile * w.tile_bytes : (long long)w.ntile * 8 * w.ts * (ideg == 19 ? 39 : 19) * ideg * sizeof(R);
+    if (bytes <= 256 * mib) return !smode && ideg == 19 && bytes <= 96 * mib;
+    return !(smode && sizeof(R) == 8 && ideg == 19 && w.ncell > 1310720);
+}
+
+template <int IDEG, int IMAX, int NQL, int TS, bool NT>
 __global__ __launch_bounds__(WAVE) void k_recon_s64(ReconWParams<double> p) {
     recon_s_body<double, IDEG, IMAX, NQL, TS, stream_depth(false, TS), false, NT>(p);
 }
@@ -157,34 +177,33 @@ template <int IDEG, int IMAX, int NQL, int TS>
 __global__ __launch_bounds__(WAVE, 2) void k_recon_sg32(ReconWParams<float> p) {
     recon_s_body<float, IDEG, IMAX, NQL, TS, stream_depth(true, TS), true>(p);
 }
-template <int IDEG, int IMAX, int NQL, int TS>
+template <int IDEG, int IMAX, int NQL, int TS, bool NT>
 __global__ __launch_bounds__(WAVE, 2) void k_recon_s32(ReconWParams<float> p) {
-    recon_s_body<float, IDEG, IMAX, NQL, TS, stream_depth(true, TS)>(p);
+    recon_s_body<float, IDEG, IMAX, NQL, TS, stream_depth(true, TS), false, NT>(p);
 }
 
 // FP64: registers for the 19x5 coefficients dominate, one wave per SIMD;
 // FP32: the compiler is asked for WAVES32 waves per SIMD.
 constexpr int WAVES32 = 1;           // waves per SIMD asked for in FP32
 constexpr int DEPTH64 = 1, DEPTH32 = 2;  // members in flight of the register-prefetch kernels
-template <int IDEG, int IMAX, int NQL>
+template <int IDEG, int IMAX, int NQL, bool NT>
 __global__ __launch_bounds__(WAVE) void k_recon_w64(ReconWParams<double> p) {
-    recon_w_body<double, IDEG, IMAX, NQL, DEPTH64>(p);
+    recon_w_body<double, IDEG, IMAX, NQL, DEPTH64, false, NT>(p);
 }
-template <int IDEG, int IMAX, int NQL>
+template <int IDEG, int IMAX, int NQL, bool NT>
 __global__ __launch_bounds__(WAVE) void k_recon_cw64(ReconWParams<double> p) {
-    recon_w_body<double, IDEG, IMAX, NQL, DEPTH64, true>(p);
+    recon_w_body<double, IDEG, IMAX, NQL, DEPTH64, true, NT>(p);
 }
-template <int IDEG, int IMAX, int NQL>
+template <int IDEG, int IMAX, int NQL, bool NT>
 __global__ __launch_bounds__(WAVE, WAVES32) void k_recon_cw32(ReconWParams<float> p) {
-    recon_w_body<float, IDEG, IMAX, NQL, DEPTH32, true>(p);
+    recon_w_body<float, IDEG, IMAX, NQL, DEPTH32, true, NT>(p);
 }
-template <int IDEG, int IMAX, int NQL>
+template <int IDEG, int IMAX, int NQL, bool NT>
 __global__ __launch_bounds__(WAVE, WAVES32) void k_recon_w32(ReconWParams<float> p) {
-    recon_w_body<float, IDEG, IMAX, NQL, DEPTH32>(p);
+    recon_w_body<float, IDEG, IMAX, NQL, DEPTH32, false, NT>(p);
 }
-// [cells][ts_in][imax][ideg] (FP64, ABI) -> tiled [tile][imax][ideg][8*ts] (R)
 
-template <typename R>
+template <typename R, bool NT>
 static void launch(const ReconWParams<R> &w, int ideg, int smode, bool cweno, hipStream_t stream) {
     const dim3 grid(w.tiles_per_xcd * NXCD), block(WAVE);
     const bool few = w.nf * w.nqm <= 24;
@@ -192,66 +211,70 @@ static void launch(const ReconWParams<R> &w, int ideg, int smode, bool cweno, hi
     if (smode) {
         // (ideg, imax, face-point slots, stencils): WENO-4 tets / hexes, WENO-3 tets / prisms and pyramids / hexes
         if constexpr (sizeof(R) == 8) {
-            if (w.gstore) {
-                if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_sg64<19, 39, 3, 5>);
-                else if (ideg == 19) UCNS_LAUNCH(k_recon_sg64<19, 39, 7, 7>);
-                else if (smode == 5) UCNS_LAUNCH(k_recon_sg64<9, 19, 3, 5>);
-                else if (smode == 6) UCNS_LAUNCH(k_recon_sg64<9, 19, 3, 6>);
-                else UCNS_LAUNCH(k_recon_sg64<9, 19, 3, 7>);
-            } else {
-                const bool nt = w.ncell <= NT_CELLS;
-                if (ideg == 19 && smode == 5 && nt) UCNS_LAUNCH(k_recon_s64<19, 39, 3, 5>);
-                else if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_s64<19, 39, 3, 5, false>);
-                else if (ideg == 19 && nt) UCNS_LAUNCH(k_recon_s64<19, 39, 7, 7>);
-                else if (ideg == 19) UCNS_LAUNCH(k_recon_s64<19, 39, 7, 7, false>);
-                else if (smode == 5) UCNS_LAUNCH(k_recon_s64<9, 19, 3, 5>);
-                else if (smode == 6) UCNS_LAUNCH(k_recon_s64<9, 19, 3, 6>);
-                else UCNS_LAUNCH(k_recon_s64<9, 19, 3, 7>);
-            }
+            if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_s64<19, 39, 3, 5, NT>);
+            else if (ideg == 19) UCNS_LAUNCH(k_recon_s64<19, 39, 7, 7, NT>);
+            else if (smode == 5) UCNS_LAUNCH(k_recon_s64<9, 19, 3, 5, NT>);
+            else if (smode == 6) UCNS_LAUNCH(k_recon_s64<9, 19, 3, 6, NT>);
+            else UCNS_LAUNCH(k_recon_s64<9, 19, 3, 7, NT>);
         } else {
-            if (w.gstore) {
-                if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_sg32<19, 39, 3, 5>);
-                else if (ideg == 19) UCNS_LAUNCH(k_recon_sg32<19, 39, 7, 7>);
-                else if (smode == 5) UCNS_LAUNCH(k_recon_sg32<9, 19, 3, 5>);
-                else if (smode == 6) UCNS_LAUNCH(k_recon_sg32<9, 19, 3, 6>);
-                else UCNS_LAUNCH(k_recon_sg32<9, 19, 3, 7>);
-            } else {
-                if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_s32<19, 39, 3, 5>);
-                else if (ideg == 19) UCNS_LAUNCH(k_recon_s32<19, 39, 7, 7>);
-                else if (smode == 5) UCNS_LAUNCH(k_recon_s32<9, 19, 3, 5>);
-                else if (smode == 6) UCNS_LAUNCH(k_recon_s32<9, 19, 3, 6>);
-                else UCNS_LAUNCH(k_recon_s32<9, 19, 3, 7>);
-            }
+            if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_s32<19, 39, 3, 5, NT>);
+            else if (ideg == 19) UCNS_LAUNCH(k_recon_s32<19, 39, 7, 7, NT>);
+            else if (smode == 5) UCNS_LAUNCH(k_recon_s32<9, 19, 3, 5, NT>);
+            else if (smode == 6) UCNS_LAUNCH(k_recon_s32<9, 19, 3, 6, NT>);
+            else UCNS_LAUNCH(k_recon_s32<9, 19, 3, 7, NT>);
         }
-        return;
-    }
-    if (cweno) {
+    } else if (cweno) {
         if constexpr (sizeof(R) == 8) {
-            if (ideg == 9) UCNS_LAUNCH(k_recon_cw64<9, 19, 3>);
-            else if (few) UCNS_LAUNCH(k_recon_cw64<19, 39, 3>);
-            else UCNS_LAUNCH(k_recon_cw64<19, 39, 7>);
+            if (ideg == 9) UCNS_LAUNCH(k_recon_cw64<9, 19, 3, NT>);
+            else if (few) UCNS_LAUNCH(k_recon_cw64<19, 39, 3, NT>);
+            else UCNS_LAUNCH(k_recon_cw64<19, 39, 7, NT>);
         } else {
-            if (ideg == 9) UCNS_LAUNCH(k_recon_cw32<9, 19, 3>);
-            else if (few) UCNS_LAUNCH(k_recon_cw32<19, 39, 3>);
-            else UCNS_LAUNCH(k_recon_cw32<19, 39, 7>);
+            if (ideg == 9) UCNS_LAUNCH(k_recon_cw32<9, 19, 3, NT>);
+            else if (few) UCNS_LAUNCH(k_recon_cw32<19, 39, 3, NT>);
+            else UCNS_LAUNCH(k_recon_cw32<19, 39, 7, NT>);
         }
-        return;
-    }
-    if constexpr (sizeof(R) == 8) {
-        if (ideg == 9) UCNS_LAUNCH(k_recon_w64<9, 19, 3>);
-        else if (few) UCNS_LAUNCH(k_recon_w64<19, 39, 3>);
-        else UCNS_LAUNCH(k_recon_w64<19, 39, 7>);
+    } else if constexpr (sizeof(R) == 8) {
+        if (ideg == 9) UCNS_LAUNCH(k_recon_w64<9, 19, 3, NT>);
+        else if (few) UCNS_LAUNCH(k_recon_w64<19, 39, 3, NT>);
+        else UCNS_LAUNCH(k_recon_w64<19, 39, 7, NT>);
     } else {
-        if (ideg == 9) UCNS_LAUNCH(k_recon_w32<9, 19, 3>);
-        else if (few) UCNS_LAUNCH(k_recon_w32<19, 39, 3>);
-        else UCNS_LAUNCH(k_recon_w32<19, 39, 7>);
+        if (ideg == 9) UCNS_LAUNCH(k_recon_w32<9, 19, 3, NT>);
+        else if (few) UCNS_LAUNCH(k_recon_w32<19, 39, 3, NT>);
+        else UCNS_LAUNCH(k_recon_w32<19, 39, 7, NT>);
     }
+}
+// the row stream storing every stencil's coefficients (w.gstore)
+template <typename R>
+static void launch_store(const ReconWParams<R> &w, int ideg, int smode, hipStream_t stream) {
+    const dim3 grid(w.tiles_per_xcd * NXCD), block(WAVE);
+    if constexpr (sizeof(R) == 8) {
+        if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_sg64<19, 39, 3, 5>);
+        else if (ideg == 19) UCNS_LAUNCH(k_recon_sg64<19, 39, 7, 7>);
+        else if (smode == 5) UCNS_LAUNCH(k_recon_sg64<9, 19, 3, 5>);
+        else if (smode == 6) UCNS_LAUNCH(k_recon_sg64<9, 19, 3, 6>);
+        else UCNS_LAUNCH(k_recon_sg64<9, 19, 3, 7>);
+    } else {
+        if (ideg == 19 && smode == 5) UCNS_LAUNCH(k_recon_sg32<19, 39, 3, 5>);
+        else if (ideg == 19) UCNS_LAUNCH(k_recon_sg32<19, 39, 7, 7>);
+        else if (smode == 5) UCNS_LAUNCH(k_recon_sg32<9, 19, 3, 5>);
+        else if (smode == 6) UCNS_LAUNCH(k_recon_sg32<9, 19, 3, 6>);
+        else UCNS_LAUNCH(k_recon_sg32<9, 19, 3, 7>);
+    }
+}
+template <typename R>
+static void launch_any(const ReconWParams<R> &w, int ideg, int smode, bool cweno, hipStream_t stream) {
+    if (smode && w.gstore)
+        launch_store(w, ideg, smode, stream);
+    else if (stream_nt(w, ideg, smode))
+        launch<R, true>(w, ideg, smode, cweno, stream);
+    else
+        launch<R, false>(w, ideg, smode, cweno, stream);
 }
 void launch_recon_tiled(const ReconWParams<double> &w, int ideg, int smode, bool cweno, hipStream_t stream) {
-    launch(w, ideg, smode, cweno, stream);
+    launch_any(w, ideg, smode, cweno, stream);
 }
 void launch_recon_tiled(const ReconWParams<float> &w, int ideg, int smode, bool cweno, hipStream_t stream) {
-    launch(w, ideg, smode, cweno, stream);
+    launch_any(w, ideg, smode, cweno, stream);
 }
 
 void launch_scatter(const ReconWParams<double> &w, int ideg, int smode, hipStream_t stream) {

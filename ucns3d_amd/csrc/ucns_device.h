@@ -487,9 +487,8 @@ __device__ __forceinline__ void lds_load16(const void *g, unsigned lds_base) {
 // the states and the face values that the flux kernel reads next.  Channel of
 // 131,000 cells, 4 steps: 4.93 -> 4.77 ms (mixed 2.22 -> 2.08); 85,000
 // hexahedra, 2 steps: 5.80 -> 5.65 ms; 197,000 tetrahedra: 8.86 -> 8.80 ms; the
-// product of 2 steps on 24,576 tetrahedra: 3.70 -> 3.40 ms.
-// (The WENO-4 reconstruction in FP64 goes back to ordinary loads on large
-// meshes: recon_tiled.hip.)
+// product of 2 steps on 24,576 tetrahedra: 3.70 -> 3.40 ms.  (Where it does not
+// pay: stream_nt in recon_tiled.hip.)
 __device__ __forceinline__ void lds_load16_nt(const void *g, unsigned lds_base) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(g), "{m0}"(lds_base) : "memory");
 }

@@ -324,7 +324,8 @@ __device__ __forceinline__ void recon_late(const ReconWParams<R> &p, R (&g)[IDEG
     if (STORE && s == 0 && cvalid) p.fstore[cell] = (reduce ? 1 : 0) | (first ? 2 : 0);
 }
 
-template <typename R, int IDEG, int IMAX, int NQL, int D, bool CW = false>
+// NT: the pseudo-inverses are loaded non-temporally
+template <typename R, int IDEG, int IMAX, int NQL, int D, bool CW, bool NT>
 __device__ __forceinline__ void recon_w_body(const ReconWParams<R> &p) {
     constexpr int NP = IDEG * (IDEG + 1) / 2;
     __shared__ R sB[8][NP];
@@ -365,6 +366,12 @@ __device__ __forceinline__ void recon_w_body(const ReconWParams<R> &p) {
         // registers) while one is accumulated.
         if (act) {
             const R *Pt = p.P + (size_t)tile * IMAX * IDEG * TP + pos;
+            auto fetch = [](const R *q) {
+                if constexpr (NT)
+                    return __builtin_nontemporal_load(q);
+                else
+                    return *q;
+            };
             R pb[D][IDEG];
             double ub[D][NV];
 #pragma unroll
@@ -374,7 +381,7 @@ __device__ __forceinline__ void recon_w_body(const ReconWParams<R> &p) {
                 for (int v = 0; v < NV; ++v) ub[d][v] = p.U[(size_t)n * NV + v];
                 const R *Pj = Pt + (size_t)d * IDEG * TP;
 #pragma unroll
-                for (int k = 0; k < IDEG; ++k) pb[d][k] = __builtin_nontemporal_load(Pj + k * TP);
+                for (int k = 0; k < IDEG; ++k) pb[d][k] = fetch(Pj + k * TP);
             }
 #pragma unroll 1
             for (int j0 = 0; j0 < IMAX; j0 += D) {
@@ -394,7 +401,7 @@ __device__ __forceinline__ void recon_w_body(const ReconWParams<R> &p) {
                             for (int v = 0; v < NV; ++v) ub[d][v] = p.U[(size_t)n * NV + v];
                             const R *Pj = Pt + (size_t)jn * IDEG * TP;
 #pragma unroll
-                            for (int k = 0; k < IDEG; ++k) pb[d][k] = __builtin_nontemporal_load(Pj + k * TP);
+                            for (int k = 0; k < IDEG; ++k) pb[d][k] = fetch(Pj + k * TP);
                         }
 #pragma unroll
                         for (int k = 0; k < IDEG; ++k)
