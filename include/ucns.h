@@ -272,7 +272,9 @@ int  ucns_residual_vjp_device(ucns_ctx *ctx, const double *w_dev, double *u_bar_
  * *t_io (or NULL) is advanced as by ucns_rk3_steps.  The last stages of the
  * forward sweep also keep their reconstruction for the reverse sweep, as
  * many as the scheme's adj_keep_gib and adj_keep_stages allow; the context
- * holds those buffers until ucns_destroy or ucns_upload_prestore. */
+ * holds those buffers until ucns_destroy or ucns_upload_prestore (or until a
+ * call of ucns_rk3_adjoint_geometry, which keeps less of a stage, or one after
+ * it, needs their room within that limit). */
 int  ucns_rk3_adjoint(ucns_ctx *ctx, int32_t nsteps, double cfl, double dt_fixed, const double *uN_bar,
                       double *u0_bar, int32_t layout, double *bc_bar, double *t_io);
 /* Same with device pointers, AOS layout (bc_bar_dev: 10 doubles or NULL). */
@@ -283,16 +285,24 @@ int  ucns_rk3_adjoint_device(ucns_ctx *ctx, int32_t nsteps, double cfl, double d
  * (no counterpart in the reference, which has no adjoint): the stencil
  * pseudo-inverses, indicators, basis integrals, VOLUME(1,1), face Gauss
  * points, face areas and normals and the cell volumes, summed over every
- * stage of the march.  FP64 contexts on the register kernels only
- * (UCNS_EUNSUPPORTED otherwise); the same discrete decisions are held as in
- * ucns_residual_vjp.  gbar->abi_version must be UCNS_ABI_VERSION. */
+ * stage of the march.  FP64 contexts only, on MUSCL, on the register kernels
+ * or on the row stream of WENO-3 meshes with up to 6 stencils a cell (prisms,
+ * pyramids); UCNS_EUNSUPPORTED otherwise.  The same discrete decisions are held
+ * as in ucns_residual_vjp.  gbar->abi_version must be UCNS_ABI_VERSION. */
 int  ucns_rk3_adjoint_geometry(ucns_ctx *ctx, int32_t nsteps, double dt_fixed, const double *uN_bar, double *u0_bar,
                                int32_t layout, double *bc_bar, const ucns_geometry_bar_v1 *gbar, double *t_io);
+/* The statistics so far: launches and kernel times since ucns_reset_stats, and
+ * the troubled-cell counts of the last residual or march. */
 int  ucns_stats(ucns_ctx *ctx, ucns_stats_v1 *out);
 /* Fault injection for tests of the error paths (no counterpart in the
  * reference): the nth device allocation the context makes from now on
  * fails with UCNS_ENOMEM (0 disarms). */
 int  ucns_debug_fail_alloc(ucns_ctx *ctx, int32_t nth);
+/* Clears the launch counts and times, and times every kernel from now on (events
+ * and a wait around each launch, for the rest of the context's life).  A context
+ * timed so runs fluxes and update as two kernels also in marches that take them
+ * in one when untimed (faces of one point, up to 32,768 cells): the times are
+ * those of the two, the results the same. */
 int  ucns_reset_stats(ucns_ctx *ctx);
 const char *ucns_last_error(const ucns_ctx *ctx);
 void ucns_destroy(ucns_ctx *ctx);

@@ -2,9 +2,9 @@
 // 69 members, quadratic sectors of 9 coefficients on their first 19), FP64 and
 // mixed (src/reconstruct_p.f90:955-1049, 1062-1199, 2044-2280, 3126-3406).
 //
-// One block of 5 waves per tile of 8 consecutive cells.  Bound: the HBM stream
-// of the pseudo-inverses (25.6 of the 34 KB a cell needs), so the design keeps
-// loads in flight and every phase spread over the block:
+// One block of 5 waves per tile of 8 consecutive cells.  The pseudo-inverses are
+// 25.6 of the 34 KB a cell needs from HBM, so the design keeps loads in flight and
+// every phase spread over the block:
 //   - the members' differences are gathered into LDS once, by all threads;
 //   - least squares: a thread takes a coefficient of a cell's central polynomial
 //     (a member row of the tile is 272 contiguous values), then three of a
@@ -16,11 +16,14 @@
 // Cells whose stencils are incomplete (FULL 0) take the MUSCL values whatever
 // the unlimited ones are, so only their central polynomial is formed.
 // Blast box of 24,247 cells in FP64: 552 us with one wave per cell, 365 us this
-// way (2.3 TB/s of the 34 KB a cell); the LDS reads of the differences and of
-// the polynomials at the face points now bound it, not the stream.  Two central
-// coefficients per thread would halve the first, and were slower (520 us: half
-// as many loads in flight); the pseudo-inverses are read with non-temporal
-// loads (390 us without: they evict the states and face values).
+// way (2.3 TB/s of the 34 KB a cell).  Bound by latency: a tile is a dozen
+// dependent memory trips with barriers between them, at three blocks a CU.
+// Counters at 295,704 cells (4.04 ms): the waves wait in 72% of their cycles, 0.5%
+// of them for the LDS to take an instruction; the LDS is busy 25% of the time, and
+// HBM moves 2.6 TB/s.  Two central coefficients per thread halve the LDS reads of
+// the differences and were slower (520 us: half as many loads in flight); the
+// pseudo-inverses are read with non-temporal loads (390 us without: they evict the
+// states and face values).
 #include "ucns_recon.h"
 
 namespace ucns {

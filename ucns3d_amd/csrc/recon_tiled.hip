@@ -1,7 +1,7 @@
 // The tiled WENO-3 / WENO-4 kernels in conserved variables: the row-stream
-// reconstruction of tetrahedra and hexahedra (with and without the
-// coefficients' copy for the adjoint) and its transposed scatter, the
-// register-prefetch reconstruction of other meshes, CWENO.
+// reconstruction of tetrahedra and hexahedra, and at WENO-3 of meshes with prisms
+// and pyramids (with and without the coefficients' copy for the adjoint), its
+// transposed scatter, the register-prefetch reconstruction of other meshes, CWENO.
 #include "ucns_recon.h"
 #include "ucns_tiled.h"
 

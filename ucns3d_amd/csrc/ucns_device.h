@@ -46,7 +46,7 @@ __host__ __device__ inline int ci_tri(int w, int f) { return (w >> (8 + f)) & 1;
 template <typename R>
 struct ReconParams {
     int ncell, nf, nqm, ts, per_xcd;
-    int iweno, qpq, qpt;
+    int qpq, qpt;
     double gamma, lwci1, eps;
     const double *U;       // [ncell][5]
     const int32_t *nbr;    // [ncell][ts][imax]
@@ -57,7 +57,7 @@ struct ReconParams {
     const int32_t *cinfo;  // [ncell]
     const int32_t *cnb;    // [ncell][nf] face neighbours
     R *uleft;              // [ncell][nf][nqm][5]
-    int *marks;            // [ncell] per block: MUSCL cells + 65536 * first-order cells (k_marks_sum)
+    int *marks;            // [ncell], or per tile: MUSCL cells + 65536 * first-order cells (summed by k_finish)
     // characteristic WENO (wenwrt 2): per cell face the neighbour (negative:
     // the boundary code) and the cell's own face angles (cos a1, sin a1, cos
     // a2, sin a2); the free-stream data of the boundary ghosts
@@ -391,13 +391,13 @@ struct ReconWParams {
     const int32_t *cinfo;
     const int32_t *cnb;    // [ncell][nf]
     R *uleft;              // [ncell][nf][nqm][5] deviations from the cell average
-    int *marks;            // [ntile] per tile: MUSCL cells + 65536 * first-order cells (k_marks_sum)
+    int *marks;            // [ntile] per tile: MUSCL cells + 65536 * first-order cells (summed by k_finish)
     const unsigned char *stream;  // per-tile row stream of the DMA kernels (StreamShape)
     long long tile_bytes;
     R *gstore;             // optional [ntile][ideg*5 + 10][8*ts]: every stencil's coefficients, then
                            // its indicators beta[5] and weights omega[5], for the adjoint
     int *fstore;           // with gstore: per cell, 1 = MUSCL (CHECKSOL), 2 = first order (CHECKSOLX)
-    // scatter of a residual product riding on the row stream (k_recon_sv*):
+    // scatter of a residual product over the row stream (k_scatter_s64/s32):
     // member j of lane position pos receives P_j^T gbs[.][.][pos]
     const double *gbs;        // [ntile][ideg*5][8*ts] cotangents of the stencil coefficients
     double *ubar;             // [ncell][5] accumulated

@@ -1233,17 +1233,24 @@ __global__ void k_dt_value(const double *slots, double *out) {
 // The residual is R_i = sum over the faces of cell i of +-F_f, F_f the
 // quadrature of ROTATEB(HLLC(ROTATEF(a_q), ROTATEF(b_q))) w_q |f|, with face
 // states a_q = U_L + ULEFT_L(q) and b_q = U_R + ULEFT_R(q) (or the ghost
-// state of a_q).  The reverse sweep runs in two kernels:
+// state of a_q).  A product runs
 //   k_flux_vjp  face-parallel: F_bar = w_owner - w_neighbour, and through
 //               each quadrature point the cotangents of a_q and b_q, written
 //               to the face-point slots of the two cells (each slot belongs
 //               to exactly one face, so no atomics);
+// then on the row stream
+//   k_recon_vjp_s  tile of 8 cells per wave: pulls the face-point cotangents back
+//               through the extrapolation, the WENO weights and indicators or the
+//               Barth limiter, from the coefficients and decisions that the
+//               forward reconstruction stored;
+//   k_scatter_s64/s32  P_s^T g_bar_s to the tile's member table, over the rows;
+// or on the other layouts (and for geometry cotangents)
 //   k_recon_vjp tile of 8 cells per wave, lane = 8 * cell + stencil: repeats
 //               the forward decisions of the reconstruction bit for bit
-//               (same arithmetic and order), then pulls the face-point
-//               cotangents back through the extrapolation, the WENO weights
-//               and indicators or the Barth limiter, and scatters
-//               P_s^T g_bar_s to the stencil members with FP64 atomics.
+//               (same arithmetic and order), pulls the cotangents back alike,
+//               and adds P_s^T g_bar_s to the tile's member table;
+// and last
+//   k_adj_gather  the member tables summed by cell.
 // Discrete decisions (CHECKSOL / CHECKSOLX flags, HLLC and boundary
 // regimes, the limiter's arg-min face point and arg-max/min neighbour) are
 // those of the state the product is taken at, so the result is the exact
@@ -1318,7 +1325,7 @@ __device__ inline void atomic_add_f64(double *a, double v) { unsafeAtomicAdd(a, 
 // the tile's distinct member cells (a tile of 8 neighbouring cells shares
 // most of its stencil members), flushed with one HBM atomic per member and
 // variable instead of one per (stencil, member, variable).
-constexpr int HT = 4096;  // hash slots, >= 2 * the 8 * 8 * 39 member entries of a tile
+constexpr int HT = 4096;  // hash slots: more than the 8 * 7 * 39 member entries a tile has at most
 
 template <typename R, int IMAX>
 __global__ __launch_bounds__(WAVE) void k_tile_members(LsqView<R> L, int ntile, int ncell, const int32_t *cinfo,
@@ -1909,7 +1916,8 @@ __global__ __launch_bounds__(WAVE) void k_recon_vjp(VjpParams<R> p) {
 // scatter.  On the WENO path every step is per variable (indicators and
 // weights are), so a lane holds one variable's column of G_s at a time; B G_s
 // runs over the packed triangle of B once per variable.
-// Bound by latency at two or three waves per SIMD (registers), and by the issue of
+// Bound by latency at two or three waves per SIMD (registers; in FP64 32 bytes a
+// lane spill for hexahedra at WENO-4, 16 at WENO-3), and by the issue of
 // the face-point pass: with each lane taking a quarter of the coefficients at
 // every other point, the monomials of run-time exponents had been most of its
 // instructions.  Adjoint of 2 steps on 24,576 tetrahedra 3.34 -> 3.13 ms, on
@@ -2849,7 +2857,6 @@ int launch_recon_t(ucns_ctx *ctx, bool packed = false) {
     p.nqm = ctx->nqm;
     p.ts = ctx->ts;
     p.per_xcd = per_xcd(ctx->ncell);
-    p.iweno = ctx->iweno;
     p.qpq = ctx->qpq;
     p.qpt = ctx->qpt;
     p.gamma = ctx->gamma;
@@ -3754,9 +3761,9 @@ int rk3_step_ckpt(ucns_ctx *ctx, int it, int nsteps, const double *dt, unsigned 
 // reversed in the order (step n: 3, 2, 1), each at its stored state, with
 //   w = -c dt ybar / V, jt = (dR/du)^T w, and k_rk3_adj_stage combining ybar
 //   and jt into the cotangents of the stage's inputs and the next w.
-// In row-stream mode the scatter of a stage's reconstruction product rides on
-// the forward reconstruction of the next stage reversed, so each reversed
-// stage streams the pseudo-inverses once.
+// In row-stream mode the scatter of a stage's reconstruction product streams the
+// pseudo-inverses, and so does the forward reconstruction of a stage that did not
+// keep its own.
 //
 // Stages q = 3 it + stage - 1 >= keep0 kept their forward reconstruction, so
 // their products start from it and only the other stages run the

@@ -316,8 +316,8 @@ __device__ __forceinline__ void recon_late(const ReconWParams<R> &p, R (&g)[IDEG
         }
     }
     {
-        // the tile's counts, summed by k_marks_sum when a caller asks for
-        // them (same-address atomics retire one per 12 ns on this chip)
+        // the tile's counts, summed by k_finish when a call returns (same-address
+        // atomics retire one per 12 ns on this chip)
         const int nred = __popcll(__ballot(s == 0 && reduce)), nfst = __popcll(__ballot(s == 0 && first));
         if (lc == 0 && s == 0) p.marks[cell >> 3] = nred + 65536 * nfst;
     }
